@@ -5,10 +5,7 @@
 //   k_eb2d        per-cell triangle bounds in LDS (8x64 vertex tiles + 1-cell
 //                 halo), ordered per-vertex min, |U|,|V| scaling and the base-4
 //                 eb id -> eb code per vertex and component, id histogram
-//   k_lorenzo2d_c strip-pipelined wavefront Lorenzo + linear quantization:
-//                 one wave = 64 rows (lane = row), the row above arrives through
-//                 DPP wave_shr:1; strips hand their last row to the next strip
-//                 as tagged agent-coherent values the consumer spins on
+//   k_wave2d      strip-pipelined wavefront Lorenzo + linear quantization (wave2d.hip)
 //   Huffman       histogram -> host tree (reference tie-break) -> encode
 //   unpredictable values compacted in 12x12 block-major order
 // Decompress mirrors it: parallel Huffman decode of ids and codes, block-major
@@ -35,6 +32,7 @@
 #include "libm_math.hpp"
 #include "lorenzo2d_step.hpp"
 #include "bounds2d_fast.hpp"
+#include "wave2d.hpp"
 
 namespace cpsz {
 
@@ -182,6 +180,14 @@ __device__ __forceinline__ uint32_t code_from_table(double x, const double* __re
   return (uint32_t)lo;
 }
 
+// The eb codes once more, where the wavefront reads them (the id encoder reads
+// them in row-major order).
+struct CodeTiles {
+  uint16_t* u;
+  uint16_t* v;
+  Tile2d t;
+};
+
 constexpr int kTH = 16, kTW = 32;  // vertex tile (17x33 cells: 9 wave rounds of triangles per 512 vertices)
 
 template <typename T>
@@ -189,7 +195,8 @@ __device__ __forceinline__ void eb2d_tile(const T* __restrict__ U, const T* __re
                                           double max_pwr_eb, const double* __restrict__ q2d, int nq,
                                           uint16_t* __restrict__ cu, uint16_t* __restrict__ cv,
                                           uint32_t* __restrict__ hist, int* __restrict__ flags, const EbOverride& ov,
-                                          const double* __restrict__ qlog, int nqlog, int bx, int by) {
+                                          const double* __restrict__ qlog, int nqlog, const CodeTiles& ct, int bx,
+                                          int by) {
   __shared__ T su[kTH + 2][kTW + 2];
   __shared__ T sv[kTH + 2][kTW + 2];
   __shared__ double tb[kTH + 1][kTW + 1][2];
@@ -249,6 +256,7 @@ __device__ __forceinline__ void eb2d_tile(const T* __restrict__ U, const T* __re
       // itself (src/sz_compress_cp_preserve_2d.cpp:327-331)
       const uint32_t a = code_from_table(eb, qlog, nqlog);
       cu[(size_t)i * r2 + j] = (uint16_t)a;
+      ct.u[ct.t.at(i, j)] = (uint16_t)a;
       atomicAdd(&sh_hist[a ? a - 1 : 0], 1u);
       continue;
     }
@@ -260,6 +268,9 @@ __device__ __forceinline__ void eb2d_tile(const T* __restrict__ U, const T* __re
     const uint32_t b = eb_code_2d(av, q2d, nq);
     cu[(size_t)i * r2 + j] = (uint16_t)a;
     cv[(size_t)i * r2 + j] = (uint16_t)b;
+    const size_t te = ct.t.at(i, j);
+    ct.u[te] = (uint16_t)a;
+    ct.v[te] = (uint16_t)b;
     atomicAdd(&sh_hist[a ? a - 1 : 0], 1u);
     atomicAdd(&sh_hist[b ? b - 1 : 0], 1u);
     if (a > 82 || b > 82) atomicOr(&flags[1], 1);  // beyond the FP32 Lorenzo path
@@ -293,6 +304,7 @@ struct Eb2dJob {
   uint32_t* hist;
   int* flags;
   EbOverride ov;
+  CodeTiles ct;
   uint32_t blk0;
 };
 
@@ -314,8 +326,8 @@ __device__ __forceinline__ const Eb2dJob& eb_job_of(const Eb2dJob* __restrict__ 
 __device__ __forceinline__ void eb2d_tile_fast(const float* __restrict__ U, const float* __restrict__ V, int r1,
                                                int r2, double max_pwr_eb, const double* __restrict__ q2d, int nq,
                                                uint16_t* __restrict__ cu, uint16_t* __restrict__ cv,
-                                               uint32_t* __restrict__ hist, int* __restrict__ flags, int bx, int by,
-                                               uint32_t tile, uint32_t* __restrict__ fix_tiles,
+                                               uint32_t* __restrict__ hist, int* __restrict__ flags,
+                                               const CodeTiles& ct, int bx, int by, uint32_t tile, uint32_t* __restrict__ fix_tiles,
                                                uint32_t* __restrict__ fix_n) {
   __shared__ float su[kTH + 2][kTW + 2];
   __shared__ float sv[kTH + 2][kTW + 2];
@@ -396,6 +408,9 @@ __device__ __forceinline__ void eb2d_tile_fast(const float* __restrict__ U, cons
     }
     cu[(size_t)i * r2 + j] = (uint16_t)a;
     cv[(size_t)i * r2 + j] = (uint16_t)b;
+    const size_t te = ct.t.at(i, j);
+    ct.u[te] = (uint16_t)a;
+    ct.v[te] = (uint16_t)b;
     atomicAdd(&sh_hist[a ? a - 1 : 0], 1u);
     atomicAdd(&sh_hist[b ? b - 1 : 0], 1u);
     if (a > 82 || b > 82) atomicOr(&flags[1], 1);  // beyond the FP32 Lorenzo path
@@ -446,6 +461,9 @@ __global__ void __launch_bounds__(256) k_eb2d_fix(const Eb2dJob* __restrict__ jo
       const uint32_t a = eb_code_2d(au, q2d, nq), b = eb_code_2d(av, q2d, nq);
       J.cu[vix] = (uint16_t)a;
       J.cv[vix] = (uint16_t)b;
+      const size_t te = J.ct.t.at(i, j);
+      J.ct.u[te] = (uint16_t)a;
+      J.ct.v[te] = (uint16_t)b;
       atomicAdd(&J.hist[a ? a - 1 : 0], 1u);
       atomicAdd(&J.hist[b ? b - 1 : 0], 1u);
       if (a > 82 || b > 82) atomicOr(&J.flags[1], 1);
@@ -460,8 +478,9 @@ __global__ void __launch_bounds__(256) k_eb2d(const T* __restrict__ U, const T* 
                                               const double* __restrict__ q2d, int nq,
                                               uint16_t* __restrict__ cu, uint16_t* __restrict__ cv,
                                               uint32_t* __restrict__ hist, int* __restrict__ flags,
-                                              EbOverride ov, const double* __restrict__ qlog, int nqlog) {
-  eb2d_tile<T>(U, V, r1, r2, max_pwr_eb, q2d, nq, cu, cv, hist, flags, ov, qlog, nqlog, blockIdx.x, blockIdx.y);
+                                              EbOverride ov, const double* __restrict__ qlog, int nqlog,
+                                              CodeTiles ct) {
+  eb2d_tile<T>(U, V, r1, r2, max_pwr_eb, q2d, nq, cu, cv, hist, flags, ov, qlog, nqlog, ct, blockIdx.x, blockIdx.y);
 }
 
 // APPROX: eb2d_tile_fast (jobs without overrides), with its fix-up list
@@ -473,500 +492,11 @@ __global__ void __launch_bounds__(256) k_eb2d_multi(const Eb2dJob* __restrict__ 
   const uint32_t t = blockIdx.x - J.blk0;
   const int bx = (int)(t % (uint32_t)J.gx), by = (int)(t / (uint32_t)J.gx);
   if constexpr (APPROX)
-    eb2d_tile_fast(J.U, J.V, J.r1, J.r2, max_pwr_eb, q2d, nq, J.cu, J.cv, J.hist, J.flags, bx, by, blockIdx.x,
-                   fix_tiles, fix_n);
+    eb2d_tile_fast(J.U, J.V, J.r1, J.r2, max_pwr_eb, q2d, nq, J.cu, J.cv, J.hist, J.flags, J.ct, bx, by,
+                   blockIdx.x, fix_tiles, fix_n);
   else
-    eb2d_tile<float>(J.U, J.V, J.r1, J.r2, max_pwr_eb, q2d, nq, J.cu, J.cv, J.hist, J.flags, J.ov, nullptr, 0, bx,
-                     by);
-}
-
-// ------------------------------------------------------------ wavefront ----
-constexpr int kCH = 32;  // steps per chunk (boundary publish / prefetch granularity)
-
-__device__ __forceinline__ float shr1(float src, float lane0) {
-  return __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(lane0), __float_as_int(src),
-                                                    0x138 /* wave_shr:1 */, 0xF, 0xF, false));
-}
-
-struct Strip2d {
-  const float* x[2];
-  const uint16_t* c[2];  // compress: eb codes; decompress: stream ids
-  uint16_t* q[2];        // quant codes (written by compress, read by decompress)
-  const float* raw[2];   // decompress: unpredictable value per element
-  float* out[2];         // decompress output
-  uint64_t* bnd;         // [2][nstrips][r2] boundary rows (kBndTag | float bits, 0 = not yet)
-  int* prog;             // [2][nstrips] unused; [2 * nstrips] the item ticket
-  int* ticket;
-  int r1, r2, nstrips;
-  int wide;   // ids above 81: double-precision step
-  int shift;  // log2 of the eb base: 2 (offline, 4^id eps) or 1 (offline_log, 2^id eps)
-  // compress of a batch: the eb pass's flags, read in place of `wide`
-  // ([1]); a field with [0] set (non-finite input) is skipped as a whole
-  const int* flags;
-  // batch: issue priority (0-3) of the field's waves on their SIMD, higher
-  // for longer wavefronts
-  int prio;
-};
-
-// One item (component, 64-row strip) of a field's wavefront. The strip's last
-// row is handed to the next strip value by value: lane 63 stores each value
-// with a tag in the high word (kBndTag | float bits; the rows are zeroed before
-// the launch), and the consumer spins until the values it needs carry the tag.
-// No progress counter and no wait for store completion sit on the producer's
-// path. The strip's own rows for chunk c+1 are loaded while chunk c computes.
-constexpr uint64_t kBndTag = 1ull << 32;
-
-__device__ __forceinline__ uint64_t ld_coh64(const uint64_t* p) {
-  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ __forceinline__ void st_coh64(uint64_t* p, uint64_t v) {
-  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
-struct StripChunk {
-  float xs[kCH];         // compress: field values
-  uint32_t cs[kCH / 2];  // eb codes (compress) / stream ids (decompress), two u16 per word
-  uint32_t qs[kCH / 2];  // decompress: quantization codes, two u16 per word
-  float raws[kCH];       // decompress: unpredictable value where the code is 0
-};
-
-__device__ __forceinline__ uint32_t lo16(uint32_t w, int k) { return (k & 1) ? w >> 16 : w & 0xFFFFu; }
-
-// Interior chunks move a lane's kCH consecutive elements of its row with
-// 16-byte loads from the 16-byte-aligned block holding the first element (a
-// 16-byte-aligned load never leaves the pages of the row it starts in), then
-// shift them into place with selects. The rows of a strip are 64 different
-// lines per instruction, so wide loads cut the lines the L1 and L2 serve per
-// element by 4 (8 for the u16 arrays) against element-wise loads.
-__device__ __forceinline__ uint32_t sel4(uint32_t a, uint32_t b, uint32_t c, uint32_t d, uint32_t q) {
-  const uint32_t lo = (q & 1) ? b : a, hi = (q & 1) ? d : c;
-  return (q & 2) ? hi : lo;
-}
-
-// kCH floats from p (4-byte aligned) into v
-__device__ __forceinline__ void ld_row_f32(const float* p, float* v) {
-  const uintptr_t a = (uintptr_t)p;
-  const uint32_t s = (uint32_t)(a >> 2) & 3;
-  const uint4* w = (const uint4*)(a & ~(uintptr_t)15);
-  uint32_t d[kCH + 4];
-#pragma unroll
-  for (int i = 0; i < kCH / 4; i++) {
-    const uint4 x = w[i];
-    d[4 * i] = x.x;
-    d[4 * i + 1] = x.y;
-    d[4 * i + 2] = x.z;
-    d[4 * i + 3] = x.w;
-  }
-  uint4 t = make_uint4(0, 0, 0, 0);
-  if (s) t = w[kCH / 4];
-  d[kCH] = t.x;
-  d[kCH + 1] = t.y;
-  d[kCH + 2] = t.z;
-  d[kCH + 3] = t.w;
-#pragma unroll
-  for (int k = 0; k < kCH; k++) v[k] = __uint_as_float(sel4(d[k], d[k + 1], d[k + 2], d[k + 3], s));
-}
-
-// kCH u16 from p (2-byte aligned) into kCH/2 words, element k in word k/2
-// (low half for even k)
-__device__ __forceinline__ void ld_row_u16(const uint16_t* p, uint32_t* e) {
-  const uintptr_t a = (uintptr_t)p;
-  const uint32_t s = (uint32_t)(a >> 1) & 7;  // u16 offset in the 16-byte block
-  const uint4* w = (const uint4*)(a & ~(uintptr_t)15);
-  uint32_t d[kCH / 2 + 4];
-#pragma unroll
-  for (int i = 0; i < kCH / 8; i++) {
-    const uint4 x = w[i];
-    d[4 * i] = x.x;
-    d[4 * i + 1] = x.y;
-    d[4 * i + 2] = x.z;
-    d[4 * i + 3] = x.w;
-  }
-  uint4 t = make_uint4(0, 0, 0, 0);
-  if (s) t = w[kCH / 8];
-  d[kCH / 2] = t.x;
-  d[kCH / 2 + 1] = t.y;
-  d[kCH / 2 + 2] = t.z;
-  d[kCH / 2 + 3] = t.w;
-  const uint32_t q = s >> 1, b = (s & 1) * 2;
-  uint32_t g[kCH / 2 + 1];
-#pragma unroll
-  for (int m = 0; m <= kCH / 2; m++)
-    g[m] = m + 3 < kCH / 2 + 4 ? sel4(d[m], d[m + 1], d[m + 2], d[m + 3], q) : d[m];
-#pragma unroll
-  for (int m = 0; m < kCH / 2; m++) e[m] = __builtin_amdgcn_alignbyte(g[m + 1], g[m], b);
-}
-
-// kCH u16 (two per word, as ld_row_u16) to p (2-byte aligned): 4-byte
-// stores, with a 2-byte store at each end when p is not 4-byte aligned
-__device__ __forceinline__ void st_row_u16(uint16_t* p, const uint32_t* e) {
-  const uintptr_t a = (uintptr_t)p;
-  const bool odd = (a & 2) != 0;
-  uint32_t* w = (uint32_t*)((a + 2) & ~(uintptr_t)3);  // first 4-byte boundary at or after p
-  if (odd) {
-    p[0] = (uint16_t)e[0];
-    p[kCH - 1] = (uint16_t)(e[kCH / 2 - 1] >> 16);
-  }
-#pragma unroll
-  for (int m = 0; m < kCH / 2; m++) {
-    const uint32_t v = odd ? (m + 1 < kCH / 2 ? __builtin_amdgcn_alignbyte(e[m + 1], e[m], 2) : 0u) : e[m];
-    if (!odd || m + 1 < kCH / 2) w[m] = v;
-  }
-}
-
-// kCH floats to p (4-byte aligned): 8-byte stores, with a 4-byte store at
-// each end when p is not 8-byte aligned
-__device__ __forceinline__ void st_row_f32(float* p, const float* v) {
-  const uintptr_t a = (uintptr_t)p;
-  const bool odd = (a & 4) != 0;
-  float2* w = (float2*)((a + 4) & ~(uintptr_t)7);
-  if (odd) {
-    p[0] = v[0];
-    p[kCH - 1] = v[kCH - 1];
-  }
-#pragma unroll
-  for (int m = 0; m < kCH / 2; m++) {
-    const float x = odd ? v[2 * m + 1] : v[2 * m];
-    const float y = odd ? (2 * m + 2 < kCH ? v[2 * m + 2] : 0.f) : v[2 * m + 1];
-    if (!odd || m + 1 < kCH / 2) w[m] = make_float2(x, y);
-  }
-}
-
-// SHIFT (a.shift as a compile-time constant) keeps the quantum's exponent a
-// shift of the id: a runtime factor costs an integer multiply per element.
-template <bool COMPRESS, bool WIDE, int SHIFT>
-__device__ __forceinline__ void strip_item(const Strip2d& a, int item, int lane) {
-  const int r1 = a.r1, r2 = a.r2;
-  const int comp = item & 1, s = item >> 1;
-  const int row = s * 64 + lane;
-  const bool rvalid = row < r1;
-  const size_t roff = (size_t)(rvalid ? row : 0) * r2;
-  // (selects rather than a.x[comp]: an indexed member would put a copied
-  // descriptor in scratch memory)
-  const float* X = COMPRESS ? (comp ? a.x[1] : a.x[0]) + roff : nullptr;
-  const uint16_t* C = (comp ? a.c[1] : a.c[0]) + roff;
-  uint16_t* Q = (comp ? a.q[1] : a.q[0]) + roff;
-  const float* RAW = COMPRESS ? nullptr : (comp ? a.raw[1] : a.raw[0]) + roff;
-  float* OUT = COMPRESS ? nullptr : (comp ? a.out[1] : a.out[0]) + roff;
-  const bool has_up = s > 0;
-  const bool publish = s + 1 < a.nstrips;
-  const uint64_t* bnd_in = a.bnd + ((size_t)comp * a.nstrips + (s > 0 ? s - 1 : 0)) * r2;
-  uint64_t* bnd_out = a.bnd + ((size_t)comp * a.nstrips + s) * r2;
-  float Rprev = 0.f, Uprev = 0.f;
-  const int steps = r2 + 63;
-  // An interior chunk has every lane's kCH columns inside the row and all 64
-  // rows present, so none of its steps needs a bounds mask; most chunks are
-  // interior and run the unmasked body, with wide loads and buffered stores.
-  const bool full_rows = s * 64 + 64 <= r1;
-  auto interior = [&](int t0) { return full_rows && t0 >= 63 && t0 + kCH <= r2; };
-  auto load = [&](StripChunk& B, int t0, auto inner) {
-    constexpr bool IN = decltype(inner)::value;
-    if constexpr (IN) {
-      const int j0 = t0 - lane;
-      ld_row_u16(C + j0, B.cs);
-      if (COMPRESS) ld_row_f32(X + j0, B.xs);
-      else ld_row_u16(Q + j0, B.qs);
-      return;
-    }
-#pragma unroll
-    for (int k = 0; k < kCH; k += 2) {
-      uint32_t c2[2], q2[2];
-#pragma unroll
-      for (int h = 0; h < 2; h++) {
-        const int j = t0 + k + h - lane;
-        const bool act = rvalid && j >= 0 && j < r2;
-        c2[h] = act ? C[j] : 0u;
-        if (COMPRESS) B.xs[k + h] = act ? X[j] : 0.f;
-        else q2[h] = act ? Q[j] : 0u;
-      }
-      B.cs[k >> 1] = c2[0] | c2[1] << 16;
-      if (!COMPRESS) B.qs[k >> 1] = q2[0] | q2[1] << 16;
-    }
-  };
-  // decompress: the unpredictable values are read only where the code is 0
-  // (a few percent of elements), once the chunk's codes have arrived
-  auto load_raw = [&](StripChunk& B, int t0, auto inner) {
-    constexpr bool IN = decltype(inner)::value;
-#pragma unroll
-    for (int k = 0; k < kCH; k++) {
-      const int j = t0 + k - lane;
-      const bool act = IN || (rvalid && j >= 0 && j < r2);
-      B.raws[k] = (act && lo16(B.qs[k >> 1], k) == 0) ? RAW[j] : 0.f;
-    }
-  };
-  auto chunk = [&](const StripChunk& B, StripChunk& N, int t0, auto inner) {
-    constexpr bool IN = decltype(inner)::value;
-    float inc = 0.f;
-    if (has_up && t0 < r2) {
-      const bool want = lane < kCH && t0 + lane < r2;
-      uint64_t v = want ? ld_coh64(bnd_in + t0 + lane) : kBndTag;
-      while (!__all((v >> 32) != 0)) {
-        __builtin_amdgcn_s_sleep(1);
-        if ((v >> 32) == 0) v = ld_coh64(bnd_in + t0 + lane);
-      }
-      inc = __uint_as_float((uint32_t)v);
-    }
-    const bool more = t0 + kCH < steps, next_in = interior(t0 + kCH);
-    if (more) {
-      if (next_in) load(N, t0 + kCH, std::true_type{});
-      else load(N, t0 + kCH, std::false_type{});
-    }
-    uint32_t qo[IN && COMPRESS ? kCH / 2 : 1];
-    float oo[IN && !COMPRESS ? kCH : 1];
-    // the boundary row's chunk (lane 63's values) gathers in lane k and
-    // leaves in one store after the chunk: the next strip waits for whole
-    // chunks anyway (one step later than per-step stores, one store in place
-    // of kCH)
-    uint32_t pubv = 0;
-#pragma unroll
-    for (int k = 0; k < kCH; k++) {
-      if (!COMPRESS && k == kCH / 2 && more) {
-        if (next_in) load_raw(N, t0 + kCH, std::true_type{});
-        else load_raw(N, t0 + kCH, std::false_type{});
-      }
-      const int t = t0 + k;
-      const int j = t - lane;
-      const bool act = IN || (rvalid && j >= 0 && j < r2);
-      const float lane0 = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(inc), k));
-      const float Uv = shr1(Rprev, lane0);
-      const float pred = (Rprev + Uv) - Uprev;
-      const uint32_t ck = lo16(B.cs[k >> 1], k);
-      float R;
-      if (COMPRESS) {
-        uint16_t code;
-        R = l2d_compress_step<WIDE>(pred, B.xs[k], ck, code, SHIFT);
-        if constexpr (IN) {
-          if (k & 1) qo[k >> 1] |= (uint32_t)code << 16;
-          else qo[k >> 1] = code;
-        } else if (act) {
-          Q[j] = code;
-        }
-      } else {
-        R = l2d_decompress_step<WIDE>(pred, lo16(B.qs[k >> 1], k), ck, B.raws[k], SHIFT);
-        if constexpr (IN) oo[k] = R;
-        else if (act) OUT[j] = R;
-      }
-      if (publish) {
-        const uint32_t r63 = (uint32_t)__builtin_amdgcn_readlane(__float_as_int(R), 63);
-        pubv = lane == k ? r63 : pubv;
-      }
-      Uprev = Uv;
-      Rprev = (!IN && j < 0) ? 0.f : R;
-    }
-    if (publish) {
-      const int jp = t0 - 63 + lane;
-      if (lane < kCH && jp >= 0 && jp < r2) st_coh64(bnd_out + jp, kBndTag | pubv);
-    }
-    if constexpr (IN) {
-      if constexpr (COMPRESS) st_row_u16(Q + (t0 - lane), qo);
-      else st_row_f32(OUT + (t0 - lane), oo);
-    }
-  };
-  auto run = [&](const StripChunk& B, StripChunk& N, int t0) {
-    if (interior(t0)) chunk(B, N, t0, std::true_type{});
-    else chunk(B, N, t0, std::false_type{});
-  };
-  StripChunk A, B;
-  load(A, 0, std::false_type{});
-  if (!COMPRESS) load_raw(A, 0, std::false_type{});
-  for (int t0 = 0; t0 < steps; t0 += 2 * kCH) {
-    run(A, B, t0);
-    if (t0 + kCH < steps) run(B, A, t0 + kCH);
-  }
-}
-
-// One strip variant per kernel (the host picks it): the unrolled strip loop
-// is large, and one variant keeps the kernel's hot code and registers small.
-template <bool COMPRESS, bool WIDE, int SHIFT>
-__global__ void __launch_bounds__(64) k_lorenzo2d(Strip2d a) {
-  const int lane = threadIdx.x;
-  const int items = 2 * a.nstrips;
-  for (;;) {
-    int item = 0;
-    if (lane == 0) item = atomicAdd(a.ticket, 1);
-    item = __shfl(item, 0);
-    if (item >= items) return;
-    strip_item<COMPRESS, WIDE, SHIFT>(a, item, lane);
-  }
-}
-
-// All fields of a batch in one persistent launch: items are numbered field by
-// field (start[f] = first item of field f) and taken from one ticket counter,
-// so every wait (strip s on strip s-1 of the same field) targets an earlier
-// ticket. Each field keeps its own boundary rows and progress counters.
-struct StripBatch {
-  const Strip2d* f;
-  const int* start;
-  int nf, items;
-  int* ticket;
-};
-
-// Clears every field's boundary rows and counters (block row y = field) and
-// the batch ticket, from the field table already on the device.
-__global__ void __launch_bounds__(256) k_zero_fields(const Strip2d* __restrict__ f, int* __restrict__ ticket) {
-  const Strip2d& a = f[blockIdx.y];
-  const size_t nb = (size_t)2 * a.nstrips * a.r2 * 2, nz = 2 * (size_t)a.nstrips + 1;
-  const size_t step = (size_t)gridDim.x * blockDim.x;
-  for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < nb; i += step) ((int*)a.bnd)[i] = 0;
-  for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < nz; i += step) a.prog[i] = 0;
-  if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) *ticket = 0;
-}
-
-template <bool COMPRESS>
-__global__ void __launch_bounds__(64) k_lorenzo2d_batch(StripBatch b) {
-  const int lane = threadIdx.x;
-  for (;;) {
-    int item = 0;
-    if (lane == 0) item = atomicAdd(b.ticket, 1);
-    item = __shfl(item, 0);
-    if (item >= b.items) return;
-    int lo = 0, hi = b.nf - 1;
-    while (lo < hi) {
-      const int mid = (lo + hi + 1) >> 1;
-      if (b.start[mid] <= item) lo = mid;
-      else hi = mid - 1;
-    }
-    const Strip2d a = b.f[lo];
-    // The batch ends when its longest wavefront does, and the waves of a
-    // SIMD share its issue slots: the longer a field's dependency chain, the
-    // higher its waves' priority, so the critical chains step at nearly their
-    // solo speed while the short fields fill the remaining slots.
-    switch (a.prio) {
-      case 3: __builtin_amdgcn_s_setprio(3); break;
-      case 2: __builtin_amdgcn_s_setprio(2); break;
-      case 1: __builtin_amdgcn_s_setprio(1); break;
-      default: __builtin_amdgcn_s_setprio(0); break;
-    }
-    bool wide = a.wide;
-    if (a.flags) {
-      if (a.flags[0]) continue;  // every item of the field skips: no strip waits on another
-      wide = a.flags[1] != 0;
-    }
-    if (wide) strip_item<COMPRESS, true, 2>(a, item - b.start[lo], lane);
-    else strip_item<COMPRESS, false, 2>(a, item - b.start[lo], lane);  // batches are plain offline fields
-  }
-}
-
-// ---- T = double wavefront ----------------------------------------------------
-// The reference's double instantiation predicts and reconstructs in double
-// (pred = (float)((L + U) - UL), include/sz_compress_block_processing.hpp:127;
-// quantize / recover in double, include/sz_compression_utils.hpp:50-65,
-// include/sz_decompression_utils.hpp:63-73), so this strip wavefront carries
-// doubles: the same one-wave-per-64-row-strip structure as the float kernel,
-// the row above arriving through two 32-bit DPP shifts, the strip's last row
-// handed to the next strip through 64-bit values that replace a NaN pattern
-// no reconstruction takes (every value is finite: non-finite input is rejected).
-constexpr uint64_t kBndEmpty = 0x7FF4DEADBEEF0000ull;
-
-struct Strip2d64 {
-  const double* x[2];
-  const uint16_t* c[2];  // compress: eb codes; decompress: stream ids
-  uint16_t* q[2];
-  const double* raw[2];
-  double* out[2];
-  uint64_t* bnd;  // [2][nstrips][r2], kBndEmpty until published
-  int* ticket;
-  int r1, r2, nstrips;
-};
-
-__device__ __forceinline__ double shr1_d(double src, double lane0) {
-  const uint64_t b = (uint64_t)__double_as_longlong(src), z = (uint64_t)__double_as_longlong(lane0);
-  const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp((int)(uint32_t)z, (int)(uint32_t)b, 0x138, 0xF, 0xF, false);
-  const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp((int)(uint32_t)(z >> 32), (int)(uint32_t)(b >> 32), 0x138,
-                                                            0xF, 0xF, false);
-  return __longlong_as_double((long long)(((uint64_t)hi << 32) | lo));
-}
-
-__device__ __forceinline__ double readlane_d(double v, int k) {
-  const uint64_t b = (uint64_t)__double_as_longlong(v);
-  const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)b, k);
-  const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(b >> 32), k);
-  return __longlong_as_double((long long)(((uint64_t)hi << 32) | lo));
-}
-
-// quantize<double> (include/sz_compression_utils.hpp:50-65) for eb code c (0:
-// zero precision, c >= 1: precision 4^(c-1) eps)
-__device__ __forceinline__ double l2d_compress_step64(float pred, double x, uint32_t c, uint16_t& code) {
-  code = 0;
-  if (c == 0) return x;
-  const double prec = ldexp(1.0, 2 * ((int)c - 1) - 52);
-  const double diff = x - (double)pred;
-  double qd = fabs(diff) / prec + 1;
-  if (qd < 65536) {
-    qd = (diff > 0) ? qd : -qd;
-    const int qi = (int)(qd / 2) + 32768;
-    const double dec = (double)pred + 2 * (qi - 32768) * prec;
-    if (fabs(dec - x) <= prec) {
-      code = (uint16_t)qi;
-      return dec;
-    }
-  }
-  return x;
-}
-
-template <bool COMPRESS>
-__device__ void strip_item64(const Strip2d64& a, int item, int lane) {
-  const int r1 = a.r1, r2 = a.r2;
-  const int comp = item & 1, s = item >> 1;
-  const int row = s * 64 + lane;
-  const bool rvalid = row < r1;
-  const size_t roff = (size_t)(rvalid ? row : 0) * r2;
-  const bool has_up = s > 0, publish = s + 1 < a.nstrips;
-  const uint64_t* bnd_in = a.bnd + ((size_t)comp * a.nstrips + (s > 0 ? s - 1 : 0)) * r2;
-  uint64_t* bnd_out = a.bnd + ((size_t)comp * a.nstrips + s) * r2;
-  double Rprev = 0, Uprev = 0;
-  const int steps = r2 + 63;
-  for (int t0 = 0; t0 < steps; t0 += kCH) {
-    double inc = 0;
-    if (has_up && t0 < r2) {
-      const bool want = lane < kCH && t0 + lane < r2;
-      uint64_t v = want ? ld_coh64(bnd_in + t0 + lane) : 0;
-      while (!__all(!want || v != kBndEmpty)) {
-        __builtin_amdgcn_s_sleep(1);
-        if (want && v == kBndEmpty) v = ld_coh64(bnd_in + t0 + lane);
-      }
-      inc = __longlong_as_double((long long)v);
-    }
-    for (int k = 0; k < kCH && t0 + k < steps; k++) {
-      const int j = t0 + k - lane;
-      const bool act = rvalid && j >= 0 && j < r2;
-      const double lane0 = readlane_d(inc, k);
-      const double Uv = shr1_d(Rprev, lane0);
-      const float pred = (float)((Rprev + Uv) - Uprev);
-      double R;
-      if (COMPRESS) {
-        uint16_t code;
-        R = l2d_compress_step64(pred, act ? a.x[comp][roff + j] : 0.0, act ? a.c[comp][roff + j] : 0u, code);
-        if (act) a.q[comp][roff + j] = code;
-      } else {
-        const uint32_t q = act ? a.q[comp][roff + j] : 0u, sid = act ? a.c[comp][roff + j] : 0u;
-        const double prec = sid ? ldexp(1.0, 2 * (int)sid - 52) : 0.0;  // pow(4, id) * DBL_EPSILON
-        R = q == 0 ? (act ? a.raw[comp][roff + j] : 0.0) : (double)pred + 2 * ((int)q - 32768) * prec;
-        if (act) a.out[comp][roff + j] = R;
-      }
-      if (publish && lane == 63 && act) st_coh64(bnd_out + j, (uint64_t)__double_as_longlong(R));
-      Uprev = Uv;
-      Rprev = j < 0 ? 0.0 : R;
-    }
-  }
-}
-
-template <bool COMPRESS>
-__global__ void __launch_bounds__(64) k_lorenzo2d_f64(Strip2d64 a) {
-  const int lane = threadIdx.x;
-  const int items = 2 * a.nstrips;
-  for (;;) {
-    int item = 0;
-    if (lane == 0) item = atomicAdd(a.ticket, 1);
-    item = __shfl(item, 0);
-    if (item >= items) return;
-    strip_item64<COMPRESS>(a, item, lane);
-  }
-}
-
-__global__ void k_fill_u64(uint64_t* p, size_t n, uint64_t v) {
-  for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x)
-    p[i] = v;
+    eb2d_tile<float>(J.U, J.V, J.r1, J.r2, max_pwr_eb, q2d, nq, J.cu, J.cv, J.hist, J.flags, J.ov, nullptr, 0,
+                     J.ct, bx, by);
 }
 
 __global__ void k_zero_i32(int* p, int n) {
@@ -1007,7 +537,8 @@ struct SrcIds2d {
 };
 
 struct SrcCodes2d {
-  const uint16_t* q;
+  const uint16_t* q;  // tiles
+  Tile2d t;
   int r1, r2, nby;
   // optional (batched compress): the values the codec ran on, the global
   // exclusive scan of the blocks' zero counts at this component's first
@@ -1039,29 +570,20 @@ struct SrcCodes2d {
     block(b, bi, bj);
     const int sx = min(kBlock2d, r1 - bi * kBlock2d), sy = min(kBlock2d, r2 - bj * kBlock2d);
     const int k = min(idx, sx * sy - 1), ii = (int)((uint32_t)k / (uint32_t)sy), jj = k - ii * sy;
-    sym[0] = q[(size_t)(bi * kBlock2d + ii) * r2 + bj * kBlock2d + jj];
+    sym[0] = q[t.at(bi * kBlock2d + ii, bj * kBlock2d + jj)];
     return idx < sx * sy;
-  }
-  template <class F>
-  __device__ void each(size_t b, F f) const {
-    const int bi = (int)(b / nby), bj = (int)(b - (size_t)bi * nby);
-    const int i0 = bi * kBlock2d, j0 = bj * kBlock2d;
-    const int sx = min(kBlock2d, r1 - i0), sy = min(kBlock2d, r2 - j0);
-    for (int ii = 0; ii < sx; ii++) {
-      const uint16_t* row = q + (size_t)(i0 + ii) * r2 + j0;
-      for (int jj = 0; jj < sy; jj++) f((uint32_t)row[jj]);
-    }
   }
 };
 
 struct SinkIds2d {
   static constexpr int kBytes = 2;
-  uint16_t* su;
+  uint16_t* su;  // tiles
   uint16_t* sv;
   size_t n;
+  Tile2d t;
   __device__ void put(uint64_t p, uint32_t s) const {
-    if (p < n) su[p] = (uint16_t)s;
-    else sv[p - n] = (uint16_t)s;
+    if (p < n) su[t.at_linear(p)] = (uint16_t)s;
+    else sv[t.at_linear(p - n)] = (uint16_t)s;
   }
 };
 
@@ -1070,19 +592,21 @@ struct SinkIds2d {
 // stage and leaves in coalesced stores, and decoded up to 3 codes per step.
 struct SinkIds2dB {
   static constexpr int kBytes = 1;
-  uint16_t* su;
+  uint16_t* su;  // tiles
   uint16_t* sv;
   size_t n;
+  Tile2d t;
   __device__ void put(uint64_t p, uint32_t s) const {
-    if (p < n) su[p] = (uint16_t)s;
-    else sv[p - n] = (uint16_t)s;
+    if (p < n) su[t.at_linear(p)] = (uint16_t)s;
+    else sv[t.at_linear(p - n)] = (uint16_t)s;
   }
 };
 
-// block-major position -> row-major element
+// block-major position -> element
 struct SinkCodes2d {
   static constexpr int kBytes = 2;
-  uint16_t* q;
+  uint16_t* q;  // tiles
+  Tile2d t;
   int r1, r2, nby;
   // optional: zero-filled per-block counts of code 0 (the unpredictable
   // marker), added up while the codes are written
@@ -1117,7 +641,7 @@ struct SinkCodes2d {
       jj = rem2 - ii * sy;
       k = rem2;
     }
-    q[(size_t)(bi * kBlock2d + ii) * r2 + bj * kBlock2d + jj] = (uint16_t)s;
+    q[t.at(bi * kBlock2d + ii, bj * kBlock2d + jj)] = (uint16_t)s;
     if (zm && s == 0)
       atomicOr((unsigned long long*)&zm[3 * ((size_t)bi * nby + bj) + (k >> 6)], 1ull << (k & 63));
     if (zc) {
@@ -1158,10 +682,14 @@ struct BlockView {
     const int ii = k / sy, jj = k - ii * sy;
     return (size_t)(i0 + ii) * r2 + j0 + jj;
   }
+  __device__ size_t tile_elem(int k, const Tile2d& t) const {
+    const int ii = k / sy, jj = k - ii * sy;
+    return t.at(i0 + ii, j0 + jj);
+  }
 };
 
-__global__ void __launch_bounds__(256) k_block_zeros(const uint16_t* __restrict__ q, int r1, int r2, int nby,
-                                                     size_t nb, uint32_t* __restrict__ cnt) {
+__global__ void __launch_bounds__(256) k_block_zeros(const uint16_t* __restrict__ q, Tile2d t, int r1, int r2,
+                                                     int nby, size_t nb, uint32_t* __restrict__ cnt) {
   const size_t b = (size_t)blockIdx.x * kUnpWaves + (threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
   if (b >= nb) return;  // uniform across the wave
@@ -1169,15 +697,15 @@ __global__ void __launch_bounds__(256) k_block_zeros(const uint16_t* __restrict_
   uint32_t z = 0;
   for (int k0 = 0; k0 < v.m; k0 += 64) {
     const int k = k0 + lane;
-    const bool zero = k < v.m && q[v.elem(k, r2)] == 0;
+    const bool zero = k < v.m && q[v.tile_elem(k, t)] == 0;
     z += (uint32_t)__popcll(__ballot(zero));
   }
   if (lane == 0) cnt[b] = z;
 }
 
 template <typename T>
-__global__ void __launch_bounds__(256) k_gather_unpred(const uint16_t* __restrict__ q, const T* __restrict__ x,
-                                                       int r1, int r2, int nby, size_t nb,
+__global__ void __launch_bounds__(256) k_gather_unpred(const uint16_t* __restrict__ q, Tile2d t,
+                                                       const T* __restrict__ x, int r1, int r2, int nby, size_t nb,
                                                        const uint64_t* __restrict__ off, T* __restrict__ out) {
   const size_t b = (size_t)blockIdx.x * kUnpWaves + (threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
@@ -1187,17 +715,16 @@ __global__ void __launch_bounds__(256) k_gather_unpred(const uint16_t* __restric
   const uint64_t below = (1ull << lane) - 1;
   for (int k0 = 0; k0 < v.m; k0 += 64) {
     const int k = k0 + lane;
-    const size_t e = k < v.m ? v.elem(k, r2) : 0;
-    const bool zero = k < v.m && q[e] == 0;
+    const bool zero = k < v.m && q[v.tile_elem(k, t)] == 0;
     const uint64_t mask = __ballot(zero);
-    if (zero) out[o + __popcll(mask & below)] = x[e];
+    if (zero) out[o + __popcll(mask & below)] = x[v.elem(k, r2)];
     o += __popcll(mask);
   }
 }
 
 template <typename T>
-__global__ void __launch_bounds__(256) k_scatter_unpred(const uint16_t* __restrict__ q, const T* __restrict__ vals,
-                                                        int r1, int r2, int nby, size_t nb,
+__global__ void __launch_bounds__(256) k_scatter_unpred(const uint16_t* __restrict__ q, Tile2d t,
+                                                        const T* __restrict__ vals, int r1, int r2, int nby, size_t nb,
                                                         const uint64_t* __restrict__ off, uint64_t count,
                                                         T* __restrict__ raw, int* __restrict__ err) {
   const size_t b = (size_t)blockIdx.x * kUnpWaves + (threadIdx.x >> 6);
@@ -1208,7 +735,7 @@ __global__ void __launch_bounds__(256) k_scatter_unpred(const uint16_t* __restri
   const uint64_t below = (1ull << lane) - 1;
   for (int k0 = 0; k0 < v.m; k0 += 64) {
     const int k = k0 + lane;
-    const size_t e = k < v.m ? v.elem(k, r2) : 0;
+    const size_t e = k < v.m ? v.tile_elem(k, t) : 0;
     const bool zero = k < v.m && q[e] == 0;
     const uint64_t mask = __ballot(zero);
     if (zero) {
@@ -1257,34 +784,32 @@ __global__ void __launch_bounds__(256) k_finish2d(float* __restrict__ U, float* 
   X[e] = y;
 }
 
+// The quantization codes as a tile array, padding and all: the histogram's
+// count of code 0 leaves the pads out.
 struct U16Hist {
   const uint16_t* p;  // 8-byte aligned (the code arrays are 256-byte aligned)
-  size_t n;
+  size_t n;           // a multiple of 1024
+  uint32_t pads;
   static constexpr int kChunk = 1024;
   // four codes per item, one 8-byte load
   static constexpr int kMaxItems = kChunk / 4, kPer = 4;
   __device__ int get(size_t c, int idx, uint32_t* sym) const {
-    const size_t i = c * kChunk + 4 * (size_t)idx;
-    if (i + 4 <= n) {
-      const uint2 w = *reinterpret_cast<const uint2*>(p + i);
-      sym[0] = w.x & 0xFFFFu;
-      sym[1] = w.x >> 16;
-      sym[2] = w.y & 0xFFFFu;
-      sym[3] = w.y >> 16;
-      return 4;
-    }
-    int k = 0;
-    for (; k < 4 && i + k < n; k++) sym[k] = p[i + k];
-    for (int q = k; q < 4; q++) sym[q] = 0;
-    return k;
+    const uint2 w = *reinterpret_cast<const uint2*>(p + c * kChunk + 4 * (size_t)idx);
+    sym[0] = w.x & 0xFFFFu;
+    sym[1] = w.x >> 16;
+    sym[2] = w.y & 0xFFFFu;
+    sym[3] = w.y >> 16;
+    return 4;
   }
+  static constexpr bool kPads = true;  // code-0 pads, counted out of bin 0
 };
 
 // ---- batched entropy stage: many fields' streams per launch -----------------
 // One component of one field for the per-block unpredictable passes
 // (kUnpWaves 12x12 blocks per workgroup, from workgroup blk0).
 struct UnpJob {
-  const uint16_t* q;
+  const uint16_t* q;     // tiles (as the scatter's output)
+  Tile2d t;
   const float* x;        // gather: values the codec ran on; scatter: the stream's unpredictable values
   int r1, r2, nby;
   size_t nb;
@@ -1306,7 +831,7 @@ __global__ void __launch_bounds__(256) k_block_zeros_multi(const UnpJob* __restr
   uint32_t z = 0;
   for (int k0 = 0; k0 < v.m; k0 += 64) {
     const int k = k0 + lane;
-    const bool zero = k < v.m && J.q[v.elem(k, J.r2)] == 0;
+    const bool zero = k < v.m && J.q[v.tile_elem(k, J.t)] == 0;
     z += (uint32_t)__popcll(__ballot(zero));
   }
   if (lane == 0) J.cnt[b] = z;
@@ -1322,7 +847,7 @@ __global__ void __launch_bounds__(256) k_scatter_unpred_multi(const UnpJob* __re
   const uint64_t below = (1ull << lane) - 1;
   for (int k0 = 0; k0 < v.m; k0 += 64) {
     const int k = k0 + lane;
-    const size_t e = k < v.m ? v.elem(k, J.r2) : 0;
+    const size_t e = k < v.m ? v.tile_elem(k, J.t) : 0;
     const bool zero = J.zm ? ((J.zm[3 * b + (k0 >> 6)] >> lane) & 1) != 0 : (k < v.m && J.q[e] == 0);
     const uint64_t mask = __ballot(zero);
     if (zero) {
@@ -1703,72 +1228,19 @@ void heads_2d(const HuffEncodeTable& t_eb, const HuffEncodeTable& t_u, const Huf
   put(H.hdr, H.v_size);
 }
 
-// Lorenzo wavefront for fields f[0..nf): one launch; a single field keeps the
-// plain kernel, several share one persistent launch.
-template <bool COMPRESS>
-void launch_wavefront(Ctx& ctx, std::vector<Strip2d>& f, int grid_cap) {
-  hipStream_t st = ctx.stream();
-  if (f.size() == 1 && !f[0].flags) {
-    Strip2d& sa = f[0];
-    const int nz = 2 * sa.nstrips + 1;
-    k_zero_i32<<<(int)div_up(nz, 256), 256, 0, st>>>(sa.prog, nz);
-    const size_t nb = (size_t)2 * sa.nstrips * sa.r2 * 2;  // tagged boundary rows as 32-bit words
-    k_zero_i32<<<(int)div_up(nb, 256), 256, 0, st>>>((int*)sa.bnd, (int)nb);
-    const int items = 2 * sa.nstrips;
-    const int grid = std::min(items, grid_cap);
-    if (sa.wide) k_lorenzo2d<COMPRESS, true, 2><<<grid, 64, 0, st>>>(sa);
-    else if (sa.shift == 1) k_lorenzo2d<COMPRESS, false, 1><<<grid, 64, 0, st>>>(sa);
-    else k_lorenzo2d<COMPRESS, false, 2><<<grid, 64, 0, st>>>(sa);
-    CPSZ_HIP(hipGetLastError());
-    return;
-  }
-  // Tickets go out field by field, the fields with the longest wavefront
-  // (one strip's hand-off lag per strip plus the row length) first, so the
-  // tallest fields are not left waiting for a free wave at the end.
-  const size_t nf = f.size();
-  CPSZ_REQUIRE(nf <= 65535, kErrUnsupported, "2D batch: at most 65535 fields per call");
-  for (const Strip2d& x : f) CPSZ_REQUIRE(x.shift == 2, kErrInternal, "2D batch wavefront: plain offline fields only");
-  std::vector<Strip2d> g(f);
-  std::stable_sort(g.begin(), g.end(), [](const Strip2d& a, const Strip2d& b) {
-    return (int64_t)a.nstrips * 96 + a.r2 > (int64_t)b.nstrips * 96 + b.r2;
-  });
-  std::vector<int> start(nf + 1, 0);
-  size_t max_words = 0;
-  const double lmax = (double)g[0].nstrips * 96 + g[0].r2;
-  for (size_t k = 0; k < nf; k++) {
-    const double l = ((double)g[k].nstrips * 96 + g[k].r2) / lmax;
-    g[k].prio = l >= 0.75 ? 3 : (l >= 0.5 ? 2 : (l >= 0.25 ? 1 : 0));
-    start[k + 1] = start[k] + 2 * g[k].nstrips;
-    max_words = std::max(max_words, (size_t)2 * g[k].nstrips * g[k].r2 * 2);
-  }
-  const size_t tbytes = nf * sizeof(Strip2d), sbytes = (nf + 1) * sizeof(int);
-  uint8_t* d = ctx.buf<uint8_t>("w2b.tab", tbytes + sbytes + 64);
-  int* ticket = (int*)(d + tbytes + sbytes + 16 - ((tbytes + sbytes) & 15));
-  uint8_t* h = (uint8_t*)ctx.host_table("w2b.tab", tbytes + sbytes);
-  std::memcpy(h, g.data(), tbytes);
-  std::memcpy(h + tbytes, start.data(), sbytes);
-  ctx.upload_table("w2b.tab", d, h, tbytes + sbytes);
-  k_zero_fields<<<dim3((unsigned)std::min<size_t>(div_up(max_words, 256 * 8), 64), (unsigned)nf), 256, 0, st>>>(
-      (const Strip2d*)d, ticket);
-  StripBatch b{(const Strip2d*)d, (const int*)(d + tbytes), (int)nf, start[nf], ticket};
-  const int grid = std::min(start[nf], grid_cap);
-  k_lorenzo2d_batch<COMPRESS><<<grid, 64, 0, st>>>(b);
-  CPSZ_HIP(hipGetLastError());
-}
-
 size_t al256(size_t x) { return (x + 255) & ~(size_t)255; }
 
 }  // namespace
 
 // ------------------------------------------------------------- staged form --
 size_t c2_scratch_bytes(size_t r1, size_t r2) {
-  const size_t n = r1 * r2, ns = div_up(r1, 64);
-  return 4 * al256(2 * n) + al256((kMaxEbCode + 2 * 65536) * 4) + al256(16) + al256(2 * ns * r2 * 8) +
-         al256((2 * ns + 1) * 4);
+  const size_t n = r1 * r2, te = Tile2d(r1, r2).elems(r1);
+  return 2 * al256(2 * n) + 4 * al256(2 * te) + al256((kMaxEbCode + 2 * 65536) * 4) + al256(16) + al256(8 * bnd_words(r1, r2)) + al256(4);
 }
 
 void c2_bind(C2Work& w, uint8_t* p) {
-  const size_t n = w.r1 * w.r2, ns = div_up(w.r1, 64);
+  w.t = Tile2d(w.r1, w.r2);
+  const size_t n = w.r1 * w.r2, te = w.t.elems(w.r1);
   auto take = [&](size_t bytes) {
     uint8_t* q = p;
     p += al256(bytes);
@@ -1776,12 +1248,14 @@ void c2_bind(C2Work& w, uint8_t* p) {
   };
   w.cu = (uint16_t*)take(2 * n);
   w.cv = (uint16_t*)take(2 * n);
-  w.qu = (uint16_t*)take(2 * n);
-  w.qv = (uint16_t*)take(2 * n);
+  w.tu = (uint16_t*)take(2 * te);
+  w.tv = (uint16_t*)take(2 * te);
+  w.qu = (uint16_t*)take(2 * te);
+  w.qv = (uint16_t*)take(2 * te);
   w.hist = (uint32_t*)take((kMaxEbCode + 2 * 65536) * 4);
   w.flags = (int*)take(16);
-  w.bnd = (uint64_t*)take(2 * ns * w.r2 * 8);
-  w.prog = (int*)take((2 * ns + 1) * 4);
+  w.bnd = (uint64_t*)take(8 * bnd_words(w.r1, w.r2));
+  w.ticket = (int*)take(4);
 }
 
 namespace {
@@ -1817,7 +1291,8 @@ void c2_eb(Ctx& ctx, C2Work& w, double max_pwr_eb, const EbOverride& ov) {
   dim3 grid((unsigned)div_up(w.r2, kTW), (unsigned)div_up(w.r1, kTH));
   if (w.f64) {
     k_eb2d<double><<<grid, 256, 0, st>>>(w.dU64, w.dV64, (int)w.r1, (int)w.r2, max_pwr_eb, ctx.d_q2d(),
-                                         ctx.q2d_size(), w.cu, w.cv, w.hist, w.flags, ov, nullptr, 0);
+                                         ctx.q2d_size(), w.cu, w.cv, w.hist, w.flags, ov, nullptr, 0,
+                                         CodeTiles{w.tu, w.tv, w.t});
   } else if (!w.log && !has_override(ov) && !exact_2d_bounds()) {
     Eb2dJob J{};
     J.U = w.dU;
@@ -1829,6 +1304,7 @@ void c2_eb(Ctx& ctx, C2Work& w, double max_pwr_eb, const EbOverride& ov) {
     J.cv = w.cv;
     J.hist = w.hist;
     J.flags = w.flags;
+    J.ct = CodeTiles{w.tu, w.tv, w.t};
     J.blk0 = 0;
     const size_t tiles = (size_t)grid.x * grid.y;
     CPSZ_REQUIRE(tiles < (1ull << 31), kErrUnsupported, "compress_2d: field too large");
@@ -1840,7 +1316,7 @@ void c2_eb(Ctx& ctx, C2Work& w, double max_pwr_eb, const EbOverride& ov) {
   } else {
     k_eb2d<float><<<grid, 256, 0, st>>>(w.dU, w.dV, (int)w.r1, (int)w.r2, max_pwr_eb, ctx.d_q2d(), ctx.q2d_size(),
                                         w.cu, w.cv, w.hist, w.flags, ov, w.log ? ctx.d_q2l() : nullptr,
-                                        ctx.q2l_size());
+                                        ctx.q2l_size(), CodeTiles{w.tu, w.tv, w.t});
   }
   CPSZ_HIP(hipGetLastError());
 }
@@ -1874,6 +1350,7 @@ void c2_eb_batch(Ctx& ctx, C2Work* const* w, size_t nf, double max_pwr_eb, const
     J.cv = W.cv;
     J.hist = W.hist;
     J.flags = W.flags;
+    J.ct = CodeTiles{W.tu, W.tv, W.t};
     J.ov = ov ? (*ov)[k] : EbOverride();
     approx = approx && !has_override(J.ov);
     J.blk0 = blk;
@@ -1908,33 +1385,22 @@ void c2_check(Ctx& ctx, C2Work* const* w, size_t nf) {
   }
 }
 
-namespace {
-void launch_wavefront64(Ctx& ctx, Strip2d64& sa, int* prog, int grid_cap) {
-  hipStream_t st = ctx.stream();
-  sa.ticket = prog;
-  k_zero_i32<<<1, 64, 0, st>>>(prog, 1);
-  const size_t nb = (size_t)2 * sa.nstrips * sa.r2;
-  k_fill_u64<<<(int)std::min<size_t>(div_up(nb, 256), 4096), 256, 0, st>>>(sa.bnd, nb, kBndEmpty);
-  const int grid = std::min(2 * sa.nstrips, grid_cap);
-  k_lorenzo2d_f64<true><<<grid, 64, 0, st>>>(sa);
-  CPSZ_HIP(hipGetLastError());
-}
-}  // namespace
-
 void c2_wavefront(Ctx& ctx, C2Work* const* w, size_t nf, int grid_cap) {
   if (nf == 1 && w[0]->f64) {
     Strip2d64 sa{};
     sa.x[0] = w[0]->dU64;
     sa.x[1] = w[0]->dV64;
-    sa.c[0] = w[0]->cu;
-    sa.c[1] = w[0]->cv;
+    sa.c[0] = w[0]->tu;
+    sa.c[1] = w[0]->tv;
     sa.q[0] = w[0]->qu;
     sa.q[1] = w[0]->qv;
     sa.bnd = w[0]->bnd;
+    sa.ticket = w[0]->ticket;
     sa.r1 = (int)w[0]->r1;
     sa.r2 = (int)w[0]->r2;
-    sa.nstrips = (int)div_up(w[0]->r1, 64);
-    launch_wavefront64(ctx, sa, w[0]->prog, grid_cap);
+    sa.ngroups = strip_groups<double>(w[0]->r1);
+    sa.shift = 2;
+    wavefront2d_compress64(ctx, sa, grid_cap);
     return;
   }
   for (size_t k = 0; k < nf; k++)
@@ -1946,22 +1412,21 @@ void c2_wavefront(Ctx& ctx, C2Work* const* w, size_t nf, int grid_cap) {
     const bool lg = w[k]->log;
     sa.x[0] = lg ? w[k]->lu : w[k]->dU;
     sa.x[1] = lg ? w[k]->lv : w[k]->dV;
-    sa.c[0] = w[k]->cu;
-    sa.c[1] = lg ? w[k]->cu : w[k]->cv;
+    sa.c[0] = w[k]->tu;
+    sa.c[1] = lg ? w[k]->tu : w[k]->tv;
     sa.shift = lg ? 1 : 2;
     sa.q[0] = w[k]->qu;
     sa.q[1] = w[k]->qv;
-    sa.nstrips = (int)div_up(w[k]->r1, 64);
+    sa.ngroups = strip_groups<float>(w[k]->r1);
     sa.bnd = w[k]->bnd;
-    sa.prog = w[k]->prog;
-    sa.ticket = w[k]->prog + 2 * sa.nstrips;
+    sa.ticket = w[k]->ticket;
     sa.r1 = (int)w[k]->r1;
     sa.r2 = (int)w[k]->r2;
     sa.wide = w[k]->wide;
     sa.flags = w[k]->flags_on_device ? w[k]->flags : nullptr;
     CPSZ_REQUIRE(!(lg && (sa.wide || sa.flags)), kErrInternal, "compress_2d_log: eb id beyond the base-2 range");
   }
-  launch_wavefront<true>(ctx, f, grid_cap);
+  wavefront2d_compress(ctx, f, grid_cap);
 }
 
 void c2_entropy(Ctx& ctx, const C2Work& w, DeviceStream& out) {
@@ -1974,8 +1439,9 @@ void c2_entropy(Ctx& ctx, const C2Work& w, DeviceStream& out) {
   // ---- histograms of the quant codes
   {
     const uint32_t win_lo = 32768 - 8192, win_n = 16384;
-    U16Hist hu{qu, n}, hv{qv, n};
-    const size_t nch = div_up(n, U16Hist::kChunk);
+    const size_t te = w.t.elems(r1);
+    U16Hist hu{qu, te, (uint32_t)(te - n)}, hv{qv, te, (uint32_t)(te - n)};
+    const size_t nch = te / U16Hist::kChunk;
     const int grid = (int)std::min<size_t>(encode_blocks(nch), 512);
     k_hist<<<grid, 256, win_n * 4, st>>>(hu, nch, hist + kMaxEbCode, win_lo, win_n);
     k_hist<<<grid, 256, win_n * 4, st>>>(hv, nch, hist + kMaxEbCode + 65536, win_lo, win_n);
@@ -1994,14 +1460,14 @@ void c2_entropy(Ctx& ctx, const C2Work& w, DeviceStream& out) {
   const size_t m_ids = w.log ? n : 2 * n;
   const size_t nch_ids = div_up(m_ids, SrcIds2d::kChunk);
   SrcIds2d s_ids{cu, cv, n, m_ids};
-  SrcCodes2d s_u{qu, (int)r1, (int)r2, nby}, s_v{qv, (int)r1, (int)r2, nby};
+  SrcCodes2d s_u{qu, w.t, (int)r1, (int)r2, nby}, s_v{qv, w.t, (int)r1, (int)r2, nby};
   uint64_t* bits = ctx.buf<uint64_t>("c2.bits", nch_ids + 2 * nb);
   uint64_t* offs = ctx.buf<uint64_t>("c2.offs", nch_ids + 2 * nb + 8);
   uint32_t* zc = ctx.buf<uint32_t>("c2.zc", 2 * nb);
   uint64_t* zoff = ctx.buf<uint64_t>("c2.zoff", 2 * nb + 4);
   uint64_t* totals = ctx.buf<uint64_t>("c2.totals", 8);
-  k_block_zeros<<<unp_grid(nb), 256, 0, st>>>(qu, (int)r1, (int)r2, nby, nb, zc);
-  k_block_zeros<<<unp_grid(nb), 256, 0, st>>>(qv, (int)r1, (int)r2, nby, nb, zc + nb);
+  k_block_zeros<<<unp_grid(nb), 256, 0, st>>>(qu, w.t, (int)r1, (int)r2, nby, nb, zc);
+  k_block_zeros<<<unp_grid(nb), 256, 0, st>>>(qv, w.t, (int)r1, (int)r2, nby, nb, zc + nb);
   CPSZ_HIP(hipGetLastError());
   scan_u32_to_u64(ctx, zc, zoff, nb, totals + 3);
   scan_u32_to_u64(ctx, zc + nb, zoff + nb, nb, totals + 4);
@@ -2060,12 +1526,12 @@ void c2_entropy(Ctx& ctx, const C2Work& w, DeviceStream& out) {
   const size_t vb = w.f64 ? 8 : 4;
   uint8_t* unp = ctx.buf<uint8_t>("c2.unp", vb * (unp_u + unp_v + 1));
   if (w.f64) {
-    k_gather_unpred<double><<<unp_grid(nb), 256, 0, st>>>(qu, w.dU64, (int)r1, (int)r2, nby, nb, zoff, (double*)unp);
-    k_gather_unpred<double><<<unp_grid(nb), 256, 0, st>>>(qv, w.dV64, (int)r1, (int)r2, nby, nb, zoff + nb,
+    k_gather_unpred<double><<<unp_grid(nb), 256, 0, st>>>(qu, w.t, w.dU64, (int)r1, (int)r2, nby, nb, zoff, (double*)unp);
+    k_gather_unpred<double><<<unp_grid(nb), 256, 0, st>>>(qv, w.t, w.dV64, (int)r1, (int)r2, nby, nb, zoff + nb,
                                                           (double*)unp + unp_u);
   } else {
-    k_gather_unpred<float><<<unp_grid(nb), 256, 0, st>>>(qu, dU, (int)r1, (int)r2, nby, nb, zoff, (float*)unp);
-    k_gather_unpred<float><<<unp_grid(nb), 256, 0, st>>>(qv, dV, (int)r1, (int)r2, nby, nb, zoff + nb,
+    k_gather_unpred<float><<<unp_grid(nb), 256, 0, st>>>(qu, w.t, dU, (int)r1, (int)r2, nby, nb, zoff, (float*)unp);
+    k_gather_unpred<float><<<unp_grid(nb), 256, 0, st>>>(qv, w.t, dV, (int)r1, (int)r2, nby, nb, zoff + nb,
                                                          (float*)unp + unp_u);
   }
   CPSZ_HIP(hipGetLastError());
@@ -2215,10 +1681,10 @@ void c2_entropy_batch(Ctx& ctx, C2Work* const* w, size_t nf, uint8_t* dout, cons
   for (size_t k = 0; k < nf; k++) {
     const C2Work& W = *w[k];
     const G& x = g[k];
-    const size_t nch = div_up(x.n, (size_t)U16Hist::kChunk);
+    const size_t te = W.t.elems(W.r1), nch = te / U16Hist::kChunk;
     for (int c = 0; c < 2; c++) {
       HistJob<U16Hist>& h = hj[2 * k + c];
-      h.src = U16Hist{c ? W.qv : W.qu, x.n};
+      h.src = U16Hist{c ? W.qv : W.qu, te, (uint32_t)(te - x.n)};
       h.nchunks = nch;
       h.hist = W.hist + kMaxEbCode + c * 65536;
       // 128 chunks per block: a block clears and flushes its 16384-bin window once per 131072 codes
@@ -2259,7 +1725,7 @@ void c2_entropy_batch(Ctx& ctx, C2Work* const* w, size_t nf, uint8_t* dout, cons
       EncJob<SrcCodes2d>& f = ej_c[2 * k + c];
       // the blocks' zero counts come with their bit counts; the encoder
       // gathers the unpredictable values (its array comes from k_layout2d)
-      f.src = SrcCodes2d{c ? W.qv : W.qu, (int)W.r1, (int)W.r2, (int)x.nby, c ? W.dV : W.dU,
+      f.src = SrcCodes2d{c ? W.qv : W.qu, W.t, (int)W.r1, (int)W.r2, (int)x.nby, c ? W.dV : W.dU,
                          zoff + x.zb + c * x.nb, nullptr};
       f.zc = zc + x.zb + c * x.nb;
       f.nchunks = x.nb;
@@ -2610,16 +2076,16 @@ void d2_unpred(Ctx& ctx, const uint8_t* d_in, const D2Plan& p, D2Work& w) {
     if (p.comp[c].unp_count)
       CPSZ_HIP(hipMemcpyAsync(vals, d_in + p.comp[c].unp_off, vb * p.comp[c].unp_count, hipMemcpyDeviceToDevice,
                               st));
-    k_block_zeros<<<unp_grid(nb), 256, 0, st>>>(qs[c], (int)r1, (int)r2, p.nby, nb, zc + c * nb);
+    k_block_zeros<<<unp_grid(nb), 256, 0, st>>>(qs[c], w.t, (int)r1, (int)r2, p.nby, nb, zc + c * nb);
     scan_u32_to_u64(ctx, zc + c * nb, zoff + c * (nb + 1), nb, zoff + c * (nb + 1) + nb);
     if (w.f64)
-      k_scatter_unpred<double><<<unp_grid(nb), 256, 0, st>>>(qs[c], (const double*)vals, (int)r1, (int)r2, p.nby,
+      k_scatter_unpred<double><<<unp_grid(nb), 256, 0, st>>>(qs[c], w.t, (const double*)vals, (int)r1, (int)r2, p.nby,
                                                              nb, zoff + c * (nb + 1), p.comp[c].unp_count,
-                                                             (double*)w.raw + c * n, w.err);
+                                                             (double*)w.raw + c * w.t.elems(r1), w.err);
     else
-      k_scatter_unpred<float><<<unp_grid(nb), 256, 0, st>>>(qs[c], (const float*)vals, (int)r1, (int)r2, p.nby, nb,
+      k_scatter_unpred<float><<<unp_grid(nb), 256, 0, st>>>(qs[c], w.t, (const float*)vals, (int)r1, (int)r2, p.nby, nb,
                                                             zoff + c * (nb + 1), p.comp[c].unp_count,
-                                                            w.raw + c * n, w.err);
+                                                            w.raw + c * w.t.elems(r1), w.err);
     CPSZ_HIP(hipGetLastError());
   }
 }
@@ -2627,25 +2093,25 @@ void d2_unpred(Ctx& ctx, const uint8_t* d_in, const D2Plan& p, D2Work& w) {
 }  // namespace
 
 size_t d2_scratch_bytes(size_t r1, size_t r2, bool f64) {
-  const size_t n = r1 * r2, ns = div_up(r1, 64);
-  return 4 * al256(2 * n) + al256((f64 ? 16 : 8) * n) + al256(2 * ns * r2 * 8) + al256((2 * ns + 1) * 4) +
-         al256(16);
+  const size_t te = Tile2d(r1, r2).elems(r1);
+  return 4 * al256(2 * te) + al256((f64 ? 16 : 8) * te) + al256(8 * bnd_words(r1, r2)) + al256(4) + al256(16);
 }
 
 void d2_bind(D2Work& w, uint8_t* p) {
-  const size_t n = w.r1 * w.r2, ns = div_up(w.r1, 64);
+  w.t = Tile2d(w.r1, w.r2);
+  const size_t te = w.t.elems(w.r1);
   auto take = [&](size_t bytes) {
     uint8_t* q = p;
     p += al256(bytes);
     return q;
   };
-  w.sid_u = (uint16_t*)take(2 * n);
-  w.sid_v = (uint16_t*)take(2 * n);
-  w.qu = (uint16_t*)take(2 * n);
-  w.qv = (uint16_t*)take(2 * n);
-  w.raw = (float*)take((w.f64 ? 16 : 8) * n);  // T = double: 2n doubles
-  w.bnd = (uint64_t*)take(2 * ns * w.r2 * 8);
-  w.prog = (int*)take((2 * ns + 1) * 4);
+  w.sid_u = (uint16_t*)take(2 * te);
+  w.sid_v = (uint16_t*)take(2 * te);
+  w.qu = (uint16_t*)take(2 * te);
+  w.qv = (uint16_t*)take(2 * te);
+  w.raw = (float*)take((w.f64 ? 16 : 8) * te);  // T = double: doubles
+  w.bnd = (uint64_t*)take(8 * bnd_words(w.r1, w.r2));
+  w.ticket = (int*)take(4);
   w.err = (int*)take(16);
 }
 
@@ -2655,6 +2121,7 @@ void d2_entropy(Ctx& ctx, const uint8_t* d_in, const uint8_t* h_in, size_t in_si
   const size_t r1 = w.r1, r2 = w.r2, n = r1 * r2;
   uint16_t *sid_u = w.sid_u, *sid_v = w.sid_v, *qu = w.qu, *qv = w.qv;
   const bool log = w.log;
+  const Tile2d tile = w.t;
   StreamReader rd(ctx, h_in, d_in, in_size);
   D2Plan p;
   d2_parse(rd, r1, r2, p, w.log, w.f64 ? 8 : 4);
@@ -2694,10 +2161,10 @@ void d2_entropy(Ctx& ctx, const uint8_t* d_in, const uint8_t* h_in, size_t in_si
     uint32_t* w = stage_bits(h_eb, "d2.w.eb");
     DeviceDecoder dd = upload_decoder(ctx, h_eb.tree.data(), h_eb.tree.size(), h_eb.node_count, "d2.eb");
     if (id_max < 256)
-      decode_stream(ctx, dd, w, h_eb.nbytes, log ? n : 2 * n, SinkIds2dB{sid_u, sid_v, n}, "d2.eb",
+      decode_stream(ctx, dd, w, h_eb.nbytes, log ? n : 2 * n, SinkIds2dB{sid_u, sid_v, n, tile}, "d2.eb",
                     [&] { prep(1); });
     else
-      decode_stream(ctx, dd, w, h_eb.nbytes, log ? n : 2 * n, SinkIds2d{sid_u, sid_v, n}, "d2.eb",
+      decode_stream(ctx, dd, w, h_eb.nbytes, log ? n : 2 * n, SinkIds2d{sid_u, sid_v, n, tile}, "d2.eb",
                     [&] { prep(1); });
     u_ready.join();  // rethrows a malformed code tree
   }
@@ -2707,8 +2174,8 @@ void d2_entropy(Ctx& ctx, const uint8_t* d_in, const uint8_t* h_in, size_t in_si
     const DeviceDecoder du = upload_decoder(ctx, hc[0], "d2.u");
     const DeviceDecoder dv = upload_decoder(ctx, hc[1], "d2.v");
     DecJob<SinkCodes2d> jobs[2] = {
-        {&du, wu, p.comp[0].h.nbytes, n, SinkCodes2d{qu, (int)r1, (int)r2, nby}, "d2.u"},
-        {&dv, wv, p.comp[1].h.nbytes, n, SinkCodes2d{qv, (int)r1, (int)r2, nby}, "d2.v"}};
+        {&du, wu, p.comp[0].h.nbytes, n, SinkCodes2d{qu, tile, (int)r1, (int)r2, nby}, "d2.u"},
+        {&dv, wv, p.comp[1].h.nbytes, n, SinkCodes2d{qv, tile, (int)r1, (int)r2, nby}, "d2.v"}};
     decode_streams(ctx, jobs, 2);
   }
   ctx.mark("huffman");
@@ -2760,6 +2227,7 @@ void d2_unpred_batch(Ctx& ctx, const std::vector<const uint8_t*>& d_in, const st
       UnpJob& u = uj[2 * k + c];
       u = UnpJob{};
       u.q = c ? W.qv : W.qu;
+      u.t = W.t;
       u.x = vals + vb[2 * k + c];
       u.r1 = (int)W.r1;
       u.r2 = (int)W.r2;
@@ -2767,7 +2235,7 @@ void d2_unpred_batch(Ctx& ctx, const std::vector<const uint8_t*>& d_in, const st
       u.nb = p.nb;
       u.cnt = zc + zb[k] + c * p.nb;
       u.off = zoff + zb[k] + c * p.nb;
-      u.out = W.raw + c * W.r1 * W.r2;
+      u.out = W.raw + c * W.t.elems(W.r1);
       u.count = p.comp[c].unp_count;
       u.err = W.err;
       u.blk0 = blk;
@@ -2951,14 +2419,14 @@ void d2_entropy_batch(Ctx& ctx, const std::vector<const uint8_t*>& d_in, const s
     const D2Plan& p = plan[k];
     // eb ids: codes of 1-5 bits over long runs of equal ids resynchronize
     // slowly from an arbitrary bit, so their speculative warm-up is longer
-    ji[k] = {&dd[3 * k], bc[3 * k].dst, p.h_eb.nbytes, 2 * n, SinkIds2d{w[k]->sid_u, w[k]->sid_v, n}, "b2d",
+    ji[k] = {&dd[3 * k], bc[3 * k].dst, p.h_eb.nbytes, 2 * n, SinkIds2d{w[k]->sid_u, w[k]->sid_v, n, w[k]->t}, "b2d",
              kIdWarm};
-    ji8[k] = {&dd[3 * k], bc[3 * k].dst, p.h_eb.nbytes, 2 * n, SinkIds2dB{w[k]->sid_u, w[k]->sid_v, n}, "b2d",
+    ji8[k] = {&dd[3 * k], bc[3 * k].dst, p.h_eb.nbytes, 2 * n, SinkIds2dB{w[k]->sid_u, w[k]->sid_v, n, w[k]->t}, "b2d",
               kIdWarm};
     uint16_t* qs[2] = {w[k]->qu, w[k]->qv};
     for (int c = 0; c < 2; c++)
       jc[2 * k + c] = {&dd[3 * k + 1 + c], bc[3 * k + 1 + c].dst, p.comp[c].h.nbytes, n,
-                       SinkCodes2d{qs[c], (int)r1, (int)r2, p.nby, zc + zb + c * p.nb, zm + 3 * (zb + c * p.nb)},
+                       SinkCodes2d{qs[c], w[k]->t, (int)r1, (int)r2, p.nby, zc + zb + c * p.nb, zm + 3 * (zb + c * p.nb)},
                        "b2d"};
     zb += 2 * p.nb;
   }
@@ -2972,8 +2440,7 @@ void d2_entropy_batch(Ctx& ctx, const std::vector<const uint8_t*>& d_in, const s
 
 void d2_wavefront(Ctx& ctx, D2Work* const* w, size_t nf, int grid_cap) {
   if (nf == 1 && w[0]->f64) {
-    hipStream_t st = ctx.stream();
-    const size_t n = w[0]->r1 * w[0]->r2;
+    const size_t n = w[0]->t.elems(w[0]->r1);
     Strip2d64 sa{};
     sa.c[0] = w[0]->sid_u;
     sa.c[1] = w[0]->sid_v;
@@ -2984,15 +2451,12 @@ void d2_wavefront(Ctx& ctx, D2Work* const* w, size_t nf, int grid_cap) {
     sa.out[0] = w[0]->dU64;
     sa.out[1] = w[0]->dV64;
     sa.bnd = w[0]->bnd;
+    sa.ticket = w[0]->ticket;
     sa.r1 = (int)w[0]->r1;
     sa.r2 = (int)w[0]->r2;
-    sa.nstrips = (int)div_up(w[0]->r1, 64);
-    sa.ticket = w[0]->prog;
-    k_zero_i32<<<1, 64, 0, st>>>(w[0]->prog, 1);
-    const size_t nb = (size_t)2 * sa.nstrips * sa.r2;
-    k_fill_u64<<<(int)std::min<size_t>(div_up(nb, 256), 4096), 256, 0, st>>>(sa.bnd, nb, kBndEmpty);
-    k_lorenzo2d_f64<false><<<std::min(2 * sa.nstrips, grid_cap), 64, 0, st>>>(sa);
-    CPSZ_HIP(hipGetLastError());
+    sa.ngroups = strip_groups<double>(w[0]->r1);
+    sa.shift = 2;
+    wavefront2d_decompress64(ctx, sa, grid_cap);
     return;
   }
   for (size_t k = 0; k < nf; k++)
@@ -3001,7 +2465,7 @@ void d2_wavefront(Ctx& ctx, D2Work* const* w, size_t nf, int grid_cap) {
   for (size_t k = 0; k < nf; k++) {
     Strip2d& sa = f[k];
     sa = Strip2d{};
-    const size_t n = w[k]->r1 * w[k]->r2;
+    const size_t n = w[k]->t.elems(w[k]->r1);
     sa.c[0] = w[k]->sid_u;
     sa.c[1] = w[k]->log ? w[k]->sid_u : w[k]->sid_v;
     sa.shift = w[k]->log ? 1 : 2;
@@ -3011,16 +2475,15 @@ void d2_wavefront(Ctx& ctx, D2Work* const* w, size_t nf, int grid_cap) {
     sa.raw[1] = w[k]->raw + n;
     sa.out[0] = w[k]->dU;
     sa.out[1] = w[k]->dV;
-    sa.nstrips = (int)div_up(w[k]->r1, 64);
+    sa.ngroups = strip_groups<float>(w[k]->r1);
     sa.bnd = w[k]->bnd;
-    sa.prog = w[k]->prog;
-    sa.ticket = w[k]->prog + 2 * sa.nstrips;
+    sa.ticket = w[k]->ticket;
     sa.r1 = (int)w[k]->r1;
     sa.r2 = (int)w[k]->r2;
     sa.wide = w[k]->wide;
     CPSZ_REQUIRE(!(w[k]->log && sa.wide), kErrStream, "decompress_2d_log: eb id beyond the base-2 range");
   }
-  launch_wavefront<false>(ctx, f, grid_cap);
+  wavefront2d_decompress(ctx, f, grid_cap);
 }
 
 void d2_check(Ctx& ctx, D2Work* const* w, size_t nf) {
@@ -3132,11 +2595,10 @@ void lorenzo2d_emulate(const float* x, const uint16_t* c, size_t r1, size_t r2, 
     for (size_t j = 0; j < r2; j++) {
       float* rp = &R[(i + 1) * W + j + 1];
       const float pred = (rp[-1] + rp[-(ptrdiff_t)W]) - rp[-(ptrdiff_t)W - 1];
-      uint16_t code;
+      float qs;
       const size_t e = i * r2 + j;
-      *rp = wide ? l2d_compress_step<true>(pred, x[e], c[e], code)
-                 : l2d_compress_step<false>(pred, x[e], c[e], code);
-      q[e] = code;
+      *rp = wide ? l2d_quantize_wide(pred, x[e], c[e], qs) : l2d_quantize(pred, x[e], l2d_prep(c[e], 2), qs);
+      q[e] = l2d_code(qs);
       if (recon) recon[e] = *rp;
     }
 }
@@ -3150,8 +2612,8 @@ void lorenzo2d_emulate_decode(const uint16_t* q, const uint16_t* sid, const floa
       float* rp = &R[(i + 1) * W + j + 1];
       const float pred = (rp[-1] + rp[-(ptrdiff_t)W]) - rp[-(ptrdiff_t)W - 1];
       const size_t e = i * r2 + j;
-      *rp = wide ? l2d_decompress_step<true>(pred, q[e], sid[e], raw[e])
-                 : l2d_decompress_step<false>(pred, q[e], sid[e], raw[e]);
+      *rp = wide ? l2d_restore_wide(pred, q[e], sid[e], raw[e])
+                 : (q[e] == 0 ? raw[e] : pred + l2d_step(q[e], sid[e], 2));
       out[e] = *rp;
     }
 }

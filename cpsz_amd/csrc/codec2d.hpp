@@ -3,6 +3,7 @@
 #include <vector>
 
 #include "ctx.hpp"
+#include "wave2d.hpp"
 
 namespace cpsz {
 
@@ -39,12 +40,14 @@ struct C2Work {
   const float* dU = nullptr;
   const float* dV = nullptr;
   size_t r1 = 0, r2 = 0;
-  uint16_t *cu = nullptr, *cv = nullptr;  // eb codes (0 = zero precision, else id + 1)
-  uint16_t *qu = nullptr, *qv = nullptr;  // quantization codes, row-major
+  Tile2d t;
+  uint16_t *cu = nullptr, *cv = nullptr;  // eb codes (0 = zero precision, else id + 1), row-major
+  uint16_t *tu = nullptr, *tv = nullptr;  // the same in tiles, for the wavefront
+  uint16_t *qu = nullptr, *qv = nullptr;  // quantization codes (tiles)
   uint32_t* hist = nullptr;               // kMaxEbCode + 2 * 65536 bins
   int* flags = nullptr;                   // [0] non-finite, [1] ids above 81
-  uint64_t* bnd = nullptr;  // wavefront boundary rows (tagged values)
-  int* prog = nullptr;      // wavefront item ticket
+  uint64_t* bnd = nullptr;  // wavefront boundary rows
+  int* ticket = nullptr;    // wavefront item ticket
   bool wide = false;
   // the flags stay on the device: the wavefront reads `wide` from flags[1]
   // and skips a field with flags[0] set (the caller reports it afterwards)
@@ -88,15 +91,16 @@ void c2_entropy_batch_finish(Ctx& ctx, size_t nf, const std::vector<size_t>& cap
 struct D2Work {
   size_t r1 = 0, r2 = 0;
   float *dU = nullptr, *dV = nullptr;         // outputs
-  uint16_t *sid_u = nullptr, *sid_v = nullptr;  // stream ids
+  Tile2d t;
+  uint16_t *sid_u = nullptr, *sid_v = nullptr;  // stream ids (tiles, as the next two)
   uint16_t *qu = nullptr, *qv = nullptr;      // quantization codes
-  float* raw = nullptr;                       // unpredictable values per element (2n)
-  uint64_t* bnd = nullptr;  // wavefront boundary rows (tagged values)
-  int *prog = nullptr, *err = nullptr;
+  float* raw = nullptr;                       // unpredictable values per element, u then v
+  uint64_t* bnd = nullptr;  // wavefront boundary rows
+  int *ticket = nullptr, *err = nullptr;
   bool wide = false;
   bool log = false;               // offline_log stream: ids shared by u and v, log values
   const uint8_t* signs = nullptr;  // offline_log: the stream's two sign bitmaps (device)
-  // T = double: outputs dU64/dV64, raw holds 2n doubles (d2_scratch_bytes(.., true))
+  // T = double: outputs dU64/dV64, raw holds doubles (d2_scratch_bytes(.., true))
   bool f64 = false;
   double *dU64 = nullptr, *dV64 = nullptr;
 };

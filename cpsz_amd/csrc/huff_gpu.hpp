@@ -152,6 +152,13 @@ __global__ void __launch_bounds__(kEncThreads) k_chunk_bits_multi(const EncJob<S
   chunk_bits_wave(J.src, c, J.len, J.bits, J.zc);
 }
 
+// A source whose symbols include `pads` extra symbols 0 (kPads), which the
+// histogram does not count.
+template <class S, class = void>
+struct HasPads : std::false_type {};
+template <class S>
+struct HasPads<S, std::void_t<decltype(S::kPads)>> : std::bool_constant<S::kPads> {};
+
 template <class Src>
 __device__ __forceinline__ void hist_block(const Src& src, size_t nchunks, uint32_t* __restrict__ hist,
                                            uint32_t win_lo, uint32_t win_n, uint32_t blk, uint32_t nblk,
@@ -186,6 +193,9 @@ __device__ __forceinline__ void hist_block(const Src& src, size_t nchunks, uint3
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) zeros += __shfl_xor(zeros, o);
   if (lane == 0 && zeros) atomicAdd(&hist[0], zeros);
+  if constexpr (HasPads<Src>::value) {
+    if (blk == 0 && threadIdx.x == 0) atomicSub(&hist[0], src.pads);
+  }
   __syncthreads();
   // blocks start their flush at different bins so that their global atomics
   // on the popular bins do not all arrive together
