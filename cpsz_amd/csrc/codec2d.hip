@@ -618,15 +618,18 @@ struct SinkCodes2d {
     const uint64_t rowblk = (uint64_t)kBlock2d * r2;
     int bi, bj, ii, jj;
     uint32_t k;  // position within the block
-    if (p < (1ull << 32) && rowblk < (1ull << 32)) {  // 32-bit divisions (a 64-bit one is a long sequence)
+    if (p < (1ull << 32) && rowblk < (1ull << 32)) {
+      // divisions by multiplication, but in the field's last blocks (a
+      // division is some 30 instructions, of 32 bits): p / (12 r2) is
+      // (p / 12) / r2
       const uint32_t p32 = (uint32_t)p, rb = (uint32_t)rowblk;
-      const uint32_t b = p32 / rb, rem = p32 - b * rb;
+      const uint32_t b = t.column ? p32 / kBlock2d : t.rows_in(p32 / kBlock2d), rem = p32 - b * rb;
       bi = (int)b;
       const uint32_t sx = (uint32_t)min(kBlock2d, r1 - bi * kBlock2d);
-      bj = min((int)(rem / (sx * kBlock2d)), nby - 1);
+      bj = min((int)(sx == kBlock2d ? rem / (kBlock2d * kBlock2d) : rem / (sx * kBlock2d)), nby - 1);
       const uint32_t rem2 = rem - (uint32_t)bj * sx * kBlock2d;
       const uint32_t sy = (uint32_t)min(kBlock2d, r2 - bj * kBlock2d);
-      ii = (int)(rem2 / sy);
+      ii = (int)(sy == kBlock2d ? rem2 / kBlock2d : rem2 / sy);
       jj = (int)(rem2 - (uint32_t)ii * sy);
       k = rem2;
     } else {
@@ -2130,18 +2133,13 @@ void d2_entropy(Ctx& ctx, const uint8_t* d_in, const uint8_t* h_in, size_t in_si
   const int nby = p.nby;
   ctx.mark("parse");
   // ---- bitstreams into aligned scratch
-  auto stage_bits = [&](const HuffSection& h, const char* name) {
-    // slack words: a speculative decode near the end peeks up to ~110 bits past it
-    uint32_t* w = ctx.buf<uint32_t>(name, div_up(h.nbytes, 4) + 8);
-    CPSZ_HIP(hipMemsetAsync(w, 0, (div_up(h.nbytes, 4) + 8) * 4, st));
-    if (h.nbytes)
-      CPSZ_HIP(hipMemcpyAsync(w, d_in + h.bits_off, h.nbytes, hipMemcpyDeviceToDevice, st));
-    return w;
-  };
+  BitsCopy bc[3] = {{d_in + h_eb.bits_off, h_eb.nbytes, nullptr, 0},
+                    {d_in + p.comp[0].h.bits_off, p.comp[0].h.nbytes, nullptr, 0},
+                    {d_in + p.comp[1].h.bits_off, p.comp[1].h.nbytes, nullptr, 0}};
   // The code trees are parsed and tabulated while the device decodes the id
-  // stream (the u tree on the helper thread, the v tree on this one between
-  // queuing the id decode and waiting for it); then the u and v streams decode
-  // in lockstep. The tables are kept per calling thread (their storage is
+  // stream (the u tree on the helper thread, the v tree on this one after
+  // queuing the id decode); then the u and v streams decode together, and the
+  // host looks at what all three held. The tables are kept per calling thread (their storage is
   // reused); the helper fills them through the pointer (a thread_local named
   // in the job would be the helper thread's own).
   thread_local HostDecoder hc_keep[2];
@@ -2156,28 +2154,28 @@ void d2_entropy(Ctx& ctx, const uint8_t* d_in, const uint8_t* h_in, size_t in_si
                  "malformed id tree");
     id_max = max_symbol(t);
   }
+  DecodeResult ids;
+  const SettleOnThrow settle{st};
   {
     HelperJob u_ready([&] { prep(0); }, !ctx.batch_worker);
-    uint32_t* w = stage_bits(h_eb, "d2.w.eb");
+    stage_bits_multi(ctx, bc, 3, "d2.bits");
     DeviceDecoder dd = upload_decoder(ctx, h_eb.tree.data(), h_eb.tree.size(), h_eb.node_count, "d2.eb");
     if (id_max < 256)
-      decode_stream(ctx, dd, w, h_eb.nbytes, log ? n : 2 * n, SinkIds2dB{sid_u, sid_v, n, tile}, "d2.eb",
-                    [&] { prep(1); });
+      ids = decode_stream(ctx, dd, bc[0].dst, h_eb.nbytes, log ? n : 2 * n, SinkIds2dB{sid_u, sid_v, n, tile}, "d2.eb");
     else
-      decode_stream(ctx, dd, w, h_eb.nbytes, log ? n : 2 * n, SinkIds2d{sid_u, sid_v, n, tile}, "d2.eb",
-                    [&] { prep(1); });
+      ids = decode_stream(ctx, dd, bc[0].dst, h_eb.nbytes, log ? n : 2 * n, SinkIds2d{sid_u, sid_v, n, tile}, "d2.eb");
+    prep(1);
     u_ready.join();  // rethrows a malformed code tree
   }
-  {
-    uint32_t* wu = stage_bits(p.comp[0].h, "d2.w.u");
-    uint32_t* wv = stage_bits(p.comp[1].h, "d2.w.v");
-    const DeviceDecoder du = upload_decoder(ctx, hc[0], "d2.u");
-    const DeviceDecoder dv = upload_decoder(ctx, hc[1], "d2.v");
-    DecJob<SinkCodes2d> jobs[2] = {
-        {&du, wu, p.comp[0].h.nbytes, n, SinkCodes2d{qu, tile, (int)r1, (int)r2, nby}, "d2.u"},
-        {&dv, wv, p.comp[1].h.nbytes, n, SinkCodes2d{qv, tile, (int)r1, (int)r2, nby}, "d2.v"}};
-    decode_streams(ctx, jobs, 2);
-  }
+  const DeviceDecoder du = upload_decoder(ctx, hc[0], "d2.u");
+  const DeviceDecoder dv = upload_decoder(ctx, hc[1], "d2.v");
+  const DecJob<SinkCodes2d> jobs[2] = {
+      {&du, bc[1].dst, p.comp[0].h.nbytes, n, SinkCodes2d{qu, tile, (int)r1, (int)r2, nby}},
+      {&dv, bc[2].dst, p.comp[1].h.nbytes, n, SinkCodes2d{qv, tile, (int)r1, (int)r2, nby}}};
+  const DecodeResult codes = decode_streams(ctx, jobs, 2, "d2.codes");
+  CPSZ_HIP(hipStreamSynchronize(st));
+  ids.check();
+  codes.check();
   ctx.mark("huffman");
   d2_unpred(ctx, d_in, p, w);
   w.wide = id_max > 81;
@@ -2259,13 +2257,11 @@ void d2_unpred_batch(Ctx& ctx, const std::vector<const uint8_t*>& d_in, const st
   CPSZ_HIP(hipStreamSynchronize(st));
 }
 
-constexpr uint32_t kIdWarm = 2048;  // speculative warm-up of the id streams, bits
-
 // Batched form: every field's headers parsed and trees tabulated on the
 // workers; all decoders uploaded in one copy and all bitstreams staged in one
 // launch; the id streams of every field decoded together, then the u and v
-// streams of every field together (one grid per pass, one host check per
-// round); the unpredictable scatter of each field on the workers.
+// streams of every field together (one grid per pass, one look at the results);
+// one unpredictable scatter.
 void d2_entropy_batch(Ctx& ctx, const std::vector<const uint8_t*>& d_in, const std::vector<size_t>& in_size,
                       D2Work* const* w, size_t nf, int workers) {
   hipStream_t st = ctx.stream();
@@ -2417,22 +2413,21 @@ void d2_entropy_batch(Ctx& ctx, const std::vector<const uint8_t*>& d_in, const s
   for (size_t k = 0; k < nf; k++) {
     const size_t r1 = w[k]->r1, r2 = w[k]->r2, n = r1 * r2;
     const D2Plan& p = plan[k];
-    // eb ids: codes of 1-5 bits over long runs of equal ids resynchronize
-    // slowly from an arbitrary bit, so their speculative warm-up is longer
-    ji[k] = {&dd[3 * k], bc[3 * k].dst, p.h_eb.nbytes, 2 * n, SinkIds2d{w[k]->sid_u, w[k]->sid_v, n, w[k]->t}, "b2d",
-             kIdWarm};
-    ji8[k] = {&dd[3 * k], bc[3 * k].dst, p.h_eb.nbytes, 2 * n, SinkIds2dB{w[k]->sid_u, w[k]->sid_v, n, w[k]->t}, "b2d",
-              kIdWarm};
+    ji[k] = {&dd[3 * k], bc[3 * k].dst, p.h_eb.nbytes, 2 * n, SinkIds2d{w[k]->sid_u, w[k]->sid_v, n, w[k]->t}};
+    ji8[k] = {&dd[3 * k], bc[3 * k].dst, p.h_eb.nbytes, 2 * n, SinkIds2dB{w[k]->sid_u, w[k]->sid_v, n, w[k]->t}};
     uint16_t* qs[2] = {w[k]->qu, w[k]->qv};
     for (int c = 0; c < 2; c++)
       jc[2 * k + c] = {&dd[3 * k + 1 + c], bc[3 * k + 1 + c].dst, p.comp[c].h.nbytes, n,
-                       SinkCodes2d{qs[c], w[k]->t, (int)r1, (int)r2, p.nby, zc + zb + c * p.nb, zm + 3 * (zb + c * p.nb)},
-                       "b2d"};
+                       SinkCodes2d{qs[c], w[k]->t, (int)r1, (int)r2, p.nby, zc + zb + c * p.nb, zm + 3 * (zb + c * p.nb)}};
     zb += 2 * p.nb;
   }
-  if (ids8) decode_streams_multi(ctx, ji8.data(), (int)nf, "b2d.ids");
-  else decode_streams_multi(ctx, ji.data(), (int)nf, "b2d.ids");
-  decode_streams_multi(ctx, jc.data(), (int)(2 * nf), "b2d.codes");
+  const SettleOnThrow settle{st};
+  const DecodeResult ids = ids8 ? decode_streams(ctx, ji8.data(), (int)nf, "b2d.ids")
+                                : decode_streams(ctx, ji.data(), (int)nf, "b2d.ids");
+  const DecodeResult codes = decode_streams(ctx, jc.data(), (int)(2 * nf), "b2d.codes");
+  CPSZ_HIP(hipStreamSynchronize(st));
+  ids.check();
+  codes.check();
   ctx.mark("huffman");
   d2_unpred_batch(ctx, d_in, plan, w, nf, true, zm);
   ctx.mark("unpred");

@@ -1286,21 +1286,14 @@ void d3_entropy(Ctx& ctx, const uint8_t* d_in, const uint8_t* h_in, size_t in_si
   thread_local HostDecoder hq_keep;
   HostDecoder& hq = hq_keep;
   HelperJob q_ready([&] { prepare_decoder(tr_q.data(), tr_q.size(), nc_q, hq); }, !ctx.batch_worker);
-  auto stage_bits = [&](size_t bo, size_t nbytes, const char* name) {
-    uint32_t* wb = ctx.buf<uint32_t>(name, div_up(nbytes, 4) + 8);
-    CPSZ_HIP(hipMemsetAsync(wb, 0, (div_up(nbytes, 4) + 8) * 4, st));
-    if (nbytes) CPSZ_HIP(hipMemcpyAsync(wb, d_in + bo, nbytes, hipMemcpyDeviceToDevice, st));
-    return wb;
-  };
-  {
-    uint32_t* wb = stage_bits(bo_id, nb_id, "d3.w.id");
-    DeviceDecoder dd = upload_decoder(ctx, tr_id.data(), tr_id.size(), nc_id, "d3.id");
-    decode_stream(ctx, dd, wb, nb_id, n, SinkU8{w.vid}, "d3.id");
-  }
+  BitsCopy bc[2] = {{d_in + bo_id, nb_id, nullptr, 0}, {d_in + bo_q, nb_q, nullptr, 0}};
+  const SettleOnThrow settle{st};
+  stage_bits_multi(ctx, bc, 2, "d3.bits");
+  const DeviceDecoder did = upload_decoder(ctx, tr_id.data(), tr_id.size(), nc_id, "d3.id");
+  const DecodeResult ids = decode_stream(ctx, did, bc[0].dst, nb_id, n, SinkU8{w.vid}, "d3.id");
   // what needs the ids but not the codes is queued while the helper may still
-  // be tabulating the code tree: the code bitstream's staging, per-chunk
-  // vertex counts and their scans, the unpredictable values and sign bitmaps
-  uint32_t* wq = stage_bits(bo_q, nb_q, "d3.w.q");
+  // be tabulating the code tree: per-chunk vertex counts and their scans, the
+  // unpredictable values and sign bitmaps
   const size_t nch = div_up(n, kVChunk);
   k_chunk_counts3d<false><<<(int)div_up(nch, 4), 256, 0, st>>>(w.vid, sk, n, nch, w.cnt, w.cnt + nch);
   scan_u32_to_u64(ctx, w.cnt, w.coff, nch, w.coff + 2 * nch + 2);
@@ -1309,10 +1302,11 @@ void d3_entropy(Ctx& ctx, const uint8_t* d_in, const uint8_t* h_in, size_t in_si
   CPSZ_HIP(hipMemsetAsync(w.err, 0, 16, st));
   CPSZ_HIP(hipMemcpyAsync(w.sm, d_in + 8, 3 * smap, hipMemcpyDeviceToDevice, st));
   q_ready.join();  // rethrows a malformed code tree
-  {
-    DeviceDecoder dd = upload_decoder(ctx, hq, "d3.q");
-    decode_stream(ctx, dd, wq, nb_q, data_num, SinkU16{w.qc}, "d3.q");
-  }
+  const DeviceDecoder dq = upload_decoder(ctx, hq, "d3.q");
+  const DecodeResult codes = decode_stream(ctx, dq, bc[1].dst, nb_q, data_num, SinkU16{w.qc}, "d3.q");
+  CPSZ_HIP(hipStreamSynchronize(st));
+  ids.check();
+  codes.check();
   ctx.mark("huffman");
   k_scatter3d<<<(int)div_up(nch, 4), 256, 0, st>>>(w.vid, sk, w.qc, w.unp, n, nch, w.coff, w.coff + nch + 1,
                                                    data_num, nunp_f, lm.log2f, w.vs, w.q, w.init, w.err);

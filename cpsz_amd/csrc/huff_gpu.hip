@@ -20,348 +20,216 @@ __global__ void k_scatter_codebook(const uint32_t* syms, const uint64_t* codes, 
   len[syms[i]] = lens[i];
 }
 
-__device__ __forceinline__ void dec_resync(const DecTree& t, const uint32_t* slut, const uint16_t* ms,
-                                           const uint32_t* __restrict__ w, const uint32_t* sw, uint64_t lbase,
-                                           uint32_t lcount, uint64_t end, uint64_t s0, uint64_t os, uint64_t oe,
-                                           uint32_t oc, uint64_t& ex, uint32_t& c, int* __restrict__ err);
+namespace {
 
-// Block `blk` of one stream's speculative / fix-up pass (k_dec_spec runs one
-// stream's blocks, k_dec_spec_multi every stream's blocks in one grid).
-__device__ __forceinline__ void dec_spec_block(const DecTree& t, const uint32_t* __restrict__ w, uint64_t nbits,
-                                               uint32_t S, uint32_t nseg, const uint64_t* __restrict__ prev_exit,
-                                               const uint64_t* __restrict__ prev_start,
-                                               uint64_t* __restrict__ start, uint64_t* __restrict__ exitp,
-                                               uint32_t* __restrict__ cnt, int* __restrict__ err, int first,
-                                               uint32_t blk, uint32_t* slut, uint32_t* sw, uint16_t* ms) {
-  const uint32_t i = blk * blockDim.x + threadIdx.x;
-  bool work = i < nseg;
-  uint64_t s0 = 0;
-  if (work) {
-    if (first) {
-      s0 = (uint64_t)i * S;
-    } else {
-      s0 = i == 0 ? 0 : prev_exit[i - 1];
-      if (s0 == prev_start[i]) {  // unchanged start: keep the previous result (and count)
-        start[i] = s0;
-        exitp[i] = prev_exit[i];
-        work = false;
-      }
-    }
-  }
-  if (!__syncthreads_or(work)) return;
-  for (int k = threadIdx.x; k < (1 << kLutBits); k += blockDim.x) slut[k] = t.lut[k];
-  uint64_t lbase;
-  const uint32_t lcount = stage_words(sw, w, nbits, S, blk * blockDim.x, lbase);
+// Length of the code at p. (A parsed tree is full, so there always is one.)
+__device__ __forceinline__ uint32_t code_len(const DecTree& t, const uint32_t* slut, const BlockBits& bits, uint32_t p) {
+  const uint32_t e = slut[bits.window(p) & kLutMask];
+  if (short_code(e)) return e & 0xFF;
+  uint32_t q = p;
+  long_code(t, bits, e, q);
+  return q - p;
+}
+
+}  // namespace
+
+// Bound by the lanes' serial walks (two LDS reads and some ten instructions a
+// step). Paths are followed as a bit set of the positions that some path
+// reaches, lowest first: the set spans max_len bits, and while it holds one
+// position the walk goes on by runs of codes. Measured in ms, on the ids of 96
+// fields of 256 to 4096 a side (1.5 bits a code): a guessed start after a
+// 2048-bit warm-up 2.61, its fix-up rounds 0.80 (22 on smoother fields, whose
+// runs of one id keep wrong phases alive); here 0.94, and 0.12 for the chain.
+// Codes of the same fields: 2.0 and 0.3 before, 1.77 and 0.20 here. One
+// 601 x 1203 log field, both decodes in all: 3.9 before, 0.4 here.
+__global__ void __launch_bounds__(256) k_dec_cand(MDecTable jobs, int* __restrict__ err, int* __restrict__ over) {
+  __shared__ uint32_t slut[1 << kLutBits];
+  __shared__ uint32_t sw[kStageWords];
+  __shared__ uint16_t ms[1 << kLutBits];
+  const int j = jobs.of_block(blockIdx.x);
+  const MDecJob& J = jobs[j];
+  const DecTree t = J.t;
+  const uint32_t b0 = (blockIdx.x - J.blk0) * 256, i = b0 + threadIdx.x;
+  stage_lut(slut, t.lut);
+  const BlockBits bits{(lds_u32*)sw};
+  const uint32_t pre = stage_words(sw, J.w, J.nbits, b0);
   __syncthreads();
   build_mstep(slut, ms);
   __syncthreads();
-  if (!work) return;
-  uint64_t end = (uint64_t)(i + 1) * S;
-  if (end > nbits) end = nbits;
-  BitReader br;
-  uint32_t c = 0;
-  if (first) {
-    // Warm-up: start kDecWarm bits before the segment and take as its start
-    // the first code boundary at or after i * S. A prefix-code path usually
-    // resyncs within a few code words, so this path is often already the true
-    // one there: its start then equals the previous segment's exit, and the
-    // fix-up passes skip the segment.
-    br.init(w, s0 - (s0 < kDecWarm ? s0 : kDecWarm), sw, lbase, lcount);
-    uint32_t skipped = 0;
-    if (!dec_until(t, slut, ms, br, s0, skipped)) *err = 1;
-    s0 = br.pos;
-    if (!dec_until(t, slut, ms, br, end, c)) *err = 1;
-    start[i] = s0;
-    exitp[i] = br.pos;
-    cnt[i] = c;
+  const uint32_t nseg = J.nseg;
+  if (i >= nseg) return;
+  const uint32_t a = pre + threadIdx.x * kSegBits;
+  const uint32_t end = a + (uint32_t)min((uint64_t)kSegBits, J.nbits - (uint64_t)i * kSegBits);
+  uint32_t p = i ? a - kWarmBits : a;
+  uint64_t m = i > 1 ? ~0ull >> (64 - J.max_len) : 1;  // positions from p on (max_len is 1 to 64)
+  while (p < a) {
+    if (m == 1) {
+      uint32_t skipped = 0;
+      dec_until(t, slut, ms, bits, p, a, skipped);
+      break;
+    }
+    m = m >> 1 | 1ull << (code_len(t, slut, bits, p) - 1);
+    const uint32_t s = (uint32_t)__ffsll((long long)m);  // on to the next position, 64 at most
+    m >>= s - 1;
+    p += s;
+  }
+  // every position is now in [a, a + max_len)
+  m <<= p - a;
+  uint32_t n = (uint32_t)__popcll(m);
+  if (n > (uint32_t)kCand) {
+    over[j] = 1;
+    n = kCand;
+  }
+  J.mask[i] = m;
+  uint8_t* const st = J.st;
+  uint8_t* const ex = J.ex;
+  uint16_t* const cnt = J.cnt;
+  for (uint32_t k = 0; k < n; k++) {
+    const uint32_t o = (uint32_t)__ffsll((long long)m) - 1;
+    m &= m - 1;
+    p = a + o;
+    uint32_t c = 0;
+    if (!dec_until(t, slut, ms, bits, p, end, c)) err[j] = 1;
+    const size_t at = (size_t)k * nseg + i;
+    st[at] = (uint8_t)o;
+    ex[at] = (uint8_t)(p > end ? p - end : 0);
+    cnt[at] = (uint16_t)c;
+  }
+}
+
+// One wave per stream; leaves at once unless the stream needs it. Lane 0 walks
+// the whole stream, so each of its segments has its one true start.
+__global__ void __launch_bounds__(64) k_dec_serial(MDecTable jobs, int* __restrict__ err, const int* __restrict__ over) {
+  __shared__ uint32_t slut[1 << kLutBits];
+  __shared__ uint32_t sw[kStageWords];
+  const int j = blockIdx.x;
+  const MDecJob& J = jobs[j];
+  if (!over[j]) return;
+  stage_lut(slut, J.t.lut);
+  const BlockBits bits{(lds_u32*)sw};
+  uint32_t o = 0;  // the next code, bits past the block's beginning
+  for (uint32_t b0 = 0; b0 < J.nseg; b0 += 256) {
+    const uint32_t pre = stage_words(sw, J.w, J.nbits, b0);
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      uint32_t p = pre + o;
+      for (uint32_t i = b0; i < min(b0 + 256, J.nseg); i++) {
+        const uint32_t a = pre + (i - b0) * kSegBits;
+        const uint32_t end = a + (uint32_t)min((uint64_t)kSegBits, J.nbits - (uint64_t)i * kSegBits);
+        J.mask[i] = 1;
+        J.st[i] = (uint8_t)(p - a);
+        uint32_t c = 0;
+        while (p < end) {
+          if (dec_one(J.t, slut, bits, p) == 0xFFFFFFFFu) {  // a bad code: the call fails, the walk ends
+            err[j] = 1;
+            p = end;
+          }
+          c++;
+        }
+        J.ex[i] = (uint8_t)(p - end);
+        J.cnt[i] = (uint16_t)c;
+      }
+      o = p - (pre + 256 * kSegBits);
+    }
+    __syncthreads();
+  }
+}
+
+// Where each possible start of a block's first segment leads. Most blocks hold
+// one start per segment: their counts are a sum. In the others lane k of the
+// first wave follows start k through the 256 segments, a table look-up each.
+__global__ void __launch_bounds__(256) k_dec_follow(MDecTable jobs) {
+  __shared__ uint64_t nx[256];            // the next segment's start for each of the segment's (4 bits each)
+  __shared__ uint16_t cn[kCand][256];
+  __shared__ uint8_t path[256][kCand];    // [segment][start of the block]
+  __shared__ uint8_t leads[kCand];
+  __shared__ int n_first;
+  __shared__ uint32_t wsum[4];
+  const MDecJob& J = jobs[jobs.of_block(blockIdx.x)];
+  const uint32_t blk = blockIdx.x - J.blk0, i = blk * 256 + threadIdx.x;
+  const uint32_t last = min(255u, J.nseg - 1 - blk * 256);  // last segment of the block
+  const bool valid = i < J.nseg;
+  const uint64_t m = valid ? J.mask[i] : 1, m1 = valid && i + 1 < J.nseg ? J.mask[i + 1] : 1;
+  const int n = min(__popcll(m), kCand);
+  auto next = [&](uint32_t e) { return m1 & (m1 - 1) ? (uint64_t)min(__popcll(m1 & ((1ull << e) - 1)), kCand - 1) : 0; };
+  uint64_t nxt = 0;
+  for (int k = 0; k < n; k++)
+    if (valid) nxt |= next(min((uint32_t)J.ex[(size_t)k * J.nseg + i], 63u)) << (4 * k);
+  if (!__syncthreads_or(n > 1)) {
+    uint32_t tot;
+    block_excl_scan(valid ? J.cnt[i] : 0u, wsum, tot);
+    if (threadIdx.x == last) J.bmap[blk] = nxt;
+    if (threadIdx.x == 0) {
+      J.btot[(size_t)blk * kCand] = tot;
+      J.bsel[blk] = 1u << 31;
+    }
     return;
   }
-  // New start: decode the new path and the previous pass's path of this
-  // segment in lockstep (always advancing the one behind) until they reach
-  // the same code boundary; from there both paths coincide, so the previous
-  // pass's exit and the rest of its count carry over. Prefix codes resync
-  // within a few code words, so a fix-up costs a few symbols, not a segment.
-  uint64_t ex = 0;
-  dec_resync(t, slut, ms, w, sw, lbase, lcount, end, s0, prev_start[i], prev_exit[i], cnt[i], ex, c, err);
-  start[i] = s0;
-  exitp[i] = ex;
-  cnt[i] = c;
-}
-
-__global__ void __launch_bounds__(256) k_dec_spec(DecTree t, const uint32_t* __restrict__ w, uint64_t nbits,
-                                                  uint32_t S, uint32_t nseg,
-                                                  const uint64_t* __restrict__ prev_exit,
-                                                  const uint64_t* __restrict__ prev_start,
-                                                  uint64_t* __restrict__ start, uint64_t* __restrict__ exitp,
-                                                  uint32_t* __restrict__ cnt, int* __restrict__ changed,
-                                                  int* __restrict__ err, int first) {
-  __shared__ uint32_t slut[1 << kLutBits];
-  __shared__ uint32_t sw[kStageWords];
-  __shared__ uint16_t ms[1 << kLutBits];
-  (void)changed;
-  dec_spec_block(t, w, nbits, S, nseg, prev_exit, prev_start, start, exitp, cnt, err, first, blockIdx.x, slut, sw,
-                 ms);
-}
-
-// ---- block-settled passes (the multi-stream decoder). A pass leaves every
-// block internally consistent: each segment but the block's first starts at
-// its predecessor's exit. So only the links between blocks need host rounds.
-
-// Decodes from s0 along the new path and along the old path of the segment
-// (start os, exit oe, count oc) in lockstep, always advancing the one behind,
-// until the two meet at a code boundary (from there they coincide, so the old
-// exit and the rest of its count carry over) or the new path reaches `end`.
-__device__ __forceinline__ void dec_resync(const DecTree& t, const uint32_t* slut, const uint16_t* ms,
-                                           const uint32_t* __restrict__ w, const uint32_t* sw, uint64_t lbase,
-                                           uint32_t lcount, uint64_t end, uint64_t s0, uint64_t os, uint64_t oe,
-                                           uint32_t oc, uint64_t& ex, uint32_t& c, int* __restrict__ err) {
-  BitReader br, old;
-  br.init(w, s0, sw, lbase, lcount);
-  old.init(w, os, sw, lbase, lcount);
-  uint32_t cn = 0, co = 0;
-  // A bounded lockstep: paths that have not met after kLock codes rarely meet
-  // soon (the codes resynchronize slowly there), so the new path then runs
-  // alone to `end` with multi-code steps, and its own count is the count.
-  constexpr int kLock = 48;
-  int steps = 0;
-  for (;;) {
-    if (br.pos >= end) {
-      ex = br.pos;
-      break;
-    }
-    if (br.pos == old.pos) {
-      ex = oe;
-      cn += oc - co;
-      break;
-    }
-    if (++steps > kLock) {
-      if (!dec_until(t, slut, ms, br, end, cn)) *err = 1;
-      ex = br.pos;
-      break;
-    }
-    const bool adv_new = br.pos < old.pos;
-    if (dec_one(t, slut, adv_new ? br : old) == 0xFFFFFFFFu) {
-      *err = 1;
-      ex = br.pos;
-      break;
-    }
-    cn += adv_new;
-    co += !adv_new;
-  }
-  c = cn;
-}
-
-// Settles a block: while some segment does not start at its predecessor's
-// exit, every such segment re-decodes from that exit (in parallel: a serial
-// fix of one segment at a time would leave all but one lane of the wave idle).
-// After iteration k the first k + 1 segments are final (the first one is
-// given), so blockDim iterations suffice; a segment that adopts a still-wrong
-// predecessor exit is corrected in a later iteration.
-// lex: blockDim LDS words.
-__device__ __forceinline__ void dec_settle(const DecTree& t, const uint32_t* slut, const uint16_t* ms,
-                                           const uint32_t* __restrict__ w, const uint32_t* sw, uint64_t lbase,
-                                           uint32_t lcount, uint64_t end, bool valid, uint64_t& st, uint64_t& ex,
-                                           uint32_t& c, uint64_t* lex, int* __restrict__ err) {
-  for (uint32_t it = 0; it < blockDim.x; it++) {
-    __syncthreads();
-    lex[threadIdx.x] = ex;
-    __syncthreads();
-    bool redo = false;
-    uint64_t want = 0;
-    if (valid && threadIdx.x > 0) {
-      want = lex[threadIdx.x - 1];
-      redo = want != st;
-    }
-    if (!__syncthreads_or(redo)) break;
-    if (redo) {
-      uint64_t e2;
-      uint32_t c2;
-      dec_resync(t, slut, ms, w, sw, lbase, lcount, end, want, st, ex, c, e2, c2, err);
-      st = want;
-      ex = e2;
-      c = c2;
-    }
-  }
-}
-
-__device__ __forceinline__ void dec_pass_block(const DecTree& t, const uint32_t* __restrict__ w, uint64_t nbits,
-                                               uint32_t S, uint32_t nseg, const uint64_t* __restrict__ prev_exit,
-                                               const uint64_t* __restrict__ prev_start,
-                                               uint64_t* __restrict__ start, uint64_t* __restrict__ exitp,
-                                               uint32_t* __restrict__ cnt, int* __restrict__ err, int first,
-                                               uint32_t blk, uint32_t* slut, uint32_t* sw, uint64_t* lex,
-                                               uint16_t* ms, uint64_t warm) {
-  const uint32_t i = blk * blockDim.x + threadIdx.x;
-  const bool valid = i < nseg;
-  uint64_t st = 0, ex = 0, s0 = 0;
-  uint32_t c = 0;
-  bool work;
-  if (first) {
-    work = valid;
-  } else {
-    // only a block whose first segment gets a new start changes
-    if (valid) {
-      st = prev_start[i];
-      ex = prev_exit[i];
-      c = cnt[i];
-    }
-    if (threadIdx.x == 0 && valid) s0 = i == 0 ? 0 : prev_exit[i - 1];
-    work = threadIdx.x == 0 && valid && s0 != st;
-    if (!__syncthreads_or(work)) {
-      if (valid) {
-        start[i] = st;
-        exitp[i] = ex;
-      }
-      return;
-    }
-  }
-  for (int k = threadIdx.x; k < (1 << kLutBits); k += blockDim.x) slut[k] = t.lut[k];
-  uint64_t lbase;
-  const uint32_t lcount = stage_words(sw, w, nbits, S, blk * blockDim.x, lbase);
+  nx[threadIdx.x] = nxt;
+  for (int k = 0; k < n; k++) cn[k][threadIdx.x] = valid ? J.cnt[(size_t)k * J.nseg + i] : 0;
+  if (threadIdx.x == 0) n_first = n;
   __syncthreads();
-  build_mstep(slut, ms);
-  __syncthreads();
-  uint64_t end = (uint64_t)(i + 1) * S;
-  if (end > nbits) end = nbits;
-  if (first && valid) {
-    // Warm-up: start `warm` bits before the segment and take as its start
-    // the first code boundary at or after i * S. A prefix-code path usually
-    // resyncs within a few code words, so this path is often already the true
-    // one there.
-    const uint64_t a = (uint64_t)i * S;
-    BitReader br;
-    br.init(w, a - (a < warm ? a : warm), sw, lbase, lcount);
-    uint32_t skipped = 0;
-    if (!dec_until(t, slut, ms, br, a, skipped)) *err = 1;
-    st = br.pos;
-    if (!dec_until(t, slut, ms, br, end, c)) *err = 1;
-    ex = br.pos;
-  } else if (work) {
-    uint64_t e2;
-    uint32_t c2;
-    dec_resync(t, slut, ms, w, sw, lbase, lcount, end, s0, st, ex, c, e2, c2, err);
-    st = s0;
-    ex = e2;
-    c = c2;
+  if (threadIdx.x < (uint32_t)n_first) {
+    uint32_t cur = threadIdx.x, tot = 0;
+    for (uint32_t s = 0; s <= last; s++) {
+      path[s][threadIdx.x] = (uint8_t)cur;
+      tot += cn[cur][s];
+      cur = (uint32_t)(nx[s] >> (4 * cur)) & 15u;
+    }
+    J.btot[(size_t)blk * kCand + threadIdx.x] = tot;
+    leads[threadIdx.x] = (uint8_t)cur;
   }
-  dec_settle(t, slut, ms, w, sw, lbase, lcount, end, valid, st, ex, c, lex, err);
+  __syncthreads();
+  uint64_t p = 0;
   if (valid) {
-    start[i] = st;
-    exitp[i] = ex;
-    cnt[i] = c;
-  }
-}
-
-// ---- multi-stream passes: block b belongs to the job j with
-// blk0[j] <= b < blk0[j + 1]; `cur` selects the ping-pong buffers.
-__device__ __forceinline__ int mdec_job(const uint32_t* __restrict__ blk0, int nj, uint32_t b) {
-  int lo = 0, hi = nj - 1;
-  while (lo < hi) {
-    const int mid = (lo + hi + 1) >> 1;
-    if (blk0[mid] <= b) lo = mid;
-    else hi = mid - 1;
-  }
-  return lo;
-}
-
-__global__ void __launch_bounds__(256) k_dec_spec_multi(const MDecJob* __restrict__ jobs,
-                                                        const uint32_t* __restrict__ blk0, int nj, int cur,
-                                                        int first, int* __restrict__ err) {
-  __shared__ uint32_t slut[1 << kLutBits];
-  __shared__ uint32_t sw[kStageWords];
-  __shared__ uint64_t lex[256];
-  __shared__ uint16_t ms[1 << kLutBits];
-  const int j = mdec_job(blk0, nj, blockIdx.x);
-  const MDecJob& J = jobs[j];
-  if (first)
-    dec_pass_block(J.t, J.w, J.nbits, J.S, J.nseg, nullptr, nullptr, J.start[0], J.ex[0], J.cnt, err + j, 1,
-                   blockIdx.x - blk0[j], slut, sw, lex, ms, J.warm);
-  else
-    dec_pass_block(J.t, J.w, J.nbits, J.S, J.nseg, J.ex[cur], J.start[cur], J.start[cur ^ 1], J.ex[cur ^ 1],
-                   J.cnt, err + j, 0, blockIdx.x - blk0[j], slut, sw, lex, ms, J.warm);
-}
-
-// changed[j] = 1 when a segment of job j does not start at its predecessor's exit
-__global__ void __launch_bounds__(256) k_dec_check_multi(const MDecJob* __restrict__ jobs,
-                                                         const uint32_t* __restrict__ blk0, int nj, int cur,
-                                                         int* __restrict__ changed) {
-  const int j = mdec_job(blk0, nj, blockIdx.x);
-  const MDecJob& J = jobs[j];
-  const uint32_t i = (blockIdx.x - blk0[j]) * blockDim.x + threadIdx.x;
-  if (i >= J.nseg) return;
-  const uint64_t want = i == 0 ? 0 : J.ex[cur][i - 1];
-  if (J.start[cur][i] != want) changed[j] = 1;
-}
-
-// Exclusive scan of the per-segment counts of every job, in three passes:
-// block sums, a scan of each job's block sums (one workgroup per job, which
-// also writes the job's total), then the in-block scans.
-__global__ void __launch_bounds__(256) k_dec_bsum_multi(const MDecJob* __restrict__ jobs,
-                                                        const uint32_t* __restrict__ blk0, int nj) {
-  __shared__ uint64_t red[256];
-  const int j = mdec_job(blk0, nj, blockIdx.x);
-  const MDecJob& J = jobs[j];
-  const uint32_t b = blockIdx.x - blk0[j];
-  const uint32_t i = b * blockDim.x + threadIdx.x;
-  red[threadIdx.x] = i < J.nseg ? J.cnt[i] : 0;
-  __syncthreads();
-  for (int s = 128; s > 0; s >>= 1) {
-    if ((int)threadIdx.x < s) red[threadIdx.x] += red[threadIdx.x + s];
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) J.bsum[b] = red[0];
-}
-
-__global__ void __launch_bounds__(256) k_dec_bscan_multi(const MDecJob* __restrict__ jobs, uint64_t* __restrict__ totals) {
-  __shared__ uint64_t sc[256];
-  const MDecJob& J = jobs[blockIdx.x];
-  uint64_t carry = 0;
-  for (uint32_t base = 0; base < J.nblk; base += 256) {
-    const uint32_t k = base + threadIdx.x;
-    const uint64_t v = k < J.nblk ? J.bsum[k] : 0;
-    sc[threadIdx.x] = v;
-    __syncthreads();
-    for (int s = 1; s < 256; s <<= 1) {  // inclusive Hillis-Steele scan
-      const uint64_t a = (int)threadIdx.x >= s ? sc[threadIdx.x - s] : 0;
-      __syncthreads();
-      sc[threadIdx.x] += a;
-      __syncthreads();
-    }
-    if (k < J.nblk) J.bsum[k] = carry + sc[threadIdx.x] - v;
-    carry += sc[255];
-    __syncthreads();
+    for (int k = 0; k < n_first; k++) p |= (uint64_t)path[threadIdx.x][k] << (4 * k);
+    J.sel[i] = p;
   }
   if (threadIdx.x == 0) {
-    J.off[J.nseg] = carry;
-    totals[blockIdx.x] = carry;
+    p = 0;
+    for (int k = 0; k < n_first; k++) p |= (uint64_t)leads[k] << (4 * k);
+    J.bmap[blk] = p;
+    J.bsel[blk] = 0;
   }
 }
 
-__global__ void __launch_bounds__(256) k_dec_off_multi(const MDecJob* __restrict__ jobs,
-                                                       const uint32_t* __restrict__ blk0, int nj) {
-  __shared__ uint64_t sc[256];
-  const int j = mdec_job(blk0, nj, blockIdx.x);
-  const MDecJob& J = jobs[j];
-  const uint32_t b = blockIdx.x - blk0[j];
-  const uint32_t i = b * blockDim.x + threadIdx.x;
-  const uint64_t v = i < J.nseg ? J.cnt[i] : 0;
-  sc[threadIdx.x] = v;
-  __syncthreads();
-  for (int s = 1; s < 256; s <<= 1) {
-    const uint64_t a = (int)threadIdx.x >= s ? sc[threadIdx.x - s] : 0;
-    __syncthreads();
-    sc[threadIdx.x] += a;
-    __syncthreads();
+// The true chain over a stream's blocks, 64 at a time: the maps of 64 blocks
+// (one per lane, the next 64 in flight) are followed with lane reads, then the
+// lanes fetch the chosen totals and sum them.
+__global__ void __launch_bounds__(64) k_dec_chain(MDecTable jobs, uint64_t* __restrict__ totals) {
+  const MDecJob& J = jobs[blockIdx.x];
+  const uint32_t lane = threadIdx.x, nblk = J.nblk;
+  uint32_t cur = 0;
+  uint64_t pos = 0;
+  // lanes past the last block lead nowhere and hold nothing
+  uint32_t one = lane < nblk ? J.bsel[lane] : 1u << 31;
+  uint64_t map = lane < nblk ? J.bmap[lane] : 0;
+  for (uint32_t b0 = 0; b0 < nblk; b0 += 64) {
+    const uint32_t b = b0 + lane, bn = b + 64;
+    const uint32_t one0 = one, lo = (uint32_t)map, hi = (uint32_t)(map >> 32);
+    one = bn < nblk ? J.bsel[bn] : 1u << 31;
+    map = bn < nblk ? J.bmap[bn] : 0;
+    uint32_t mine = 0;
+    if (__all(one0 >> 31)) {
+      cur = __builtin_amdgcn_readlane(lo, 63) & 15u;
+    } else {
+#pragma unroll
+      for (uint32_t k = 0; k < 64; k++) {
+        mine = lane == k ? cur : mine;
+        const uint64_t m = (uint64_t)(uint32_t)__builtin_amdgcn_readlane(hi, k) << 32 |
+                           (uint32_t)__builtin_amdgcn_readlane(lo, k);
+        cur = (uint32_t)(m >> (4 * cur)) & 15u;
+      }
+    }
+    const uint32_t tot = b < nblk ? J.btot[(size_t)b * kCand + mine] : 0u;
+    uint32_t incl = wave_incl_scan(tot);
+    if (b < nblk) {
+      J.bsel[b] = one0 | mine;
+      J.boff[b] = pos + incl - tot;
+    }
+    pos += __builtin_amdgcn_readlane(incl, 63);
   }
-  if (i < J.nseg) J.off[i] = J.bsum[b] + sc[threadIdx.x] - v;
-}
-
-__global__ void k_dec_check(uint32_t nseg, const uint64_t* exitp, const uint64_t* start,
-                            int* changed) {
-  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= nseg) return;
-  const uint64_t want = i == 0 ? 0 : exitp[i - 1];
-  if (start[i] != want) *changed = 1;
+  if (lane == 0) totals[blockIdx.x] = pos;
 }
 
 // Level-2 entry for the K bits u below `node`: sym << 8 | length of the leaf
@@ -526,6 +394,7 @@ DeviceDecoder upload_decoder(Ctx& ctx, const HostDecoder& hd, const char* tag) {
     out.single_sym = d.root_sym;
     return out;
   }
+  out.max_len = (uint32_t)d.max_len;
   const std::vector<uint32_t>& lut = hd.lut;
   const std::vector<uint32_t>& pfx = hd.pfx;
   const size_t n2 = hd.n2;
@@ -684,6 +553,7 @@ void upload_decoders(Ctx& ctx, const HostDecoder* const* hd, int n, DeviceDecode
     o.tree.leaf = da + 3 * arr_b;
     o.tree.lut2 = dl2 + l2base[k] / 4;
     o.tree.nodes = (uint32_t)N;
+    o.max_len = (uint32_t)h.d.max_len;
     if (h.n2) {
       Lut2Fill& f = hf[nf++];
       f.left = o.tree.left;

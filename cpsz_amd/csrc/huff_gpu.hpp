@@ -11,15 +11,17 @@
 //               chunk's codes MSB-first in LDS (lane offsets from a wave
 //               prefix sum) and stores 32-bit big-endian words coalesced; only
 //               the first and last (shared) word of a chunk use atomicOr
-//   decode    : self-synchronizing parallel decode of the single unchunked
-//               bitstream (speculative segment decode, fix-up rounds until every
-//               segment starts on its predecessor's exit, scan, final decode)
+//   decode    : parallel decode of the single unchunked bitstream: every code
+//               boundary that a segment can start on, given nothing but the
+//               bits before it; the exit and count from each; then the one true
+//               chain through them, and the final decode
 #pragma once
 #include <hip/hip_runtime.h>
 
 #include <rocprim/device/device_scan.hpp>
 #include <rocprim/iterator/transform_iterator.hpp>
 #include <cstring>
+#include <exception>
 #include <functional>
 #include <string>
 #include <type_traits>
@@ -33,8 +35,9 @@ namespace cpsz {
 
 constexpr int kLutBits = 11;
 constexpr int kLut2Bits = 12;  // width cap of the level-2 decode tables
-constexpr int kFixPerCheck = 2;   // fix-up passes queued per host convergence check
-constexpr uint64_t kDecWarm = 384;  // bits decoded before a segment in the speculative pass
+constexpr uint32_t kSegBits = 256;   // bits per decode segment
+constexpr uint32_t kWarmBits = 256;  // bits before a segment from which its possible starts are worked out
+constexpr int kCand = 16;            // possible starts kept per segment
 
 __device__ __forceinline__ uint32_t bswap32(uint32_t x) { return __builtin_bswap32(x); }
 
@@ -379,106 +382,82 @@ struct DecTree {
   uint32_t nodes;
 };
 
-// MSB-first reader over big-endian 32-bit words; the word array needs at
-// least two zero words past the last bit. Words [lbase, lbase + lcount) are
-// also staged in LDS (lw) and read from there: a refill is then an LDS read,
-// not a global-memory round trip on the decoder's serial dependency chain.
 typedef __attribute__((address_space(3))) const uint32_t lds_u32;  // an LDS word
 
-struct BitReader {
-  const uint32_t* w;
-  lds_u32* lw;
-  uint64_t lbase;
-  uint32_t lcount;
-  uint64_t buf;   // upcoming bits, MSB-aligned
-  int nb;         // valid bits in buf (> 32 after every refill)
-  uint64_t widx;  // next word to load
-  uint64_t pos;   // bit position of buf's MSB
-  __device__ __forceinline__ uint32_t word(uint64_t k) const {
-    const uint64_t d = k - lbase;
-    uint32_t x;
-    if (d < lcount) x = lw[d];
-    else x = w[k];
-    return bswap32(x);
-  }
-  __device__ __forceinline__ void init(const uint32_t* __restrict__ words, uint64_t p,
-                                       const uint32_t* staged = nullptr, uint64_t sbase = 0, uint32_t scount = 0) {
-    w = words;
-    lw = (lds_u32*)staged;
-    lbase = sbase;
-    lcount = scount;
-    pos = p;
-    widx = p >> 5;
-    const int s = (int)(p & 31);
-    buf = (((uint64_t)word(widx) << 32) | word(widx + 1)) << s;
-    nb = 64 - s;
-    widx += 2;
-    refill();
-  }
-  __device__ __forceinline__ void refill() {
-    if (nb <= 32) {
-      buf |= (uint64_t)word(widx++) << (32 - nb);
-      nb += 32;
-    }
-  }
-  __device__ __forceinline__ uint32_t peek() const { return (uint32_t)(buf >> 32); }
-  __device__ __forceinline__ void skip(int L) {
-    buf <<= L;
-    nb -= L;
-    pos += (uint64_t)L;
-    refill();
+// A block decodes 256 segments: their 2048 words, the words before them (the
+// first segment's warm-up) and a few past them (the last code's overrun, 64
+// bits, and one window) are staged in LDS, zeros beyond the stream. A staged
+// word is bit-reversed, the stream's first bit lowest, so that the 32 bits
+// from any position are one funnel shift of two neighbouring words: no bit
+// buffer to refill, 32-bit positions counted from the first staged bit, and no
+// read outside LDS.
+constexpr uint32_t kPreWords = kWarmBits / 32;
+constexpr uint32_t kStageWords = kPreWords + 256 * (kSegBits / 32) + 8;
+
+struct BlockBits {
+  lds_u32* w;
+  __device__ __forceinline__ uint32_t window(uint32_t p) const {
+    return __builtin_amdgcn_alignbit(w[(p >> 5) + 1], w[p >> 5], p & 31);
   }
 };
 
-// A block's 256 segments of 256 bits span 2048 words; the few words past them
-// cover the last segment's overrun to its first boundary past the end.
-constexpr uint32_t kStageWords = 2048 + 8;
-
-// Stages the words of block segments [b0, b0 + 256) (segment size S bits) into
-// sw; returns how many were staged (0 unless S == 256). Callers synchronize.
+// Stages the words of segments [b0, b0 + 256); returns the position of the
+// first of them. Callers synchronize.
 __device__ __forceinline__ uint32_t stage_words(uint32_t* sw, const uint32_t* __restrict__ w, uint64_t nbits,
-                                                uint32_t S, uint32_t b0, uint64_t& lbase) {
-  lbase = (uint64_t)b0 * (S / 32);
-  if (S != 256) return 0;
-  const uint64_t avail = (nbits + 31) / 32 + 8;  // words allocated, zero padded
-  uint32_t cnt = kStageWords;
-  if (lbase + cnt > avail) cnt = avail > lbase ? (uint32_t)(avail - lbase) : 0u;
-  for (uint32_t k = threadIdx.x; k < cnt; k += blockDim.x) sw[k] = w[lbase + k];
-  return cnt;
+                                                uint32_t b0) {
+  const uint32_t pre = b0 ? kPreWords : 0;
+  const uint64_t base = (uint64_t)b0 * (kSegBits / 32) - pre, have = (nbits + 31) / 32;
+  for (uint32_t k = threadIdx.x; k < kStageWords; k += blockDim.x)
+    sw[k] = base + k < have ? __brev(bswap32(w[base + k])) : 0u;
+  return pre * 32;
 }
 
-// Decodes one symbol; returns it or 0xFFFFFFFF on a bad code. `lut` is the
-// level-1 table (in LDS): sym << 8 | length for short codes, off << 8 | 0x80 |
-// K for prefixes continued by a level-2 table (t.lut2, global memory) over the
-// next K bits; codes longer still continue bit by bit down the tree.
-__device__ __forceinline__ uint32_t dec_one(const DecTree& t, const uint32_t* lut, BitReader& br) {
-  const uint32_t e = lut[br.peek() >> (32 - kLutBits)];
-  const uint32_t L = e & 0xFF;
-  if (L && !(L & 0x80u)) {
-    br.skip((int)L);
-    return e >> 8;
-  }
+// The level-1 table in the order of the windows' low bits. Callers synchronize.
+__device__ __forceinline__ void stage_lut(uint32_t* slut, const uint32_t* __restrict__ lut) {
+  for (uint32_t k = threadIdx.x; k < (1u << kLutBits); k += blockDim.x) slut[__brev(k) >> (32 - kLutBits)] = lut[k];
+}
+
+constexpr uint32_t kLutMask = (1u << kLutBits) - 1;
+
+// A level-1 entry is sym << 8 | length for short codes, off << 8 | 0x80 | K for
+// prefixes continued by a level-2 table (t.lut2, global memory) over the next
+// K bits; codes longer still continue bit by bit down the tree.
+__device__ __forceinline__ bool short_code(uint32_t e) { return (e & 0xFF) - 1 < 0x7F; }
+
+// The rest of the code whose level-1 entry at p is e: its symbol, or
+// 0xFFFFFFFF for a bad code. p moves past it, 64 bits at most.
+__device__ __forceinline__ uint32_t long_code(const DecTree& t, const BlockBits& bits, uint32_t e, uint32_t& p) {
   uint32_t node = e >> 8;
-  br.skip(kLutBits);
-  if (L & 0x80u) {
-    const int K = (int)(L & 0x7F);
-    const uint32_t e2 = t.lut2[node + (br.peek() >> (32 - K))];
+  p += kLutBits;
+  if (e & 0x80u) {
+    const int K = (int)(e & 0x7F);
+    const uint32_t e2 = t.lut2[node + (__brev(bits.window(p)) >> (32 - K))];
     const uint32_t L2 = e2 & 0xFF;
     if (L2) {
-      br.skip((int)L2);
+      p += L2;
       return e2 >> 8;
     }
     node = e2 >> 8;
-    br.skip(K);
+    p += (uint32_t)K;
   }
   for (int d = 0; d < 64; d++) {
-    const uint32_t b = br.peek() >> 31;
-    br.skip(1);
+    const uint32_t b = bits.window(p) & 1;
+    p++;
     node = b ? t.right[node] : t.left[node];
     if (node == 0 || node >= t.nodes) return 0xFFFFFFFFu;
     if (t.leaf[node]) return t.sym[node];
   }
   return 0xFFFFFFFFu;
+}
+
+// Decodes one symbol (0xFFFFFFFF: a bad code).
+__device__ __forceinline__ uint32_t dec_one(const DecTree& t, const uint32_t* slut, const BlockBits& bits, uint32_t& p) {
+  const uint32_t e = slut[bits.window(p) & kLutMask];
+  if (short_code(e)) {
+    p += e & 0xFF;
+    return e >> 8;
+  }
+  return long_code(t, bits, e, p);
 }
 
 // Multi-code steps for the passes that only locate code boundaries: for each
@@ -487,35 +466,40 @@ __device__ __forceinline__ uint32_t dec_one(const DecTree& t, const uint32_t* lu
 // stored as n << 8 | length (0 when the first code is longer). Built from the
 // level-1 table in LDS by the whole block; callers synchronize before use.
 __device__ __forceinline__ void build_mstep(const uint32_t* slut, uint16_t* ms) {
-  constexpr uint32_t kMask = (1u << kLutBits) - 1;
-  for (uint32_t w = threadIdx.x; w <= kMask; w += blockDim.x) {
+  for (uint32_t w = threadIdx.x; w <= kLutMask; w += blockDim.x) {
     uint32_t pos = 0, n = 0;
     for (;;) {
-      const uint32_t e = slut[(w << pos) & kMask];
-      const uint32_t L = e & 0xFF;
-      if (!L || (L & 0x80u) || pos + L > (uint32_t)kLutBits) break;
-      pos += L;
+      const uint32_t e = slut[w >> pos];
+      if (!short_code(e) || pos + (e & 0xFF) > (uint32_t)kLutBits) break;
+      pos += e & 0xFF;
       n++;
     }
     ms[w] = (uint16_t)(n << 8 | pos);
   }
 }
 
-// Decodes from br's position up to the first code boundary at or after
-// `stop`, adding the number of codes to c: a window's run of short codes at a
-// time while the run ends at or before `stop` (so no boundary at or after
+// Decodes from p up to the first code boundary at or after `stop`, adding the
+// number of codes to c: a window's run of short codes at a time (two from one
+// fetch) while the run ends at or before `stop` (so no boundary at or after
 // `stop` is stepped over), one code at a time otherwise. False on a bad code.
-__device__ __forceinline__ bool dec_until(const DecTree& t, const uint32_t* slut, const uint16_t* ms, BitReader& br,
-                                          uint64_t stop, uint32_t& c) {
-  while (br.pos < stop) {
-    const uint32_t m = ms[br.peek() >> (32 - kLutBits)];
-    const uint32_t len = m & 0xFF;
-    if (len && br.pos + len <= stop) {
-      br.skip((int)len);
+__device__ __forceinline__ bool dec_until(const DecTree& t, const uint32_t* slut, const uint16_t* ms,
+                                          const BlockBits& bits, uint32_t& p, uint32_t stop, uint32_t& c) {
+  while (p < stop) {
+    const uint32_t win = bits.window(p);
+    const uint32_t m = ms[win & kLutMask], len = m & 0xFF;
+    if (len && p + len <= stop) {
+      p += len;
       c += m >> 8;
+      const uint32_t m2 = ms[(win >> len) & kLutMask], len2 = m2 & 0xFF;
+      if (p + len2 <= stop) {  // (nothing to add if the next code is a long one)
+        p += len2;
+        c += m2 >> 8;
+      }
       continue;
     }
-    if (dec_one(t, slut, br) == 0xFFFFFFFFu) return false;
+    const uint32_t e = slut[win & kLutMask];
+    if (short_code(e)) p += e & 0xFF;
+    else if (long_code(t, bits, e, p) == 0xFFFFFFFFu) return false;
     c++;
   }
   return true;
@@ -525,156 +509,203 @@ __device__ __forceinline__ bool dec_until(const DecTree& t, const uint32_t* slut
 // up to 3 whole short codes: length | n << 4 | sym0 << 8 | sym1 << 16 | sym2 << 24
 // (n = 0 when the first code is longer than the window).
 __device__ __forceinline__ void build_mdec8(const uint32_t* slut, uint32_t* md) {
-  constexpr uint32_t kMask = (1u << kLutBits) - 1;
-  for (uint32_t w = threadIdx.x; w <= kMask; w += blockDim.x) {
+  for (uint32_t w = threadIdx.x; w <= kLutMask; w += blockDim.x) {
     uint32_t pos = 0, n = 0, syms = 0;
     while (n < 3) {
-      const uint32_t e = slut[(w << pos) & kMask];
-      const uint32_t L = e & 0xFF;
-      if (!L || (L & 0x80u) || pos + L > (uint32_t)kLutBits || (e >> 8) > 0xFFu) break;
+      const uint32_t e = slut[w >> pos];
+      if (!short_code(e) || pos + (e & 0xFF) > (uint32_t)kLutBits || (e >> 8) > 0xFFu) break;
       syms |= (e >> 8) << (8 * n);
-      pos += L;
+      pos += e & 0xFF;
       n++;
     }
     md[w] = pos | n << 4 | syms << 8;
   }
 }
 
-// Phase 1 / fix-up: decode from start to the first boundary >= seg_end.
-__global__ void __launch_bounds__(256) k_dec_spec(DecTree t, const uint32_t* __restrict__ w, uint64_t nbits,
-                                                  uint32_t S, uint32_t nseg, const uint64_t* __restrict__ prev_exit,
-                           const uint64_t* __restrict__ prev_start, uint64_t* __restrict__ start,
-                           uint64_t* __restrict__ exitp, uint32_t* __restrict__ cnt,
-                           int* __restrict__ changed, int* __restrict__ err, int first);
-
-__global__ void k_dec_check(uint32_t nseg, const uint64_t* exitp, const uint64_t* start,
-                            int* changed);
-
-// One bitstream of a multi-stream decode (every stream's segments in one grid):
-// its grid blocks are [blk0, blk0 + nblk); start/ex are the ping-pong buffers of
-// the passes, cnt the per-segment counts, off their exclusive scan (nseg + 1
-// entries) and bsum the per-block sums, then block offsets.
+// ---- finding the code boundaries. A segment's start (its first code boundary)
+// depends on everything before it, but only a few starts are possible: those
+// that some path reaches from one of the max_len bit positions kWarmBits
+// earlier. Paths merge within a few codes, so mostly one is left; where codes of
+// one length follow each other (runs of one symbol, near-uniform alphabets) up
+// to that length stay apart, however far back one begins, and a guessed start
+// would be wrong for the whole run.
+//   k_dec_cand    per segment: its possible starts, and from each the exit (first
+//                 boundary at or past the segment's end) and the code count
+//   k_dec_serial  streams in which some segment has more than kCand starts: the
+//                 true chain, one segment after the other
+//   k_dec_follow  per block of 256 segments: where each start of its first
+//                 segment leads, and the counts on the way
+//   k_dec_chain   per stream: the true start and output offset of every block
+// No pass waits for the host, and the result does not depend on how fast the
+// codes resynchronize.
 struct MDecJob {
   DecTree t;
   const uint32_t* w;
   uint64_t nbits, n;
-  uint32_t S, nseg, blk0, nblk;
-  uint32_t warm;  // bits decoded before a segment in the speculative pass
-  uint64_t* start[2];
-  uint64_t* ex[2];
-  uint32_t* cnt;
-  uint64_t* off;
-  uint64_t* bsum;
+  uint32_t nseg, nblk, blk0, max_len;
+  uint64_t* mask;   // per segment: possible starts (bit o: o bits past its beginning)
+  uint8_t* st;      // [kCand][nseg] the same as offsets
+  uint8_t* ex;      // [kCand][nseg] exit, bits past the segment's end
+  uint16_t* cnt;    // [kCand][nseg] codes
+  uint64_t* sel;    // per segment: the start (4 bits) that each start of its block's first segment leads to
+  uint64_t* bmap;   // per block: the next block's start for each of its own (4 bits each)
+  uint32_t* btot;   // [nblk][kCand] codes from each
+  uint32_t* bsel;   // per block: the true start; bit 31: all its segments have one start
+  uint64_t* boff;   // per block: the first code's position
 };
 template <class Sink>
 struct MDecJobS {
   MDecJob j;
   Sink sink;
 };
-__global__ void k_dec_spec_multi(const MDecJob* jobs, const uint32_t* blk0, int nj, int cur, int first, int* err);
-__global__ void k_dec_check_multi(const MDecJob* jobs, const uint32_t* blk0, int nj, int cur, int* changed);
-__global__ void k_dec_bsum_multi(const MDecJob* jobs, const uint32_t* blk0, int nj);
-__global__ void k_dec_bscan_multi(const MDecJob* jobs, uint64_t* totals);
-__global__ void k_dec_off_multi(const MDecJob* jobs, const uint32_t* blk0, int nj);
+// A table of MDecJob at the start of larger elements.
+struct MDecTable {
+  const char* base;
+  size_t stride;
+  const uint32_t* blk0;  // first block of each job, nj + 1 entries
+  int nj;
+  __device__ __forceinline__ const MDecJob& operator[](int j) const { return *(const MDecJob*)(base + (size_t)j * stride); }
+  __device__ __forceinline__ int of_block(uint32_t b) const {
+    int lo = 0, hi = nj - 1;
+    while (lo < hi) {
+      const int mid = (lo + hi + 1) >> 1;
+      if (blk0[mid] <= b) lo = mid;
+      else hi = mid - 1;
+    }
+    return lo;
+  }
+};
+__global__ void k_dec_cand(MDecTable jobs, int* err, int* over);
+__global__ void k_dec_serial(MDecTable jobs, int* err, const int* over);
+__global__ void k_dec_follow(MDecTable jobs);
+__global__ void k_dec_chain(MDecTable jobs, uint64_t* totals);
 
-// Phase 3: decode every segment into its final position. The symbols of a
+// Decode every segment into its final position. The symbols of a
 // block's 256 consecutive segments are contiguous in the output: they are
 // gathered in LDS and written out by consecutive threads (coalesced), instead
 // of each thread storing its own run one symbol at a time (64 scattered
 // 2-byte stores per instruction, which reach HBM as ~15x the bytes). A block
 // whose run exceeds the staging buffer writes directly. Sink::kBytes (1 or 2)
-// is the width of a staged symbol.
+// is the width of a staged symbol. Bound by the decode's LDS latency, then by
+// the sinks' index arithmetic: 96 fields' ids 1.85 -> 1.56 ms and codes
+// 2.97 -> 2.38 ms with several codes from one fetched window in place of a bit
+// buffer refilled under a branch.
 template <int kBytes>
 struct DecStage {
   using T = typename std::conditional<kBytes == 1, uint8_t, uint16_t>::type;
   static constexpr uint32_t kCap = kBytes == 1 ? 32768 : 12288;  // symbols per block
 };
 
-template <class Sink>
-__device__ __forceinline__ void dec_write_block(const DecTree& t, const uint32_t* __restrict__ w, uint64_t nbits,
-                                                uint32_t S, uint32_t nseg, const uint64_t* __restrict__ start,
-                                                const uint64_t* __restrict__ exitp,
-                                                const uint64_t* __restrict__ off, uint64_t n, const Sink& sink,
-                                                uint32_t blk, uint32_t* slut, uint32_t* sw,
-                                                typename DecStage<Sink::kBytes>::T* stage, uint32_t* md) {
-  using Stage = DecStage<Sink::kBytes>;
-  for (int k = threadIdx.x; k < (1 << kLutBits); k += blockDim.x) slut[k] = t.lut[k];
-  uint64_t lbase;
-  const uint32_t lcount = stage_words(sw, w, nbits, S, blk * blockDim.x, lbase);
+// Exclusive scan of the block's 256 values (x of thread 255 is the last);
+// tot receives the sum.
+__device__ __forceinline__ uint32_t block_excl_scan(uint32_t x, uint32_t* wsum, uint32_t& tot) {
+  const uint32_t incl = wave_incl_scan(x);
+  const int wv = threadIdx.x >> 6;
+  if ((threadIdx.x & 63) == 63) wsum[wv] = incl;
   __syncthreads();
+  uint32_t before = 0, all = 0;
+#pragma unroll
+  for (int k = 0; k < 4; k++) {
+    const uint32_t v = wsum[k];
+    before += k < wv ? v : 0u;
+    all += v;
+  }
+  tot = all;
+  return before + incl - x;
+}
+
+template <class Sink>
+__device__ __forceinline__ void dec_write_block(const MDecJob& J, const Sink& sink, uint32_t blk, uint32_t* slut,
+                                                uint32_t* sw, typename DecStage<Sink::kBytes>::T* stage, uint32_t* md,
+                                                uint32_t* wsum) {
+  using Stage = DecStage<Sink::kBytes>;
+  const DecTree t = J.t;  // (and the sink below: LDS stores may alias what a reference reaches)
+  const Sink out = sink;
+  stage_lut(slut, t.lut);
+  const uint32_t b0 = blk * 256, i = b0 + threadIdx.x;
+  const BlockBits bits{(lds_u32*)sw};
+  const uint32_t pre = stage_words(sw, J.w, J.nbits, b0);
+  // the segment's start, exit and count on the true chain
+  uint32_t p = 0, end = 0, codes = 0;
+  const uint32_t bs = J.bsel[blk];
+  if (i < J.nseg) {
+    const uint32_t c = bs >> 31 ? 0u : (uint32_t)(J.sel[i] >> (4 * bs)) & 15u;
+    const size_t at = (size_t)c * J.nseg + i;
+    p = pre + threadIdx.x * kSegBits + J.st[at];
+    end = pre + (uint32_t)(min((uint64_t)(i + 1) * kSegBits, J.nbits) - (uint64_t)b0 * kSegBits) + J.ex[at];
+    codes = J.cnt[at];
+  }
+  const uint64_t n = J.n, first = J.boff[blk];
+  uint32_t tot;
+  uint32_t o = block_excl_scan(codes, wsum, tot);  // synchronizes
+  if (first >= n) return;
   if (Sink::kBytes == 1) {
     build_mdec8(slut, md);
     __syncthreads();
   }
-  const uint32_t b0 = blk * blockDim.x;
-  const uint32_t b1 = min(b0 + blockDim.x, nseg);  // off[] holds nseg + 1 entries
-  const uint64_t o_begin = min(off[b0], n), o_end = min(off[b1], n);
-  const bool staged = o_end - o_begin <= (uint64_t)Stage::kCap;
-  const uint32_t i = b0 + threadIdx.x;
-  if (i < nseg) {
-    BitReader br;
-    br.init(w, start[i], sw, lbase, lcount);
-    const uint64_t end = exitp[i];
-    uint64_t o = off[i];
-    if (staged) {
-      if (Sink::kBytes == 1) {
-        // up to 3 codes per step while they all start before `end` and fit
-        while (br.pos < end && o < o_end) {
-          const uint32_t m = md[br.peek() >> (32 - kLutBits)];
-          const uint32_t len = m & 0xF, k = (m >> 4) & 3;
-          if (k && br.pos + len <= end && o + k <= o_end) {
-            typename Stage::T* d = stage + (o - o_begin);
-            d[0] = (typename Stage::T)(m >> 8);
-            if (k > 1) d[1] = (typename Stage::T)(m >> 16);
-            if (k > 2) d[2] = (typename Stage::T)(m >> 24);
-            o += k;
-            br.skip((int)len);
-          } else {
-            stage[o++ - o_begin] = (typename Stage::T)dec_one(t, slut, br);
-          }
-        }
-      } else {
-        while (br.pos < end && o < o_end) stage[o++ - o_begin] = (typename Stage::T)dec_one(t, slut, br);
+  const uint32_t limit = (uint32_t)min((uint64_t)tot, n - first);
+  if (limit > Stage::kCap) {  // uniform across the block
+    while (p < end && o < limit) out.put(first + o++, dec_one(t, slut, bits, p));
+    return;
+  }
+  using S = typename Stage::T;
+  if (Sink::kBytes == 1) {
+    // up to 6 codes per fetch while they all start before `end` and fit
+    while (p < end && o < limit) {
+      uint32_t win = bits.window(p);
+      bool none = true;
+#pragma unroll
+      for (int r = 0; r < 2; r++) {
+        const uint32_t m = md[win & kLutMask];
+        const uint32_t len = m & 0xF, k = (m >> 4) & 3;
+        if (!k || p + len > end || o + k > limit) break;
+        S* d = stage + o;
+        d[0] = (S)(m >> 8);
+        if (k > 1) d[1] = (S)(m >> 16);
+        if (k > 2) d[2] = (S)(m >> 24);
+        o += k;
+        p += len;
+        win >>= len;
+        none = false;
       }
-    } else {
-      while (br.pos < end && o < n) sink.put(o++, dec_one(t, slut, br));
+      if (none) stage[o++] = (S)dec_one(t, slut, bits, p);
+    }
+  } else {
+    // up to 3 codes per fetch
+    while (p < end && o < limit) {
+      const uint32_t win = bits.window(p);
+      uint32_t e = slut[win & kLutMask];
+      if (!short_code(e)) {
+        stage[o++] = (S)long_code(t, bits, e, p);
+        continue;
+      }
+      uint32_t used = e & 0xFF;
+      stage[o++] = (S)(e >> 8);
+      p += used;
+#pragma unroll
+      for (int r = 0; r < 2; r++) {
+        e = slut[(win >> used) & kLutMask];
+        if (p >= end || o >= limit || !short_code(e) || used > 32 - kLutBits) break;
+        stage[o++] = (S)(e >> 8);
+        used += e & 0xFF;
+        p += e & 0xFF;
+      }
     }
   }
-  if (!staged) return;  // uniform across the block
   __syncthreads();
-  const uint32_t cnt = (uint32_t)(o_end - o_begin);
-  for (uint32_t x = threadIdx.x; x < cnt; x += blockDim.x) sink.put(o_begin + x, stage[x]);
+  for (uint32_t x = threadIdx.x; x < limit; x += blockDim.x) out.put(first + x, stage[x]);
 }
 
 template <class Sink>
-__global__ void __launch_bounds__(256) k_dec_write(DecTree t, const uint32_t* __restrict__ w, uint64_t nbits,
-                                                   uint32_t S, uint32_t nseg, const uint64_t* __restrict__ start,
-                                                   const uint64_t* __restrict__ exitp,
-                                                   const uint64_t* __restrict__ off, uint64_t n,
-                                                   Sink sink) {
+__global__ void __launch_bounds__(256) k_dec_write(MDecTable jobs) {
   __shared__ uint32_t slut[1 << kLutBits];
   __shared__ uint32_t sw[kStageWords];
   __shared__ typename DecStage<Sink::kBytes>::T stage[DecStage<Sink::kBytes>::kCap];
   __shared__ uint32_t md[Sink::kBytes == 1 ? (1 << kLutBits) : 1];
-  dec_write_block(t, w, nbits, S, nseg, start, exitp, off, n, sink, blockIdx.x, slut, sw, stage, md);
-}
-
-template <class Sink>
-__global__ void __launch_bounds__(256) k_dec_write_multi(const MDecJobS<Sink>* __restrict__ jobs,
-                                                         const uint32_t* __restrict__ blk0, int nj, int cur) {
-  __shared__ uint32_t slut[1 << kLutBits];
-  __shared__ uint32_t sw[kStageWords];
-  __shared__ typename DecStage<Sink::kBytes>::T stage[DecStage<Sink::kBytes>::kCap];
-  __shared__ uint32_t md[Sink::kBytes == 1 ? (1 << kLutBits) : 1];
-  int lo = 0, hi = nj - 1;  // the job owning this block
-  while (lo < hi) {
-    const int mid = (lo + hi + 1) >> 1;
-    if (blk0[mid] <= blockIdx.x) lo = mid;
-    else hi = mid - 1;
-  }
-  const MDecJob& J = jobs[lo].j;
-  dec_write_block(J.t, J.w, J.nbits, J.S, J.nseg, J.start[cur], J.ex[cur], J.off, J.n, jobs[lo].sink,
-                  blockIdx.x - J.blk0, slut, sw, stage, md);
+  __shared__ uint32_t wsum[4];
+  const int j = jobs.of_block(blockIdx.x);
+  const MDecJobS<Sink>& J = *(const MDecJobS<Sink>*)&jobs[j];
+  dec_write_block(J.j, J.sink, blockIdx.x - J.j.blk0, slut, sw, stage, md, wsum);
 }
 
 template <class Sink>
@@ -695,6 +726,7 @@ void upload_codebook(Ctx& ctx, const HuffEncodeTable& t, uint64_t* d_code, uint8
 
 struct DeviceDecoder {
   DecTree tree{};
+  uint32_t max_len = 0;  // longest code
   bool single = false;
   uint32_t single_sym = 0;
 };
@@ -732,145 +764,53 @@ constexpr uint32_t kStageBlockWords = 2048;
 void stage_bits_multi(Ctx& ctx, BitsCopy* c, int n, const char* tag);
 
 // One bitstream to decode: n symbols of words already copied to aligned
-// device words (padded with at least 8 zero bytes) into `sink`; `tag` names
-// its buffers.
+// device words (padded with at least 8 zero words) into `sink`.
 template <class Sink>
 struct DecJob {
   const DeviceDecoder* dd;
   const uint32_t* words;
   uint64_t nbytes, n;
   Sink sink;
-  const char* tag;
-  // speculative warm-up in bits (0: kDecWarm); codes of a few bits that
-  // resynchronize slowly want a longer one (multi-code steps keep it cheap)
-  uint32_t warm = 0;
 };
 
-// Decodes several independent bitstreams in lockstep on the context's stream:
-// their passes are queued together, so one host check serves every stream of
-// a round, and one read of the totals serves all. `overlap` (may be empty) is
-// host work run once the first round is queued, before the first wait.
-template <class Sink>
-void decode_streams(Ctx& ctx, DecJob<Sink>* jobs, int nj, const std::function<void()>& overlap = {}) {
-  hipStream_t st = ctx.stream();
-  struct State {
-    uint64_t nbits = 0;
-    uint32_t S = 256, nseg = 0;
-    int blocks = 0, cur = 0;
-    bool active = false, done = false;
-    uint64_t *start[2] = {nullptr, nullptr}, *ex[2] = {nullptr, nullptr}, *off = nullptr;
-    uint32_t* cnt = nullptr;
-    int* flags = nullptr;
-  };
-  std::vector<State> sv(nj);
-  bool overlapped = false;
-  auto run_overlap = [&] {
-    if (!overlapped && overlap) {
-      overlapped = true;
-      overlap();
-    }
-  };
-  for (int k = 0; k < nj; k++) {
-    const DecJob<Sink>& j = jobs[k];
-    State& s = sv[k];
-    if (j.n == 0) continue;
-    if (j.dd->single) {
-      k_dec_const<<<1024, 256, 0, st>>>(j.n, j.dd->single_sym, j.sink);
-      CPSZ_HIP(hipGetLastError());
-      continue;
-    }
-    s.nbits = j.nbytes * 8;
-    CPSZ_REQUIRE(s.nbits > 0, kErrStream, "empty huffman bitstream for a multi-symbol tree");
-    while (div_up(s.nbits, s.S) > (1u << 21)) s.S *= 2;
-    s.nseg = (uint32_t)div_up(s.nbits, s.S);
-    const std::string t(j.tag);
-    s.start[0] = ctx.buf<uint64_t>((t + ".st0").c_str(), s.nseg);
-    s.start[1] = ctx.buf<uint64_t>((t + ".st1").c_str(), s.nseg);
-    s.ex[0] = ctx.buf<uint64_t>((t + ".ex0").c_str(), s.nseg);
-    s.ex[1] = ctx.buf<uint64_t>((t + ".ex1").c_str(), s.nseg);
-    s.cnt = ctx.buf<uint32_t>((t + ".cnt").c_str(), s.nseg);
-    s.off = ctx.buf<uint64_t>((t + ".off").c_str(), s.nseg + 1);
-    s.flags = ctx.buf<int>((t + ".flags").c_str(), 2);
-    s.blocks = (int)div_up(s.nseg, 256);
-    s.active = true;
-    CPSZ_HIP(hipMemsetAsync(s.flags, 0, 2 * sizeof(int), st));
-    k_dec_spec<<<s.blocks, 256, 0, st>>>(j.dd->tree, j.words, s.nbits, s.S, s.nseg, nullptr, nullptr, s.start[0],
-                                         s.ex[0], s.cnt, s.flags, s.flags + 1, 1);
-    CPSZ_HIP(hipGetLastError());
-  }
-  int* hflags = (int*)ctx.host_buf("dec.hflags", 2 * sizeof(int) * (size_t)(nj > 0 ? nj : 1));
-  for (int round = 0; round < 4096; round++) {
-    bool any = false;
-    for (int k = 0; k < nj; k++) {
-      State& s = sv[k];
-      if (!s.active || s.done) continue;
-      const DecJob<Sink>& j = jobs[k];
-      // kFixPerCheck fix-up rounds per host check
-      for (int r = 0; r < kFixPerCheck; r++) {
-        k_dec_spec<<<s.blocks, 256, 0, st>>>(j.dd->tree, j.words, s.nbits, s.S, s.nseg, s.ex[s.cur],
-                                             s.start[s.cur], s.start[s.cur ^ 1], s.ex[s.cur ^ 1], s.cnt, s.flags,
-                                             s.flags + 1, 0);
-        s.cur ^= 1;
-      }
-      CPSZ_HIP(hipMemsetAsync(s.flags, 0, sizeof(int), st));
-      k_dec_check<<<s.blocks, 256, 0, st>>>(s.nseg, s.ex[s.cur], s.start[s.cur], s.flags);
-      CPSZ_HIP(hipMemcpyAsync(hflags + 2 * k, s.flags, 2 * sizeof(int), hipMemcpyDeviceToHost, st));
-      any = true;
-    }
-    run_overlap();
-    if (!any) break;
-    CPSZ_HIP(hipStreamSynchronize(st));
-    for (int k = 0; k < nj; k++) {
-      State& s = sv[k];
-      if (!s.active || s.done) continue;
-      CPSZ_REQUIRE(hflags[2 * k + 1] == 0, kErrStream, "invalid huffman code in stream");
-      if (!hflags[2 * k]) s.done = true;
+// What a decode found, to be looked at once the stream has passed it.
+struct DecodeResult {
+  const uint64_t* totals = nullptr;  // pinned: codes found per stream
+  const int* err = nullptr;          // pinned
+  std::vector<uint64_t> want;
+  void check() const {
+    for (size_t k = 0; k < want.size(); k++) {
+      CPSZ_REQUIRE(err[k] == 0, kErrStream, "invalid huffman code in stream");
+      CPSZ_REQUIRE(totals[k] >= want[k], kErrStream, "huffman bitstream holds fewer symbols than expected");
     }
   }
-  run_overlap();
-  // a stream whose segment starts have not settled within the round limit
-  // would decode from inconsistent starts: refuse it
-  for (int k = 0; k < nj; k++)
-    CPSZ_REQUIRE(!sv[k].active || sv[k].done, kErrStream,
-                 "huffman decode did not converge (bitstream does not resynchronize)");
-  uint64_t* htot = (uint64_t*)ctx.host_buf("dec.htotals", sizeof(uint64_t) * (size_t)(nj > 0 ? nj : 1));
-  bool any = false;
-  for (int k = 0; k < nj; k++) {
-    State& s = sv[k];
-    if (!s.active) continue;
-    scan_u32_to_u64(ctx, s.cnt, s.off, s.nseg, s.off + s.nseg);
-    CPSZ_HIP(hipMemcpyAsync(htot + k, s.off + s.nseg, sizeof(uint64_t), hipMemcpyDeviceToHost, st));
-    any = true;
-  }
-  if (!any) return;
-  CPSZ_HIP(hipStreamSynchronize(st));
-  for (int k = 0; k < nj; k++)
-    if (sv[k].active)
-      CPSZ_REQUIRE(htot[k] >= jobs[k].n, kErrStream, "huffman bitstream holds fewer symbols than expected");
-  for (int k = 0; k < nj; k++) {
-    const State& s = sv[k];
-    if (!s.active) continue;
-    const DecJob<Sink>& j = jobs[k];
-    k_dec_write<<<s.blocks, 256, 0, st>>>(j.dd->tree, j.words, s.nbits, s.S, s.nseg, s.start[s.cur], s.ex[s.cur],
-                                          s.off, j.n, j.sink);
-    CPSZ_HIP(hipGetLastError());
-  }
-}
+};
 
-// Decodes many independent bitstreams with every stream's segments in one grid
-// per pass: one launch per pass for all streams, one host check per round
-// (the streams whose segments have settled pass through unchanged), a
-// three-launch scan of all streams' counts and one write launch. `tag` names
-// the buffers (one arena for all streams).
+// Waits for the stream when a call is left by an exception, so that nothing
+// queued still reads the caller's buffers after it.
+struct SettleOnThrow {
+  hipStream_t st;
+  int before = std::uncaught_exceptions();
+  ~SettleOnThrow() {
+    if (std::uncaught_exceptions() > before) (void)hipStreamSynchronize(st);
+  }
+};
+
+// Decodes many independent bitstreams, every stream's segments in one grid per
+// pass. Queues all passes on the context's stream and returns without waiting;
+// whatever the streams hold, the sinks get positions below n only. `tag` names
+// the buffers: one decode per tag until its result has been checked.
 template <class Sink>
-void decode_streams_multi(Ctx& ctx, const DecJob<Sink>* jobs, int nj, const char* tag) {
+DecodeResult decode_streams(Ctx& ctx, const DecJob<Sink>* jobs, int nj, const char* tag) {
   hipStream_t st = ctx.stream();
+  DecodeResult res;
   std::vector<int> act;
   for (int k = 0; k < nj; k++) {
     const DecJob<Sink>& j = jobs[k];
     if (j.n == 0) continue;
     if (j.dd->single) {
-      k_dec_const<<<1024, 256, 0, st>>>(j.n, j.dd->single_sym, j.sink);
+      k_dec_const<<<(unsigned)std::min<uint64_t>(div_up(j.n, (uint64_t)256), 1024), 256, 0, st>>>(
+          j.n, j.dd->single_sym, j.sink);
       CPSZ_HIP(hipGetLastError());
       continue;
     }
@@ -878,33 +818,39 @@ void decode_streams_multi(Ctx& ctx, const DecJob<Sink>* jobs, int nj, const char
     act.push_back(k);
   }
   const int na = (int)act.size();
-  if (!na) return;
-  std::vector<MDecJobS<Sink>> h(na);
-  std::vector<uint32_t> blk0(na + 1, 0);
-  size_t arena = 0;
+  if (!na) return res;
   auto al = [](size_t b) { return (b + 255) & ~(size_t)255; };
+  const std::string t(tag);
+  // the job table, block starts and (zero) flags travel in one copy
+  const size_t tb = al(na * sizeof(MDecJobS<Sink>)), bb = al((na + 1) * 4), fb = al(2 * na * 4), ob = na * 8;
+  uint8_t* hh = (uint8_t*)ctx.host_table((t + ".tab").c_str(), tb + bb + fb);
+  uint8_t* dt = ctx.buf<uint8_t>((t + ".tab").c_str(), tb + bb + fb + ob);
+  MDecJobS<Sink>* h = (MDecJobS<Sink>*)hh;
+  uint32_t* blk0 = (uint32_t*)(hh + tb);
+  blk0[0] = 0;
+  size_t arena = 0;
   for (int a = 0; a < na; a++) {
     const DecJob<Sink>& j = jobs[act[a]];
     MDecJob& m = h[a].j;
     m = MDecJob{};
     m.t = j.dd->tree;
+    m.max_len = j.dd->max_len;
     m.w = j.words;
     m.nbits = j.nbytes * 8;
     m.n = j.n;
-    m.S = 256;
-    m.warm = j.warm ? j.warm : (uint32_t)kDecWarm;
-    while (div_up(m.nbits, (uint64_t)m.S) > (1u << 21)) m.S *= 2;
-    m.nseg = (uint32_t)div_up(m.nbits, (uint64_t)m.S);
+    const uint64_t nseg = div_up(m.nbits, (uint64_t)kSegBits);
+    CPSZ_REQUIRE(nseg < (1ull << 31) && (uint64_t)blk0[a] + div_up(nseg, (uint64_t)256) < (1ull << 31), kErrUnsupported,
+                 "huffman decode: too many segments");
+    m.nseg = (uint32_t)nseg;
     m.nblk = (uint32_t)div_up(m.nseg, 256u);
     m.blk0 = blk0[a];
-    CPSZ_REQUIRE((uint64_t)blk0[a] + m.nblk < (1ull << 31), kErrUnsupported, "huffman decode: too many segments");
     blk0[a + 1] = blk0[a] + m.nblk;
     h[a].sink = j.sink;
-    arena += 4 * al(8 * (size_t)m.nseg) + al(4 * (size_t)m.nseg) + al(8 * ((size_t)m.nseg + 1)) +
-             al(8 * (size_t)m.nblk);
+    res.want.push_back(j.n);
+    arena += 2 * al(8 * (size_t)m.nseg) + 2 * al(kCand * (size_t)m.nseg) + al(2 * kCand * (size_t)m.nseg) +
+             2 * al(8 * (size_t)m.nblk) + al(4 * kCand * (size_t)m.nblk) + al(4 * (size_t)m.nblk);
   }
-  const uint32_t nblocks = blk0[na];
-  uint8_t* d = ctx.buf<uint8_t>((std::string(tag) + ".arena").c_str(), arena);
+  uint8_t* d = ctx.buf<uint8_t>((t + ".arena").c_str(), arena);
   for (int a = 0; a < na; a++) {
     MDecJob& m = h[a].j;
     auto take = [&](size_t bytes) {
@@ -912,84 +858,45 @@ void decode_streams_multi(Ctx& ctx, const DecJob<Sink>* jobs, int nj, const char
       d += al(bytes);
       return q;
     };
-    m.start[0] = (uint64_t*)take(8 * (size_t)m.nseg);
-    m.start[1] = (uint64_t*)take(8 * (size_t)m.nseg);
-    m.ex[0] = (uint64_t*)take(8 * (size_t)m.nseg);
-    m.ex[1] = (uint64_t*)take(8 * (size_t)m.nseg);
-    m.cnt = (uint32_t*)take(4 * (size_t)m.nseg);
-    m.off = (uint64_t*)take(8 * ((size_t)m.nseg + 1));
-    m.bsum = (uint64_t*)take(8 * (size_t)m.nblk);
+    m.mask = (uint64_t*)take(8 * (size_t)m.nseg);
+    m.sel = (uint64_t*)take(8 * (size_t)m.nseg);
+    m.st = (uint8_t*)take(kCand * (size_t)m.nseg);
+    m.ex = (uint8_t*)take(kCand * (size_t)m.nseg);
+    m.cnt = (uint16_t*)take(2 * kCand * (size_t)m.nseg);
+    m.bmap = (uint64_t*)take(8 * (size_t)m.nblk);
+    m.boff = (uint64_t*)take(8 * (size_t)m.nblk);
+    m.btot = (uint32_t*)take(4 * kCand * (size_t)m.nblk);
+    m.bsel = (uint32_t*)take(4 * (size_t)m.nblk);
   }
-  // job table, block starts and flags travel in one copy each way
-  const size_t tb = al(na * sizeof(MDecJobS<Sink>)), bb = al((na + 1) * 4), fb = al(2 * na * 4), ob = na * 8;
-  const std::string t(tag);
-  uint8_t* hh = (uint8_t*)ctx.host_buf((t + ".tab").c_str(), tb + bb + fb + ob);
-  std::memcpy(hh, h.data(), na * sizeof(MDecJobS<Sink>));
-  std::memcpy(hh + tb, blk0.data(), (na + 1) * 4);
-  uint8_t* dt = ctx.buf<uint8_t>((t + ".tab").c_str(), tb + bb + fb + ob);
-  CPSZ_HIP(hipMemcpyAsync(dt, hh, tb + bb, hipMemcpyHostToDevice, st));
-  const MDecJobS<Sink>* djs = (const MDecJobS<Sink>*)dt;
-  // MDecJobS<Sink> starts with its MDecJob, so a stride-aware view is needed
-  // for the Sink-agnostic kernels: they take an MDecJob table of their own
-  std::vector<MDecJob> hj(na);
-  for (int a = 0; a < na; a++) hj[a] = h[a].j;
-  MDecJob* dj = ctx.buf<MDecJob>((t + ".jobs").c_str(), na);
-  uint8_t* hjb = (uint8_t*)ctx.host_buf((t + ".jobs").c_str(), na * sizeof(MDecJob));
-  std::memcpy(hjb, hj.data(), na * sizeof(MDecJob));
-  CPSZ_HIP(hipMemcpyAsync(dj, hjb, na * sizeof(MDecJob), hipMemcpyHostToDevice, st));
-  const uint32_t* dblk0 = (const uint32_t*)(dt + tb);
-  int* changed = (int*)(dt + tb + bb);
-  int* err = changed + na;
+  std::memset(hh + tb + bb, 0, fb);
+  const uint32_t nblocks = blk0[na];
+  ctx.upload_table((t + ".tab").c_str(), dt, hh, tb + bb + fb);
+  const MDecTable tab{(const char*)dt, sizeof(MDecJobS<Sink>), (const uint32_t*)(dt + tb), na};
+  int* err = (int*)(dt + tb + bb);
+  int* over = err + na;
   uint64_t* totals = (uint64_t*)(dt + tb + bb + fb);
-  int* hflags = (int*)(hh + tb + bb);
-  uint64_t* htot = (uint64_t*)(hh + tb + bb + fb);
-  CPSZ_HIP(hipMemsetAsync(err, 0, na * 4, st));
-  k_dec_spec_multi<<<nblocks, 256, 0, st>>>(dj, dblk0, na, 0, 1, err);
-  CPSZ_HIP(hipGetLastError());
-  ctx.mark((t + ".spec").c_str());
-  int cur = 0;
-  bool settled = false;
-  int rounds = 0;
-  for (int round = 0; round < 4096 && !settled; round++, rounds++) {
-    for (int r = 0; r < kFixPerCheck; r++) {
-      k_dec_spec_multi<<<nblocks, 256, 0, st>>>(dj, dblk0, na, cur, 0, err);
-      cur ^= 1;
-    }
-    CPSZ_HIP(hipMemsetAsync(changed, 0, na * 4, st));
-    k_dec_check_multi<<<nblocks, 256, 0, st>>>(dj, dblk0, na, cur, changed);
-    CPSZ_HIP(hipGetLastError());
-    CPSZ_HIP(hipMemcpyAsync(hflags, changed, 2 * na * 4, hipMemcpyDeviceToHost, st));
-    CPSZ_HIP(hipStreamSynchronize(st));
-    settled = true;
-    for (int a = 0; a < na; a++) {
-      CPSZ_REQUIRE(hflags[na + a] == 0, kErrStream, "invalid huffman code in stream");
-      if (hflags[a]) settled = false;
-    }
-  }
-  // a stream whose segment starts have not settled within the round limit
-  // would decode from inconsistent starts: refuse it
-  CPSZ_REQUIRE(settled, kErrStream, "huffman decode did not converge (bitstream does not resynchronize)");
-  ctx.mark((t + ".fix" + std::to_string(rounds)).c_str());
-  k_dec_bsum_multi<<<nblocks, 256, 0, st>>>(dj, dblk0, na);
-  k_dec_bscan_multi<<<na, 256, 0, st>>>(dj, totals);
-  k_dec_off_multi<<<nblocks, 256, 0, st>>>(dj, dblk0, na);
-  CPSZ_HIP(hipGetLastError());
-  CPSZ_HIP(hipMemcpyAsync(htot, totals, na * 8, hipMemcpyDeviceToHost, st));
-  CPSZ_HIP(hipStreamSynchronize(st));
-  for (int a = 0; a < na; a++)
-    CPSZ_REQUIRE(htot[a] >= h[a].j.n, kErrStream, "huffman bitstream holds fewer symbols than expected");
-  ctx.mark((t + ".scan").c_str());
-  k_dec_write_multi<Sink><<<nblocks, 256, 0, st>>>(djs, dblk0, na, cur);
+  k_dec_cand<<<nblocks, 256, 0, st>>>(tab, err, over);
+  k_dec_serial<<<na, 64, 0, st>>>(tab, err, over);
+  ctx.mark((t + ".cand").c_str());
+  k_dec_follow<<<nblocks, 256, 0, st>>>(tab);
+  k_dec_chain<<<na, 64, 0, st>>>(tab, totals);
+  ctx.mark((t + ".chain").c_str());
+  k_dec_write<Sink><<<nblocks, 256, 0, st>>>(tab);
   CPSZ_HIP(hipGetLastError());
   ctx.mark((t + ".write").c_str());
+  uint8_t* hr = (uint8_t*)ctx.host_buf((t + ".res").c_str(), fb + ob);
+  CPSZ_HIP(hipMemcpyAsync(hr, dt + tb + bb, fb + ob, hipMemcpyDeviceToHost, st));
+  res.err = (const int*)hr;
+  res.totals = (const uint64_t*)(hr + fb);
+  return res;
 }
 
 // Decodes n symbols of one bitstream (see decode_streams).
 template <class Sink>
-void decode_stream(Ctx& ctx, const DeviceDecoder& dd, const uint32_t* d_words, uint64_t nbytes, uint64_t n,
-                   Sink sink, const char* tag, const std::function<void()>& overlap = {}) {
-  DecJob<Sink> j{&dd, d_words, nbytes, n, sink, tag};
-  decode_streams(ctx, &j, 1, overlap);
+DecodeResult decode_stream(Ctx& ctx, const DeviceDecoder& dd, const uint32_t* d_words, uint64_t nbytes, uint64_t n,
+                           Sink sink, const char* tag) {
+  DecJob<Sink> j{&dd, d_words, nbytes, n, sink};
+  return decode_streams(ctx, &j, 1, tag);
 }
 
 }  // namespace cpsz

@@ -46,12 +46,17 @@ struct Tile2d {
     const uint32_t l = (uint32_t)i & 63, t = (uint32_t)j + l;
     return ((size_t)((uint32_t)i >> 6) * nch + t / kTileSteps) * (64 * kTileSteps) + l * kTileSteps + t % kTileSteps;
   }
+  // n / row_len
+  __host__ __device__ uint32_t rows_in(uint32_t n) const {
+    const uint32_t q = (uint32_t)(((uint64_t)mul * n) >> 32);
+    return row_len > 1 ? (((n - q) >> 1) + q) >> shift : n;
+  }
   // element e of the row-major field
   __host__ __device__ size_t at_linear(uint64_t e) const {
     uint32_t i, j;
     if (e < (1ull << 32)) {
-      const uint32_t n = (uint32_t)e, q = (uint32_t)(((uint64_t)mul * n) >> 32);
-      i = row_len > 1 ? (((n - q) >> 1) + q) >> shift : 0;
+      const uint32_t n = (uint32_t)e;
+      i = rows_in(n);
       j = n - i * row_len;
     } else {
       i = (uint32_t)(e / row_len);
