@@ -505,75 +505,155 @@ __global__ void k_zero_i32(int* p, int n) {
 }
 
 // ------------------------------------------------------- huffman sources ----
-// m ids: the u codes then the v codes (offline, m = 2n), or the one code per
-// vertex of offline_log (m = n)
+// The ids: the u codes then the v codes (offline), or the one code per vertex
+// of offline_log.
 struct SrcIds2d {
-  const uint16_t* cu;  // 256-byte aligned
+  const uint16_t* cu;  // 256-byte aligned, and padded to that
   const uint16_t* cv;
-  size_t n, m;
-  static constexpr int kChunk = 512;
-  // four consecutive ids per item: one 8-byte load where the four lie in one
-  // array at an 8-byte boundary, element loads otherwise
-  static constexpr int kMaxItems = kChunk / 4, kPer = 4;
-  __device__ int get(size_t c, int idx, uint32_t* sym) const {
-    const size_t p0 = c * kChunk + 4 * (size_t)idx;
-    uint32_t x[4] = {0, 0, 0, 0};
-    int k = 0;
-    const uint16_t* src = p0 + 4 <= n ? cu + p0 : (p0 >= n && p0 + 4 <= m ? cv + (p0 - n) : nullptr);
-    if (src && ((uintptr_t)src & 7) == 0) {
-      const uint2 w = *reinterpret_cast<const uint2*>(src);
-      x[0] = w.x & 0xFFFFu;
-      x[1] = w.x >> 16;
-      x[2] = w.y & 0xFFFFu;
-      x[3] = w.y >> 16;
-      k = 4;
-    } else {
-      for (; k < 4 && p0 + k < m; k++) x[k] = p0 + k < n ? cu[p0 + k] : cv[p0 + k - n];
-    }
+  size_t n, per;       // chunks of one component
+  // 16 ids a lane, two 16-byte loads: each component starts a chunk of its own,
+  // so that these are aligned whatever its length
+  static constexpr int kRun = 16, kLds = 8, kChunk = 64 * kRun;
+  SrcIds2d(const uint16_t* u, const uint16_t* v, size_t n_) : cu(u), cv(v), n(n_), per((n_ + kChunk - 1) / kChunk) {}
+  size_t chunks(bool both) const { return both ? 2 * per : per; }
+  __device__ void stage(size_t, uint16_t*) const {}
+  __device__ int load(size_t c, const uint16_t*, uint32_t* sym) const {
+    const bool v = c >= per;
+    const size_t p = (v ? c - per : c) * kChunk + kRun * (threadIdx.x & 63);
+    const auto s = glob(reinterpret_cast<const u32x4*>((v ? cv : cu) + min(p, (n - 1) & ~(size_t)(kRun - 1))));
+    const u32x4 a = s[0], b = s[1];
+    const uint32_t w[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
 #pragma unroll
-    for (int q = 0; q < 4; q++) sym[q] = x[q] ? x[q] - 1 : 0;
-    return k;
+    for (int k = 0; k < kRun; k++) {
+      const uint32_t x = k & 1 ? w[k / 2] >> 16 : w[k / 2] & 0xFFFFu;
+      sym[k] = x ? min(x, (uint32_t)kMaxEbCode) - 1 : 0;  // (the padding may hold anything)
+    }
+    return (int)max((long long)0, min((long long)kRun, (long long)n - (long long)p));
   }
 };
 
-struct SrcCodes2d {
+// The codes of 8 consecutive 12x12 blocks of a block row. Their 12 row pieces
+// lie in the tiles as runs of 16 codes: the wave copies them to LDS by 16-byte
+// loads (3 a lane) and reads 18 codes a lane from there, in the blocks' order.
+// Row ii of the chunk lands one code later than row ii - 1 (the tiles are
+// skewed by a step a row), so row ii, column j is at first + ii (kPitch + 1) + j.
+template <typename T>
+struct SrcCodes2dT {
   const uint16_t* q;  // tiles
   Tile2d t;
-  int r1, r2, nby;
-  // optional (batched compress): the values the codec ran on, the global
-  // exclusive scan of the blocks' zero counts at this component's first
-  // block, and where the encoder gathers the unpredictable values
-  const float* x = nullptr;
+  int r1, r2, nby, per;  // per: chunks of a block row
+  // optional: the values the codec ran on, the exclusive scan of the chunks'
+  // zero counts at this component's first chunk, and where the encoder
+  // gathers the unpredictable values
+  const T* x = nullptr;
   const uint64_t* uoff = nullptr;
-  float* unp = nullptr;
+  T* unp = nullptr;
   static constexpr bool kUnpred = true;
-  static constexpr int kMaxItems = kBlock2d * kBlock2d, kPer = 1;
-  // block row and column (32-bit division when the block index allows it)
-  __device__ void block(size_t b, int& bi, int& bj) const {
-    if (b < (1ull << 32)) {
-      bi = (int)((uint32_t)b / (uint32_t)nby);
-      bj = (int)((uint32_t)b - (uint32_t)bi * (uint32_t)nby);
+  static constexpr int kBlocks = 8, kRun = 18, kPitch = 128, kSegs = 15, kLds = kBlock2d * kPitch;
+  static_assert(kBlocks * kBlock2d * kBlock2d == 64 * kRun && kSegs * 8 >= 7 + kBlock2d - 1 + kBlocks * kBlock2d);
+  // a one-column field is laid out, and has its codes in the order of, a one-row field
+  SrcCodes2dT(const uint16_t* q_, const Tile2d& t_, size_t r1_, size_t r2_, const T* x_ = nullptr)
+      : q(q_), t(t_), r1((int)(t_.column ? 1 : r1_)), r2((int)(t_.column ? r1_ : r2_)),
+        nby((int)div_up((size_t)r2, (size_t)kBlock2d)), per((int)div_up((size_t)nby, (size_t)kBlocks)), x(x_) {}
+  size_t chunks() const { return div_up((size_t)r1, (size_t)kBlock2d) * per; }
+  // first block of chunk c
+  __device__ void first(size_t c, int& bi, int& bj) const {
+    if (c < (1ull << 32)) {
+      bi = (int)((uint32_t)c / (uint32_t)per);
+      bj = (int)((uint32_t)c - (uint32_t)bi * (uint32_t)per) * kBlocks;
     } else {
-      bi = (int)(b / nby);
-      bj = (int)(b - (size_t)bi * nby);
+      bi = (int)(c / per);
+      bj = (int)(c - (size_t)bi * per) * kBlocks;
     }
   }
-  __device__ size_t elem(size_t b, int idx) const {
+  __device__ void stage(size_t c, uint16_t* lds) const {
     int bi, bj;
-    block(b, bi, bj);
-    const int sy = min(kBlock2d, r2 - bj * kBlock2d);
-    const int ii = (int)((uint32_t)idx / (uint32_t)sy), jj = idx - ii * sy;
-    return (size_t)(bi * kBlock2d + ii) * r2 + bj * kBlock2d + jj;
+    first(c, bi, bj);
+    const uint32_t i0 = (uint32_t)bi * kBlock2d, sx = (uint32_t)min(kBlock2d, r1 - (int)i0);
+    const uint32_t t0 = ((uint32_t)bj * kBlock2d + (i0 & 63)) & ~7u;
+    u32x4 v[3];
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+      const uint32_t s = (threadIdx.x & 63) + 64 * k, row = s / kSegs, seg = s % kSegs;
+      const uint32_t i = i0 + row, l = i & 63;
+      // the step within the row's own strip (the next one's steps start over)
+      const int step = (int)(t0 + 8 * seg) - (l < (i0 & 63) ? 64 : 0);
+      const bool in = row < sx && step >= 0 && step < (int)(t.nch * kTileSteps);
+      const uint32_t u = in ? (uint32_t)step : 0u;
+      const size_t at = ((size_t)(in ? i >> 6 : 0u) * t.nch + u / kTileSteps) * (64 * kTileSteps) +
+                        (in ? l : 0u) * kTileSteps + u % kTileSteps;
+      v[k] = *glob(reinterpret_cast<const u32x4*>(q + at));
+    }
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+      const uint32_t s = (threadIdx.x & 63) + 64 * k, row = s / kSegs, seg = s % kSegs;
+      if (row < kBlock2d) *reinterpret_cast<u32x4*>(lds + row * kPitch + 8 * seg) = v[k];
+    }
   }
-  __device__ int get(size_t b, int idx, uint32_t* sym) const {
-    int bi, bj;
-    block(b, bi, bj);
-    const int sx = min(kBlock2d, r1 - bi * kBlock2d), sy = min(kBlock2d, r2 - bj * kBlock2d);
-    const int k = min(idx, sx * sy - 1), ii = (int)((uint32_t)k / (uint32_t)sy), jj = k - ii * sy;
-    sym[0] = q[t.at(bi * kBlock2d + ii, bj * kBlock2d + jj)];
-    return idx < sx * sy;
+  // row and column (from the chunk's first) of the lane's first symbol, its
+  // block's width and the symbols left in the chunk from there
+  __device__ int place(size_t c, int& bi, int& bj, int& sx, int& b, int& ii, int& jj, int& w, int& last_w) const {
+    first(c, bi, bj);
+    sx = min(kBlock2d, r1 - bi * kBlock2d);
+    const int nblk = min(kBlocks, nby - bj);
+    last_w = min(kBlock2d, r2 - (bj + nblk - 1) * kBlock2d);
+    const int m0 = kRun * (int)(threadIdx.x & 63), area = sx * kBlock2d;
+    const int total = (nblk - 1) * area + sx * last_w;
+    b = min((int)((uint32_t)m0 / (uint32_t)area), nblk - 1);
+    w = b == nblk - 1 ? last_w : kBlock2d;
+    const int r = m0 - b * area;
+    ii = (int)((uint32_t)r / (uint32_t)w);
+    jj = r - ii * w;
+    return total - m0;
+  }
+  __device__ int load(size_t c, const uint16_t* lds, uint32_t* sym) const {
+    int bi, bj, sx, b, ii, jj, w, last_w;
+    first(c, bi, bj);
+    const uint32_t rem = ((uint32_t)bj * kBlock2d + ((uint32_t)(bi * kBlock2d) & 63)) & 7u;
+    if (bi * kBlock2d + kBlock2d <= r1 && (bj + kBlocks) * kBlock2d <= r2) {
+      // whole blocks: three half rows a lane, eight lanes a block
+      const uint32_t lane = threadIdx.x & 63, s = lane & 7, odd = s & 1;
+      const uint16_t* p = lds + rem + ((3 * s) >> 1) * (kPitch + 1) + (lane >> 3) * kBlock2d + 6 * odd;
+      const uint16_t* p2 = p + (odd ? kPitch + 1 - 6 : 6);
+#pragma unroll
+      for (int k = 0; k < 6; k++) {
+        sym[k] = p[k];
+        sym[6 + k] = p2[k];
+        sym[12 + k] = p[kPitch + 1 + k];
+      }
+      return kRun;
+    }
+    const int left = place(c, bi, bj, sx, b, ii, jj, w, last_w);
+#pragma unroll
+    for (int k = 0; k < kRun; k++) {
+      const bool in = k < left;
+      sym[k] = lds[in ? (int)rem + ii * (kPitch + 1) + b * kBlock2d + jj : (int)rem];
+      if (++jj == w) {
+        jj = 0;
+        if (++ii == sx) {
+          ii = 0;
+          b++;
+          w = bj + b == nby - 1 ? last_w : kBlock2d;
+        }
+      }
+    }
+    return max(0, min(kRun, left));
+  }
+  __device__ size_t elem(size_t c, int k) const {
+    int bi, bj, sx, b, ii, jj, w, last_w;
+    place(c, bi, bj, sx, b, ii, jj, w, last_w);
+    for (jj += k; jj >= w;) {
+      jj -= w;
+      if (++ii == sx) {
+        ii = 0;
+        b++;
+        w = bj + b == nby - 1 ? last_w : kBlock2d;
+      }
+    }
+    return (size_t)(bi * kBlock2d + ii) * r2 + (bj + b) * kBlock2d + jj;
   }
 };
+using SrcCodes2d = SrcCodes2dT<float>;
 
 struct SinkIds2d {
   static constexpr int kBytes = 2;
@@ -704,25 +784,6 @@ __global__ void __launch_bounds__(256) k_block_zeros(const uint16_t* __restrict_
     z += (uint32_t)__popcll(__ballot(zero));
   }
   if (lane == 0) cnt[b] = z;
-}
-
-template <typename T>
-__global__ void __launch_bounds__(256) k_gather_unpred(const uint16_t* __restrict__ q, Tile2d t,
-                                                       const T* __restrict__ x, int r1, int r2, int nby, size_t nb,
-                                                       const uint64_t* __restrict__ off, T* __restrict__ out) {
-  const size_t b = (size_t)blockIdx.x * kUnpWaves + (threadIdx.x >> 6);
-  const int lane = threadIdx.x & 63;
-  if (b >= nb) return;
-  const BlockView v(b, r1, r2, nby);
-  uint64_t o = off[b];
-  const uint64_t below = (1ull << lane) - 1;
-  for (int k0 = 0; k0 < v.m; k0 += 64) {
-    const int k = k0 + lane;
-    const bool zero = k < v.m && q[v.tile_elem(k, t)] == 0;
-    const uint64_t mask = __ballot(zero);
-    if (zero) out[o + __popcll(mask & below)] = x[v.elem(k, r2)];
-    o += __popcll(mask);
-  }
 }
 
 template <typename T>
@@ -1021,54 +1082,80 @@ struct Layout2d {
   uint64_t at[11];  // hdr, h_eb, eb bits, hu1, unp u, hu2, u bits, hv1, unp v, hv2, v bits
 };
 
-// One thread: sizes, offsets, the word and value arrays of every field (in
-// the preallocated pools: *err set when they would overflow), sizes[k].
-__global__ void k_layout2d(Layout2d* __restrict__ L, int nf, uint32_t* words, uint64_t words_cap, float* unp,
-                           uint64_t unp_cap, uint64_t* __restrict__ sizes, uint64_t* __restrict__ words_used,
-                           int* __restrict__ err) {
-  if (threadIdx.x != 0 || blockIdx.x != 0) return;
+__device__ __forceinline__ uint64_t wave_incl_scan64(uint64_t x) {
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const uint64_t y = __shfl_up((unsigned long long)x, o);
+    if ((int)(threadIdx.x & 63) >= o) x += y;
+  }
+  return x;
+}
+
+// One wave, a lane per field: sizes, offsets, the word and value arrays of
+// every field (in the preallocated pools: *err set when they would overflow),
+// sizes[k]. One thread going through the fields measured 1.3 us a field, the
+// latency of its loads.
+__global__ void __launch_bounds__(64) k_layout2d(Layout2d* __restrict__ L, int nf, uint32_t* words, uint64_t words_cap,
+                                                 float* unp, uint64_t unp_cap, uint64_t* __restrict__ sizes,
+                                                 uint64_t* __restrict__ words_used, int* __restrict__ err) {
+  const int lane = threadIdx.x;
   uint64_t wpos = 0, upos = 0;
-  for (int k = 0; k < nf; k++) {
-    Layout2d& F = L[k];
-    uint64_t tb[3];
-    for (int t = 0; t < 3; t++) {
-      F.bytes[t] = (F.tot[t] + 7) / 8;
-      F.wn[t] = (F.bytes[t] + 3) / 4 + 2;
-      tb[t] = F.tinfo[t][1];
+  for (int k0 = 0; k0 < nf; k0 += 64) {
+    const int k = k0 + lane;
+    const bool in = k < nf;
+    Layout2d& F = L[in ? k : 0];
+    uint64_t wneed = 0, uneed = 0, wn[3], un[2], size = 0;
+    if (in) {
+      uint64_t tb[3], bytes[3];
+      for (int t = 0; t < 3; t++) {
+        bytes[t] = (F.tot[t] + 7) / 8;
+        wn[t] = (bytes[t] + 3) / 4 + 2;
+        F.bytes[t] = bytes[t];
+        F.wn[t] = wn[t];
+        tb[t] = F.tinfo[t][1];
+      }
+      for (int c = 0; c < 2; c++) F.unp_n[c] = un[c] = F.tot[3 + c];
+      const uint64_t ind = (F.nb - 1) / 8 + 1;
+      const uint64_t h_eb = 8 + 4 + tb[0] + 8, h1 = 4 + 1 + 4 + 8 + 8 + 8;
+      const uint64_t hu2 = ind + 8 + 4 + tb[1] + 8, hv2 = ind + 8 + 4 + tb[2] + 8;
+      uint64_t p = F.off;
+      const uint64_t sec[11] = {36, h_eb, bytes[0], h1, 4 * un[0], hu2, bytes[1], h1, 4 * un[1], hv2, bytes[2]};
+      for (int q = 0; q < 11; q++) {
+        F.at[q] = p;
+        p += sec[q];
+      }
+      size = p - F.off;
+      F.size = size;
+      sizes[k] = size;
+      wneed = (wn[0] + wn[1] + wn[2] + 63) & ~63ull;
+      uneed = (un[0] + un[1] + 63) & ~63ull;
     }
-    F.unp_n[0] = F.tot[3];
-    F.unp_n[1] = F.tot[4];
-    const uint64_t ind = (F.nb - 1) / 8 + 1;
-    const uint64_t h_eb = 8 + 4 + tb[0] + 8, h1 = 4 + 1 + 4 + 8 + 8 + 8;
-    const uint64_t hu2 = ind + 8 + 4 + tb[1] + 8, hv2 = ind + 8 + 4 + tb[2] + 8;
-    uint64_t p = F.off;
-    const uint64_t sec[11] = {36, h_eb, F.bytes[0], h1, 4 * F.unp_n[0], hu2, F.bytes[1], h1, 4 * F.unp_n[1], hv2,
-                              F.bytes[2]};
-    for (int q = 0; q < 11; q++) {
-      F.at[q] = p;
-      p += sec[q];
+    const uint64_t wi = wave_incl_scan64(wneed), ui = wave_incl_scan64(uneed);
+    const uint64_t wp = wpos + wi - wneed, up = upos + ui - uneed;
+    const uint64_t bad = __ballot(in && (size > F.cap || wp + wneed > words_cap || up + uneed > unp_cap));
+    const int first_bad = bad ? __ffsll((long long)bad) - 1 : 64;
+    if (in && lane < first_bad) {
+      F.words = words + wp;
+      F.unp = unp + up;
+      F.ej_ids->words = F.words;
+      F.ej_codes[0].words = F.words + wn[0];
+      F.ej_codes[1].words = F.words + wn[0] + wn[1];
+      F.ej_codes[0].src.unp = F.unp;
+      F.ej_codes[1].src.unp = F.unp + un[0];
     }
-    F.size = p - F.off;
-    sizes[k] = F.size;
-    const uint64_t wneed = (F.wn[0] + F.wn[1] + F.wn[2] + 63) & ~63ull;
-    const uint64_t uneed = (F.unp_n[0] + F.unp_n[1] + 63) & ~63ull;
-    if (F.size > F.cap || wpos + wneed > words_cap || upos + uneed > unp_cap) {
+    if (bad) {
       // this and the remaining fields keep null arrays: the passes that
       // follow skip them, and the host reports the error
-      *err = 1;
-      break;
+      if (lane == first_bad) {
+        *err = 1;
+        *words_used = wp;
+      }
+      return;
     }
-    F.words = words + wpos;
-    F.unp = unp + upos;
-    wpos += wneed;
-    upos += uneed;
-    F.ej_ids->words = F.words;
-    F.ej_codes[0].words = F.words + F.wn[0];
-    F.ej_codes[1].words = F.words + F.wn[0] + F.wn[1];
-    F.ej_codes[0].src.unp = F.unp;
-    F.ej_codes[1].src.unp = F.unp + F.unp_n[0];
+    wpos += (uint64_t)__shfl((unsigned long long)wi, 63);
+    upos += (uint64_t)__shfl((unsigned long long)ui, 63);
   }
-  *words_used = wpos;
+  if (lane == 0) *words_used = wpos;
 }
 
 __global__ void k_fill_words(uint32_t* __restrict__ w, const uint64_t* __restrict__ n) {
@@ -1432,7 +1519,9 @@ void c2_wavefront(Ctx& ctx, C2Work* const* w, size_t nf, int grid_cap) {
   wavefront2d_compress(ctx, f, grid_cap);
 }
 
-void c2_entropy(Ctx& ctx, const C2Work& w, DeviceStream& out) {
+namespace {
+template <bool F64>
+void c2_entropy_of(Ctx& ctx, const C2Work& w, DeviceStream& out) {
   hipStream_t st = ctx.stream();
   const size_t r1 = w.r1, r2 = w.r2, n = r1 * r2;
   // the values the codec ran on (unpredictable ones are stored as they are)
@@ -1456,24 +1545,43 @@ void c2_entropy(Ctx& ctx, const C2Work& w, DeviceStream& out) {
   uint32_t* hh = (uint32_t*)ctx.host_buf("c2.hist", hist_n * 4);
   CPSZ_HIP(hipMemcpyAsync(hh, hist, hist_n * 4, hipMemcpyDeviceToHost, st));
   const hipEvent_t hist_done = ctx.record_point();
-  // per-block unpredictable counts and their scans need no tree: they run
-  // while the host builds the trees
-  const int nby = (int)div_up(r2, kBlock2d);
-  const size_t nb = div_up(r1, kBlock2d) * nby;
-  const size_t m_ids = w.log ? n : 2 * n;
-  const size_t nch_ids = div_up(m_ids, SrcIds2d::kChunk);
-  SrcIds2d s_ids{cu, cv, n, m_ids};
-  SrcCodes2d s_u{qu, w.t, (int)r1, (int)r2, nby}, s_v{qv, w.t, (int)r1, (int)r2, nby};
-  uint64_t* bits = ctx.buf<uint64_t>("c2.bits", nch_ids + 2 * nb);
-  uint64_t* offs = ctx.buf<uint64_t>("c2.offs", nch_ids + 2 * nb + 8);
-  uint32_t* zc = ctx.buf<uint32_t>("c2.zc", 2 * nb);
-  uint64_t* zoff = ctx.buf<uint64_t>("c2.zoff", 2 * nb + 4);
+  // the job table needs no tree: it travels while the host builds them
+  const size_t nb = div_up(r1, kBlock2d) * div_up(r2, kBlock2d);
+  using SrcV = std::conditional_t<F64, SrcCodes2dT<double>, SrcCodes2d>;
+  using V = std::conditional_t<F64, double, float>;
+  const V* xs[2];
+  if constexpr (F64) xs[0] = w.dU64, xs[1] = w.dV64;
+  else xs[0] = dU, xs[1] = dV;
+  const SrcIds2d s_ids(cu, cv, n);
+  const SrcV s_q[2] = {SrcV(qu, w.t, r1, r2, xs[0]), SrcV(qv, w.t, r1, r2, xs[1])};
+  const size_t nch_ids = s_ids.chunks(!w.log), ncc = s_q[0].chunks();
+  uint64_t* bits = ctx.buf<uint64_t>("c2.bits", nch_ids + 2 * ncc);
+  uint64_t* offs = ctx.buf<uint64_t>("c2.offs", nch_ids + 2 * ncc + 8);
+  uint32_t* zc = ctx.buf<uint32_t>("c2.zc", 2 * ncc);
+  uint64_t* zoff = ctx.buf<uint64_t>("c2.zoff", 2 * ncc + 4);
   uint64_t* totals = ctx.buf<uint64_t>("c2.totals", 8);
-  k_block_zeros<<<unp_grid(nb), 256, 0, st>>>(qu, w.t, (int)r1, (int)r2, nby, nb, zc);
-  k_block_zeros<<<unp_grid(nb), 256, 0, st>>>(qv, w.t, (int)r1, (int)r2, nby, nb, zc + nb);
-  CPSZ_HIP(hipGetLastError());
-  scan_u32_to_u64(ctx, zc, zoff, nb, totals + 3);
-  scan_u32_to_u64(ctx, zc + nb, zoff + nb, nb, totals + 4);
+  uint64_t* cb_code = ctx.buf<uint64_t>("c2.cbcode", 3 * 65536);
+  uint8_t* cb_len = ctx.buf<uint8_t>("c2.cblen", 3 * 65536);
+  struct Jobs {
+    EncJob<SrcIds2d> ids;
+    EncJob<SrcV> q[2];
+  };
+  Jobs* d_jobs = (Jobs*)ctx.buf<uint8_t>("c2.jobs", sizeof(Jobs));
+  const uint32_t iblk = (uint32_t)encode_blocks(nch_ids), cblk = (uint32_t)encode_blocks(ncc);
+  // words, unp: null before the encode
+  auto send_jobs = [&](uint32_t* const (&words)[3], V* const (&unp)[2]) {
+    Jobs* j = (Jobs*)ctx.host_table("c2.jobs", sizeof(Jobs));
+    j->ids = {s_ids, nch_ids, cb_code, cb_len, offs, bits, words[0], 0, nullptr};
+    for (int c = 0; c < 2; c++) {
+      const size_t at = nch_ids + c * ncc;
+      j->q[c] = {s_q[c], ncc, cb_code + (c + 1) * 65536, cb_len + (c + 1) * 65536, offs + at, bits + at, words[c + 1],
+                 c * cblk, zc + c * ncc};
+      j->q[c].src.uoff = zoff + c * ncc;
+      j->q[c].src.unp = unp[c];
+    }
+    ctx.upload_table("c2.jobs", d_jobs, j, sizeof(Jobs));
+  };
+  send_jobs({nullptr, nullptr, nullptr}, {nullptr, nullptr});
   CPSZ_HIP(hipEventSynchronize(hist_done));
   // the v tree is built on the helper thread beside the eb and u trees, and
   // the id stream's bit counts run on the device meanwhile; the tables are
@@ -1486,15 +1594,13 @@ void c2_entropy(Ctx& ctx, const C2Work& w, DeviceStream& out) {
   std::vector<uint64_t>& fv = fv_keep;
   f.resize(65536);
   fv.resize(65536);
-  uint64_t* cb_code = ctx.buf<uint64_t>("c2.cbcode", 3 * 65536);
-  uint8_t* cb_len = ctx.buf<uint8_t>("c2.cblen", 3 * 65536);
   for (int k = 0; k < 65536; k++) fv[k] = hh[kMaxEbCode + 65536 + k];
   {
     HelperJob v_tree([&] { huff_build(fv.data(), 65536, 2 * kCapacity, t_v); }, !ctx.batch_worker);
     for (int k = 0; k < kMaxEbCode; k++) f[k] = hh[k];
     huff_build(f.data(), kMaxEbCode, 2 * 1024, t_eb);
     upload_codebook(ctx, t_eb, cb_code, cb_len, "c2.eb");
-    k_chunk_bits<<<(int)encode_blocks(nch_ids), kEncThreads, 0, st>>>(s_ids, nch_ids, cb_len, bits);
+    k_run_bits<SrcIds2d><<<iblk, kEncThreads, 0, st>>>(&d_jobs->ids, 1);
     CPSZ_HIP(hipGetLastError());
     scan_u64(ctx, bits, offs, nch_ids, totals + 0);
     for (int k = 0; k < 65536; k++) f[k] = hh[kMaxEbCode + k];
@@ -1505,38 +1611,29 @@ void c2_entropy(Ctx& ctx, const C2Work& w, DeviceStream& out) {
   // ---- codebooks and encode pass A (bits per chunk)
   upload_codebook(ctx, t_u, cb_code + 65536, cb_len + 65536, "c2.u");
   upload_codebook(ctx, t_v, cb_code + 2 * 65536, cb_len + 2 * 65536, "c2.v");
-  k_chunk_bits<<<(int)encode_blocks(nb), kEncThreads, 0, st>>>(s_u, nb, cb_len + 65536, bits + nch_ids);
-  k_chunk_bits<<<(int)encode_blocks(nb), kEncThreads, 0, st>>>(s_v, nb, cb_len + 2 * 65536, bits + nch_ids + nb);
+  k_run_bits<SrcV><<<2 * cblk, kEncThreads, 0, st>>>(d_jobs->q, 2);
   CPSZ_HIP(hipGetLastError());
-  scan_u64(ctx, bits + nch_ids, offs + nch_ids, nb, totals + 1);
-  scan_u64(ctx, bits + nch_ids + nb, offs + nch_ids + nb, nb, totals + 2);
+  // one scan for both components: the second one's first offset is the first one's total
+  scan_u64(ctx, bits + nch_ids, offs + nch_ids, 2 * ncc, totals + 1);
+  scan_u32_to_u64(ctx, zc, zoff, 2 * ncc, totals + 2);
   uint64_t* ht = (uint64_t*)ctx.host_buf("c2.totals", 8 * 8);
-  CPSZ_HIP(hipMemcpyAsync(ht, totals, 5 * 8, hipMemcpyDeviceToHost, st));
+  CPSZ_HIP(hipMemcpyAsync(ht, totals, 3 * 8, hipMemcpyDeviceToHost, st));
+  CPSZ_HIP(hipMemcpyAsync(ht + 3, offs + nch_ids + ncc, 8, hipMemcpyDeviceToHost, st));
+  CPSZ_HIP(hipMemcpyAsync(ht + 4, zoff + ncc, 8, hipMemcpyDeviceToHost, st));
   CPSZ_HIP(hipStreamSynchronize(st));
-  const uint64_t bits_eb = ht[0], bits_u = ht[1], bits_v = ht[2], unp_u = ht[3], unp_v = ht[4];
+  const uint64_t bits_eb = ht[0], bits_u = ht[3], bits_v = ht[1] - ht[3], unp_u = ht[4], unp_v = ht[2] - ht[4];
   ctx.mark("scan");
   // ---- encode pass B into aligned scratch
   const size_t bytes_eb = div_up(bits_eb, 8), bytes_u = div_up(bits_u, 8), bytes_v = div_up(bits_v, 8);
   const size_t w_eb = div_up(bytes_eb, 4) + 2, w_u = div_up(bytes_u, 4) + 2, w_v = div_up(bytes_v, 4) + 2;
   uint32_t* words = ctx.buf<uint32_t>("c2.words", w_eb + w_u + w_v);
   k_fill_u32<<<1024, 256, 0, st>>>(words, w_eb + w_u + w_v, 0);
-  k_encode<<<(int)encode_blocks(nch_ids), kEncThreads, 0, st>>>(s_ids, nch_ids, cb_code, cb_len, offs, bits, words);
-  k_encode<<<(int)encode_blocks(nb), kEncThreads, 0, st>>>(s_u, nb, cb_code + 65536, cb_len + 65536, offs + nch_ids,
-                                                   bits + nch_ids, words + w_eb);
-  k_encode<<<(int)encode_blocks(nb), kEncThreads, 0, st>>>(s_v, nb, cb_code + 2 * 65536, cb_len + 2 * 65536,
-                                                   offs + nch_ids + nb, bits + nch_ids + nb, words + w_eb + w_u);
   // unpredictable values in the field's own type (T = double: 8 bytes each)
-  const size_t vb = w.f64 ? 8 : 4;
-  uint8_t* unp = ctx.buf<uint8_t>("c2.unp", vb * (unp_u + unp_v + 1));
-  if (w.f64) {
-    k_gather_unpred<double><<<unp_grid(nb), 256, 0, st>>>(qu, w.t, w.dU64, (int)r1, (int)r2, nby, nb, zoff, (double*)unp);
-    k_gather_unpred<double><<<unp_grid(nb), 256, 0, st>>>(qv, w.t, w.dV64, (int)r1, (int)r2, nby, nb, zoff + nb,
-                                                          (double*)unp + unp_u);
-  } else {
-    k_gather_unpred<float><<<unp_grid(nb), 256, 0, st>>>(qu, w.t, dU, (int)r1, (int)r2, nby, nb, zoff, (float*)unp);
-    k_gather_unpred<float><<<unp_grid(nb), 256, 0, st>>>(qv, w.t, dV, (int)r1, (int)r2, nby, nb, zoff + nb,
-                                                         (float*)unp + unp_u);
-  }
+  constexpr size_t vb = sizeof(V);
+  V* unp = ctx.buf<V>("c2.unp", unp_u + unp_v + 1);
+  send_jobs({words, words + w_eb, words + w_eb + w_u}, {unp, unp + unp_u});
+  k_run_encode<SrcIds2d><<<iblk, kEncThreads, 0, st>>>(&d_jobs->ids, 1);
+  k_run_encode<SrcV><<<2 * cblk, kEncThreads, 0, st>>>(d_jobs->q, 2);
   CPSZ_HIP(hipGetLastError());
   ctx.mark("encode");
   // ---- stream layout
@@ -1580,7 +1677,7 @@ void c2_entropy(Ctx& ctx, const C2Work& w, DeviceStream& out) {
   host_piece(hu2);
   dev_piece(words + w_eb, bytes_u);
   host_piece(hv1);
-  dev_piece(unp + vb * unp_u, vb * unp_v);
+  dev_piece(unp + unp_u, vb * unp_v);
   host_piece(hv2);
   dev_piece(words + w_eb + w_u, bytes_v);
   CPSZ_REQUIRE(pos == total, kErrInternal, "stream layout mismatch");
@@ -1593,6 +1690,13 @@ void c2_entropy(Ctx& ctx, const C2Work& w, DeviceStream& out) {
   out.data = dout;
   out.size = total;
   CPSZ_HIP(hipStreamSynchronize(st));
+}
+
+}  // namespace
+
+void c2_entropy(Ctx& ctx, const C2Work& w, DeviceStream& out) {
+  if (w.f64) c2_entropy_of<true>(ctx, w, out);
+  else c2_entropy_of<false>(ctx, w, out);
 }
 
 // Batched entropy stage (plain offline, float), on the device from the codes
@@ -1610,7 +1714,7 @@ void c2_entropy_batch(Ctx& ctx, C2Work* const* w, size_t nf, uint8_t* dout, cons
   constexpr size_t HN = kMaxEbCode + 2 * 65536;  // dense codebook entries per field
   constexpr uint32_t kMaxCodeLeaves = 65536, kMaxIdLeaves = kMaxEbCode;
   struct G {
-    size_t n, nb, nby, nch_ids, zb, cb;
+    size_t n, nb, nch_ids, ncc, zb, cb;  // ncc: chunks of one component's codes
   };
   std::vector<G> g(nf);
   size_t Z = 0, CB = 0, words_cap = 0, unp_cap = 0;
@@ -1619,13 +1723,13 @@ void c2_entropy_batch(Ctx& ctx, C2Work* const* w, size_t nf, uint8_t* dout, cons
     CPSZ_REQUIRE(!W.log && !W.f64, kErrInternal, "batched entropy: plain float fields only");
     G& x = g[k];
     x.n = W.r1 * W.r2;
-    x.nby = div_up(W.r2, kBlock2d);
-    x.nb = div_up(W.r1, kBlock2d) * x.nby;
-    x.nch_ids = div_up(2 * x.n, (size_t)SrcIds2d::kChunk);
+    x.nb = div_up(W.r1, kBlock2d) * div_up(W.r2, kBlock2d);
+    x.nch_ids = SrcIds2d(W.cu, W.cv, x.n).chunks(true);
+    x.ncc = SrcCodes2d(W.qu, W.t, W.r1, W.r2).chunks();
     x.zb = Z;
-    Z += 2 * x.nb;
+    Z += 2 * x.ncc;
     x.cb = CB;
-    CB += x.nch_ids + 2 * x.nb;
+    CB += x.nch_ids + 2 * x.ncc;
     words_cap += cap[k] / 4 + 6 + 64;
     unp_cap += 2 * x.n + 64;
   }
@@ -1714,7 +1818,7 @@ void c2_entropy_batch(Ctx& ctx, C2Work* const* w, size_t nf, uint8_t* dout, cons
       T.info = d_info + 4 * tt;
     }
     EncJob<SrcIds2d>& e = ej_i[k];
-    e.src = SrcIds2d{W.cu, W.cv, x.n, 2 * x.n};
+    e.src = SrcIds2d(W.cu, W.cv, x.n);
     e.nchunks = x.nch_ids;
     e.code = cb_code + k * HN;
     e.len = cb_len + k * HN;
@@ -1726,26 +1830,26 @@ void c2_entropy_batch(Ctx& ctx, C2Work* const* w, size_t nf, uint8_t* dout, cons
     iblk += (uint32_t)encode_blocks(x.nch_ids);
     for (int c = 0; c < 2; c++) {
       EncJob<SrcCodes2d>& f = ej_c[2 * k + c];
-      // the blocks' zero counts come with their bit counts; the encoder
+      // the chunks' zero counts come with their bit counts; the encoder
       // gathers the unpredictable values (its array comes from k_layout2d)
-      f.src = SrcCodes2d{c ? W.qv : W.qu, W.t, (int)W.r1, (int)W.r2, (int)x.nby, c ? W.dV : W.dU,
-                         zoff + x.zb + c * x.nb, nullptr};
-      f.zc = zc + x.zb + c * x.nb;
-      f.nchunks = x.nb;
+      f.src = SrcCodes2d(c ? W.qv : W.qu, W.t, W.r1, W.r2, c ? W.dV : W.dU);
+      f.src.uoff = zoff + x.zb + c * x.ncc;
+      f.zc = zc + x.zb + c * x.ncc;
+      f.nchunks = x.ncc;
       f.code = cb_code + k * HN + kMaxEbCode + c * 65536;
       f.len = cb_len + k * HN + kMaxEbCode + c * 65536;
-      f.bits = bits + x.cb + x.nch_ids + c * x.nb;
-      f.off = offs + x.cb + x.nch_ids + c * x.nb;
+      f.bits = bits + x.cb + x.nch_ids + c * x.ncc;
+      f.off = offs + x.cb + x.nch_ids + c * x.ncc;
       f.words = nullptr;
       f.blk0 = cblk;
-      cblk += (uint32_t)encode_blocks(x.nb);
+      cblk += (uint32_t)encode_blocks(x.ncc);
     }
-    const size_t c0 = x.cb, c1 = c0 + x.nch_ids, c2 = c1 + x.nb, c3 = c2 + x.nb;
+    const size_t c0 = x.cb, c1 = c0 + x.nch_ids, c2 = c1 + x.ncc, c3 = c2 + x.ncc;
     sd[5 * k + 0] = ScanDiff{offs + c0, offs + c1};
     sd[5 * k + 1] = ScanDiff{offs + c1, offs + c2};
     sd[5 * k + 2] = ScanDiff{offs + c2, offs + c3};
-    sd[5 * k + 3] = ScanDiff{zoff + x.zb, zoff + x.zb + x.nb};
-    sd[5 * k + 4] = ScanDiff{zoff + x.zb + x.nb, zoff + x.zb + 2 * x.nb};
+    sd[5 * k + 3] = ScanDiff{zoff + x.zb, zoff + x.zb + x.ncc};
+    sd[5 * k + 4] = ScanDiff{zoff + x.zb + x.ncc, zoff + x.zb + 2 * x.ncc};
     Layout2d& l = lj[k];
     l = Layout2d{};
     l.off = off[k];
@@ -1855,10 +1959,10 @@ void c2_entropy_batch(Ctx& ctx, C2Work* const* w, size_t nf, uint8_t* dout, cons
     CPSZ_HIP(hipGetLastError());
   }
   ctx.mark("tree");
-  // ---- chunk bit counts (and the code blocks' zero counts), one scan for
+  // ---- chunk bit counts (and the code chunks' zero counts), one scan for
   // every stream, per-stream totals
-  k_chunk_bits_multi<SrcIds2d><<<iblk, kEncThreads, 0, st>>>(d_ej_i, (int)nf);
-  k_chunk_bits_multi<SrcCodes2d><<<cblk, kEncThreads, 0, st>>>(d_ej_c, (int)(2 * nf));
+  k_run_bits<SrcIds2d><<<iblk, kEncThreads, 0, st>>>(d_ej_i, (int)nf);
+  k_run_bits<SrcCodes2d><<<cblk, kEncThreads, 0, st>>>(d_ej_c, (int)(2 * nf));
   CPSZ_HIP(hipGetLastError());
   scan_u64(ctx, bits, offs, CB, offs + CB);
   scan_u32_to_u64(ctx, zc, zoff, Z, zoff + Z);
@@ -1866,10 +1970,10 @@ void c2_entropy_batch(Ctx& ctx, C2Work* const* w, size_t nf, uint8_t* dout, cons
   CPSZ_HIP(hipGetLastError());
   ctx.mark("scan");
   // ---- layout, encode (with the unpredictable gather), headers, assembly
-  k_layout2d<<<1, 1, 0, st>>>(d_lj, (int)nf, words, words_cap, unp, unp_cap, d_sizes, d_words_used, d_err);
+  k_layout2d<<<1, 64, 0, st>>>(d_lj, (int)nf, words, words_cap, unp, unp_cap, d_sizes, d_words_used, d_err);
   k_fill_words<<<2048, 256, 0, st>>>(words, d_words_used);
-  k_encode_multi<SrcIds2d><<<iblk, kEncThreads, 0, st>>>(d_ej_i, (int)nf);
-  k_encode_multi<SrcCodes2d><<<cblk, kEncThreads, 0, st>>>(d_ej_c, (int)(2 * nf));
+  k_run_encode<SrcIds2d><<<iblk, kEncThreads, 0, st>>>(d_ej_i, (int)nf);
+  k_run_encode<SrcCodes2d><<<cblk, kEncThreads, 0, st>>>(d_ej_c, (int)(2 * nf));
   CPSZ_HIP(hipGetLastError());
   ctx.mark("encode");
   k_write_heads2d<<<(unsigned)nf, 256, 0, st>>>(d_lj, dout);

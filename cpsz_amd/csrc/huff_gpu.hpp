@@ -51,7 +51,7 @@ __global__ void __launch_bounds__(256) k_hist(Src src, size_t nchunks, uint32_t*
 
 // ------------------------------------------------------------------ encode --
 // The encode-side kernels run one wave per chunk (4 chunks per 256-thread
-// block). A source exposes its chunk as items taken by lanes in stream order:
+// block). A source exposes its chunk (of the 3D streams; the 2D ones follow below) as items taken by lanes in stream order:
 //   Src::kMaxItems            items per chunk at most
 //   Src::kPer                 symbols per item at most
 //   int get(c, idx, sym[])    the symbols of item idx, in stream order, and
@@ -80,11 +80,9 @@ struct HasUnpred : std::false_type {};
 template <class S>
 struct HasUnpred<S, std::void_t<decltype(S::kUnpred)>> : std::bool_constant<S::kUnpred> {};
 
-// zc (optional): the chunk's count of symbol 0 (the 2D codes' unpredictable
-// marker) for the caller's offsets of the gathered values
 template <class Src>
 __device__ __forceinline__ void chunk_bits_wave(const Src& src, size_t c, const uint8_t* __restrict__ len,
-                                                uint64_t* __restrict__ bits, uint32_t* __restrict__ zc = nullptr) {
+                                                uint64_t* __restrict__ bits) {
   constexpr int kRounds = (Src::kMaxItems + 63) / 64;
   const int lane = threadIdx.x & 63;
   // every round's symbols are fetched before any is used (overlapped latency)
@@ -101,14 +99,6 @@ __device__ __forceinline__ void chunk_bits_wave(const Src& src, size_t c, const 
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) b += __shfl_xor(b, o);
   if (lane == 0) bits[c] = b;
-  if (zc) {
-    uint32_t z = 0;
-#pragma unroll
-    for (int r = 0; r < kRounds; r++)
-#pragma unroll
-      for (int q = 0; q < Src::kPer; q++) z += (uint32_t)__popcll(__ballot(q < ns[r] && sym[r][q] == 0));
-    if (lane == 0) zc[c] = z;
-  }
 }
 
 template <class Src>
@@ -143,17 +133,8 @@ struct EncJob {
   uint64_t* bits;        // chunk bits, at this stream's first chunk
   uint32_t* words;       // this stream's zero-filled word array
   uint32_t blk0;         // first block (kEncWaves chunks per block)
-  uint32_t* zc;          // optional: per-chunk symbol-0 counts (with the bits)
+  uint32_t* zc;          // optional: per-chunk symbol-0 counts (with the bits), for the offsets of gathered values
 };
-
-template <class Src>
-__global__ void __launch_bounds__(kEncThreads) k_chunk_bits_multi(const EncJob<Src>* __restrict__ jobs, int nj) {
-  const uint32_t b = xcd_block(blockIdx.x, gridDim.x);
-  const EncJob<Src>& J = jobs[job_of(jobs, nj, b)];
-  const size_t c = (size_t)(b - J.blk0) * kEncWaves + (threadIdx.x >> 6);
-  if (c >= J.nchunks) return;
-  chunk_bits_wave(J.src, c, J.len, J.bits, J.zc);
-}
 
 // A source whose symbols include `pads` extra symbols 0 (kPads), which the
 // histogram does not count.
@@ -264,20 +245,6 @@ __device__ __forceinline__ void encode_wave(const Src& src, size_t c, bool live,
     int ns[kRounds];
 #pragma unroll
     for (int r = 0; r < kRounds; r++) ns[r] = src.get(c, r * 64 + lane, sym[r]);
-    if constexpr (HasUnpred<Src>::value) {
-      if (src.unp) {
-        // the chunk's unpredictable values, at its offset among the stream's
-        uint64_t o = src.uoff[c] - src.uoff[0];
-        const uint64_t below = (1ull << lane) - 1;
-#pragma unroll
-        for (int r = 0; r < kRounds; r++) {
-          const bool z = ns[r] && sym[r][0] == 0;
-          const uint64_t m = __ballot(z);
-          if (z) src.unp[o + __popcll(m & below)] = src.x[src.elem(c, r * 64 + lane)];
-          o += __popcll(m);
-        }
-      }
-    }
 #pragma unroll
     for (int r = 0; r < kRounds; r++)
 #pragma unroll
@@ -329,19 +296,154 @@ __global__ void __launch_bounds__(kEncThreads) k_encode(Src src, size_t nchunks,
   encode_wave(src, c, live, live ? off[c] : 0, live ? bits[c] : 0, code, len, words, stage[wv]);
 }
 
+// ---- chunks that give every lane a run of consecutive symbols (the 2D
+// streams). A source exposes
+//   Src::kRun                 symbols per lane at most
+//   Src::kLds                 16-bit words of LDS that a wave's chunk takes
+//   void stage(c, lds)        the wave brings chunk c's symbols into LDS
+//   int load(c, lds, sym)     the lane's symbols, in stream order, and their
+//                             count (the others are valid table indices)
+// and, with kUnpred, elem(c, k): where the value of the lane's k-th symbol is.
+// One scan per chunk places the lanes; a lane packs its codes into words by
+// itself and merges each finished word into the wave's LDS words: an OR per 32
+// bits in place of one or two per code. Bound by instruction issue and the
+// gathers of lengths and codes. 96 fields of 256 to 4096 a side (220 million
+// vertices), against one symbol per lane and a scan per 64 of them: bit counts
+// and scans 2.02 -> 0.60 ms, encode with the unpredictable values 4.35 -> 2.25.
+//
+// (Pointers that come out of a job table are generic to the compiler, and a
+// load through one waits for LDS as well: glob() says that they are global.)
+template <class T>
+__device__ __forceinline__ __attribute__((address_space(1))) T* glob(T* p) {
+  return (__attribute__((address_space(1))) T*)p;
+}
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+
+constexpr uint32_t kRunWords = 580;  // words of a chunk kept in LDS: 16 bits a symbol and more
+
 template <class Src>
-__global__ void __launch_bounds__(kEncThreads) k_encode_multi(const EncJob<Src>* __restrict__ jobs, int nj) {
-  constexpr int kStage = Src::kMaxItems * Src::kPer * 2 + 2;
-  __shared__ uint32_t stage[kEncWaves][kStage];
+__device__ __forceinline__ void run_bits_wave(const Src& src, size_t c, const uint8_t* __restrict__ len,
+                                              uint64_t* __restrict__ bits, uint32_t* __restrict__ zc,
+                                              const uint16_t* lds) {
+  uint32_t sym[Src::kRun];
+  const int ns = src.load(c, lds, sym);
+  uint32_t l[Src::kRun];
+#pragma unroll
+  for (int k = 0; k < Src::kRun; k++) l[k] = glob(len)[sym[k]];
+  uint32_t b = 0;  // bits, and in the upper 12 bits the symbols 0
+#pragma unroll
+  for (int k = 0; k < Src::kRun; k++) b += k < ns ? l[k] + (sym[k] == 0 ? 1u << 20 : 0u) : 0u;
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) b += __shfl_xor(b, o);
+  if ((threadIdx.x & 63) == 0) {
+    bits[c] = b & 0xFFFFFu;
+    if (zc) zc[c] = b >> 20;
+  }
+}
+
+template <class Src>
+__device__ __forceinline__ void run_encode_wave(const Src& src, size_t c, bool live, uint64_t b0, uint64_t nbits,
+                                                const uint64_t* __restrict__ code, const uint8_t* __restrict__ len,
+                                                uint32_t* __restrict__ words, uint32_t* st, uint16_t* lds) {
+  static_assert(64 * Src::kRun * 64 < 1 << 20 && 64 * Src::kRun < 1 << 12, "bits and zeros share a word");
+  const int lane = threadIdx.x & 63;
+  const uint32_t sh = (uint32_t)(b0 & 31), nw = (uint32_t)((sh + nbits + 31) >> 5);
+  const bool direct = nw > kRunWords;
+  if (!direct)
+    for (uint32_t k = lane; k < nw; k += 64) st[k] = 0;
+  if (live) src.stage(c, lds);
+  __syncthreads();
+  uint32_t* const w0 = words + (b0 >> 5);
+  if (live) {
+    uint32_t sym[Src::kRun], l[Src::kRun], hi[Src::kRun];
+    const int ns = src.load(c, lds, sym);
+    const auto code32 = glob((const uint32_t*)code);
+#pragma unroll
+    for (int k = 0; k < Src::kRun; k++) {
+      l[k] = glob(len)[sym[k]];
+      hi[k] = code32[2 * (size_t)sym[k] + 1];
+    }
+    uint32_t b = 0;
+#pragma unroll
+    for (int k = 0; k < Src::kRun; k++) {
+      l[k] = k < ns ? l[k] : 0u;
+      b += l[k];
+      if constexpr (HasUnpred<Src>::value) b += k < ns && sym[k] == 0 ? 1u << 20 : 0u;
+    }
+    const uint32_t before = wave_incl_scan(b) - b;
+    if constexpr (HasUnpred<Src>::value) {
+      if (src.unp) {
+        // the chunk's unpredictable values, at its offset among the stream's
+        uint64_t o = glob(src.uoff)[c] - glob(src.uoff)[0] + (before >> 20);
+        if (b >> 20) {
+#pragma unroll
+          for (int k = 0; k < Src::kRun; k++)
+            if (k < ns && sym[k] == 0) glob(src.unp)[o++] = glob(src.x)[src.elem(c, k)];
+        }
+      }
+    }
+    const uint32_t pos = sh + (before & 0xFFFFFu);
+    uint32_t wi = pos >> 5, fill = pos & 31, acc = 0;
+    auto out = [&](uint32_t x) {
+      if (direct) atomicOr(&w0[wi], bswap32(x));
+      else atomicOr(&st[wi], x);
+    };
+    // n <= 32 bits from the top of x
+    auto push = [&](uint32_t x, uint32_t n) {
+      acc |= x >> fill;
+      const uint32_t f = fill + n;
+      if (f >= 32) {
+        out(acc);
+        wi++;
+        acc = __builtin_amdgcn_alignbit(x, 0u, fill);  // what did not fit
+      }
+      fill = f & 31;
+    };
+#pragma unroll
+    for (int k = 0; k < Src::kRun; k++) {
+      push(l[k] ? hi[k] : 0u, min(l[k], 32u));
+      if (l[k] > 32) push(code32[2 * (size_t)sym[k]], l[k] - 32);
+    }
+    if (fill) out(acc);
+  }
+  __syncthreads();
+  if (live && !direct) {
+    const bool tail_shared = ((b0 + nbits) & 31) != 0;
+    for (uint32_t k = lane; k < nw; k += 64) {
+      const uint32_t word = bswap32(st[k]);
+      if ((k == 0 && sh != 0) || (k == nw - 1 && tail_shared)) atomicOr(&w0[k], word);
+      else glob(w0)[k] = word;
+    }
+  }
+}
+
+template <class Src>
+__global__ void __launch_bounds__(kEncThreads) k_run_bits(const EncJob<Src>* __restrict__ jobs, int nj) {
+  __shared__ __align__(16) uint16_t lds[kEncWaves][Src::kLds];
+  const uint32_t b = xcd_block(blockIdx.x, gridDim.x);
+  const EncJob<Src>& J = jobs[job_of(jobs, nj, b)];
+  const int wv = threadIdx.x >> 6;
+  const size_t c = (size_t)(b - J.blk0) * kEncWaves + wv;
+  const bool live = c < J.nchunks;  // uniform per wave
+  const Src src = J.src;  // (LDS stores may alias what a reference reaches)
+  if (live) src.stage(c, lds[wv]);
+  __syncthreads();
+  if (live) run_bits_wave(src, c, J.len, J.bits, J.zc, lds[wv]);
+}
+
+template <class Src>
+__global__ void __launch_bounds__(kEncThreads) k_run_encode(const EncJob<Src>* __restrict__ jobs, int nj) {
+  __shared__ __align__(16) uint16_t lds[kEncWaves][Src::kLds];
+  __shared__ uint32_t stage[kEncWaves][kRunWords];
   const uint32_t b = xcd_block(blockIdx.x, gridDim.x);
   const EncJob<Src>& J = jobs[job_of(jobs, nj, b)];
   if (!J.words) return;  // a stream without an output array is skipped (whole block)
   const int wv = threadIdx.x >> 6;
   const size_t c = (size_t)(b - J.blk0) * kEncWaves + wv;
   const bool live = c < J.nchunks;
-  const uint64_t base = J.off[0];
-  encode_wave(J.src, c, live, live ? J.off[c] - base : 0, live ? J.bits[c] : 0, J.code, J.len, J.words,
-              stage[wv]);
+  const Src src = J.src;
+  run_encode_wave(src, c, live, live ? J.off[c] - J.off[0] : 0, live ? J.bits[c] : 0, J.code, J.len, J.words,
+                  stage[wv], lds[wv]);
 }
 
 // One Huffman tree built on the device (huff_tree.hip) from a histogram's
