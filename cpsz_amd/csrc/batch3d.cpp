@@ -1,8 +1,7 @@
 // Batched compression / decompression of many 3D fields (timesteps of a
 // simulation, ensemble members), possibly of different sizes.
 //
-// Compress: the eb, sign and log kernels run per field on the caller's
-// stream, then ONE persistent wavefront launch covers every field's (plane
+// Compress: the eb, sign and log kernels take all fields in a launch each, then ONE persistent wavefront launch covers every field's (plane
 // group, row block) items (a 192^3 field alone offers 144 workgroups of work
 // to 256 CUs), then the entropy stages (histograms, host Huffman trees,
 // encode, stream assembly) of different fields run concurrently on the worker
@@ -78,20 +77,7 @@ void compress_3d_batch(Ctx& ctx, const std::vector<Field3d>& fields, double max_
     c3_bind(w[k], scratch + soff[k]);
     wp[k] = &w[k];
   }
-  // inputs written on the caller's stream must be complete before the workers'
-  // streams read them
-  CPSZ_HIP(hipStreamSynchronize(ctx.stream()));
-  // bounds passes on the workers' streams: one field's grid fills only part of
-  // the device, so several fields run at once
-  {
-    std::vector<std::function<void(Ctx&)>> eb_jobs(nf);
-    for (size_t k = 0; k < nf; k++)
-      eb_jobs[k] = [&, k](Ctx& wc) {
-        c3_eb(wc, w[k], max_pwr_eb, ov ? (*ov)[k] : EbOverride());
-        CPSZ_HIP(hipStreamSynchronize(wc.stream()));
-      };
-    pool_run(pool_for(ctx.device()), eb_jobs, cfg.workers);
-  }
+  c3_eb(ctx, wp.data(), nf, max_pwr_eb, ov ? ov->data() : nullptr);
   c3_check(ctx, wp.data(), nf);
   ctx.mark("eb");
   c3_wavefront(ctx, wp.data(), nf, cfg.grid_cap);

@@ -2,7 +2,7 @@
 // sz_compress_cp_preserve_3d_offline_log / sz_decompress_cp_preserve_3d_online_log.
 //
 // Compress (inputs in HBM):
-//   k_eb3d       per-cell 6-tet bounds, marching along i over 16-plane strips
+//   k_eb3d       per-cell 6-tet bounds, marching along i over strips of planes
 //                of a 15x63 vertex tile, folded into per-vertex minima with
 //                LDS atomic-min on float bits, then the id code from the
 //                host-libm threshold table
@@ -40,6 +40,10 @@ namespace cpsz {
 
 namespace {
 
+// global address space: pointers read from memory (the job tables) are
+// generic; accessed through these the loads and stores stay global (not flat)
+// accesses, which LDS waits do not wait for
+#define GLB __attribute__((address_space(1)))
 
 constexpr int kP3 = 8;  // planes (waves) per wavefront workgroup
 constexpr int kC3 = 4;  // steps per wavefront chunk (a multiple of 4)
@@ -82,11 +86,11 @@ __device__ __forceinline__ uint32_t lanes_below(uint64_t m) {
 }
 
 // Per-vertex bounds, marching along i. A block owns an output tile of kMJ
-// rows x kMK columns over kMS consecutive planes and walks the cell layers
+// rows x kMK columns over job.ms consecutive planes and walks the cell layers
 // between them; each layer's 16 x 64 cells (origin rows j0-1 .. j0+14,
 // columns k0-1 .. k0+62) are computed once, so only a one-cell halo in j and k
 // (and one extra layer per plane strip) is recomputed: 1.16 cell evaluations
-// per vertex instead of the 1.43 of a cubic tile. Two vertex planes sit in LDS;
+// per vertex with 16 planes a strip instead of the 1.43 of a cubic tile. Two vertex planes sit in LDS;
 // a thread takes one cell, evaluates its six tetrahedra from registers, folds
 // them into the eight corner minima and applies those to the two planes'
 // partial minima with LDS atomic-min on the float bits (the bounds are floats,
@@ -97,25 +101,87 @@ __device__ __forceinline__ uint32_t lanes_below(uint64_t m) {
 // a vertex whose id is constant over the error envelope of its approximate
 // bound gets that id; the others are appended to `fix` (count in *nfix) and
 // recomputed exactly by k_eb3d_fix. FAST never writes eb_out.
-constexpr int kMJ = 15, kMK = 63, kMS = 16;
+constexpr int kMJ = 15, kMK = 63;
 constexpr int kVJ = kMJ + 2, kVK = kMK + 2;  // vertex halo box of one plane
 constexpr uint32_t kInfBits = 0x7f800000u;
 
+// One field's passes before the wavefront; the fields of a batch share the
+// launches (first block of each field's part in eb0, fx0, sg0, lg0).
+struct Eb3Job {
+  const float *U, *V, *W;
+  int r1, r2, r3;
+  int ms, gx, gy;        // k_eb3d: planes per strip, tiles along k and j
+  Skew3 sk;
+  uint8_t* code;
+  int* flags;            // [0] non-finite input or bound; [1] undecided vertices
+  const uint8_t* gain;
+  const uint8_t* fb;
+  double* eb_out;
+  uint32_t* fix;         // undecided vertices, at most n
+  size_t n, nq;
+  uint64_t* smap;
+  float* L;
+  uint32_t eb0, fx0, fxn, sg0, sgn, lg0;
+  int rows, bx;          // k_log: rows of bx threads per block
+};
+
+__device__ __forceinline__ const Eb3Job& eb3_job(const Eb3Job* __restrict__ jobs, int nj, uint32_t b,
+                                                 uint32_t Eb3Job::* first) {
+  int lo = 0, hi = nj - 1;
+  while (lo < hi) {
+    const int mid = (lo + hi + 1) >> 1;
+    if (jobs[mid].*first <= b) lo = mid;
+    else hi = mid - 1;
+  }
+  return jobs[lo];
+}
+
+__global__ void k_eb3d_flags(const Eb3Job* __restrict__ jobs, int nj) {
+  for (int k = threadIdx.x; k < 4 * nj; k += blockDim.x) jobs[k >> 2].flags[k & 3] = 0;
+}
+
+// Planes per strip. A strip of ms planes evaluates ms + 1 layers, so long
+// strips are the least work; but all kEbSlots resident blocks should have a
+// strip, and the last ones to finish leave the others idle for about a seventh
+// of a strip (measured at 256^3: 3.06 ms in one round of 990 strips of 24
+// planes, 2.9 with 1440 of 16; 8 fields of 97 x 130 x 111: 1.88 ms with 1008
+// of 16).
+constexpr size_t kEbSlots = 256 * 4;  // 4 blocks of 4 waves a CU (the kernel's launch bounds)
+int eb3_strip(const std::vector<std::pair<size_t, size_t>>& tiles) {  // (tiles of a plane, planes) per field
+  int best = 1;
+  size_t best_t = ~(size_t)0;
+  for (int ms = 2; ms <= 32; ms++) {
+    size_t blocks = 0;
+    for (const auto& [t, planes] : tiles) blocks += t * div_up(planes, (size_t)ms);
+    const size_t cost = (size_t)(ms + 1) * (7 * std::max(blocks, kEbSlots) + kEbSlots);
+    if (cost < best_t) {
+      best_t = cost;
+      best = ms;
+    }
+  }
+  return best;
+}
+
 template <bool FAST>
-__global__ void __launch_bounds__(256, 4) k_eb3d(const float* __restrict__ U, const float* __restrict__ V,
-                                              const float* __restrict__ W, int r1, int r2, int r3,
-                                              double max_pwr_eb, const double* __restrict__ q3d, int nq,
-                                              Skew3 sk, uint8_t* __restrict__ code, int* __restrict__ flags,
-                                              const uint8_t* __restrict__ gain, const uint8_t* __restrict__ fb,
-                                              double* __restrict__ eb_out, uint32_t* __restrict__ fix,
-                                              uint32_t* __restrict__ nfix) {
+__global__ void __launch_bounds__(256, 4) k_eb3d(const Eb3Job* __restrict__ jobs, int njobs, double max_pwr_eb,
+                                              const double* __restrict__ q3d, int nq) {
   __shared__ float sv[2][3][kVJ][kVK];
   __shared__ uint32_t seb[2][kMJ][kMK];
   const int tid = threadIdx.x;
-  const int k0 = blockIdx.x * kMK, j0 = blockIdx.y * kMJ, i0 = blockIdx.z * kMS;
-  const int i1 = min(i0 + kMS, r1);
+  const Eb3Job& J = eb3_job(jobs, njobs, blockIdx.x, &Eb3Job::eb0);
+  const int r1 = J.r1, r2 = J.r2, r3 = J.r3;
+  const Skew3 sk = J.sk;
+  const uint8_t* const gain = J.gain;
+  const uint8_t* const fb = J.fb;
+  const auto code = glob(J.code);
+  const auto fix = glob(J.fix);
+  uint32_t* const nfix = (uint32_t*)(J.flags + 1);
+  const uint32_t blk = blockIdx.x - J.eb0, by = blk / J.gx;
+  const int k0 = (int)(blk - by * J.gx) * kMK, j0 = (int)(by % J.gy) * kMJ, i0 = (int)(by / J.gy) * J.ms;
+  const int i1 = min(i0 + J.ms, r1);
   const size_t d0 = (size_t)r2 * r3, d1 = r3;
-  const float* src[3] = {U, V, W};
+  const GLB float* const src[3] = {glob(J.U), glob(J.V), glob(J.W)};
+  double* const eb_out = J.eb_out;
   int bad = 0;
   for (int e = tid; e < 2 * kMJ * kMK; e += 256) (&seb[0][0][0])[e] = kInfBits;
   auto load_plane = [&](int pl) {
@@ -218,25 +284,27 @@ __global__ void __launch_bounds__(256, 4) k_eb3d(const float* __restrict__ U, co
       }
     }
   }
-  if (bad) atomicOr(flags, 1);
+  if (bad) atomicOr(J.flags, 1);
 }
 
 // Exact bounds for the vertices k_eb3d<true> could not decide: the minimum of
 // the exact bounds of the 24 tetrahedra around the vertex (those of the eight
 // cells that hold it). The set of tetrahedra and their bounds equal the
 // marching kernel's, so the minimum does too. Grid-stride over the list.
-__global__ void __launch_bounds__(256) k_eb3d_fix(const float* __restrict__ U, const float* __restrict__ V,
-                                                  const float* __restrict__ W, int r1, int r2, int r3,
-                                                  double max_pwr_eb, const double* __restrict__ q3d, int nq,
-                                                  Skew3 sk, uint8_t* __restrict__ code, int* __restrict__ flags,
-                                                  const uint8_t* __restrict__ gain,
-                                                  const uint8_t* __restrict__ fb,
-                                                  const uint32_t* __restrict__ fix,
-                                                  const uint32_t* __restrict__ nfix) {
-  const uint32_t count = *nfix;
+__global__ void __launch_bounds__(256) k_eb3d_fix(const Eb3Job* __restrict__ jobs, int nj, double max_pwr_eb,
+                                                  const double* __restrict__ q3d, int nq) {
+  const Eb3Job& J = eb3_job(jobs, nj, blockIdx.x, &Eb3Job::fx0);
+  const auto U = glob(J.U), V = glob(J.V), W = glob(J.W);
+  const int r1 = J.r1, r2 = J.r2, r3 = J.r3;
+  const Skew3 sk = J.sk;
+  const uint8_t* const gain = J.gain;
+  const uint8_t* const fb = J.fb;
+  const auto code = glob(J.code);
+  const auto fix = glob(J.fix);
+  const uint32_t count = (uint32_t)J.flags[1];
   const size_t d0 = (size_t)r2 * r3, d1 = r3;
   int bad = 0;
-  for (uint32_t e = blockIdx.x * blockDim.x + threadIdx.x; e < count; e += gridDim.x * blockDim.x) {
+  for (uint32_t e = (blockIdx.x - J.fx0) * blockDim.x + threadIdx.x; e < count; e += J.fxn * blockDim.x) {
     const uint32_t v = fix[e];
     const int i = (int)(v / d0), rem = (int)(v - (size_t)i * d0), j = rem / r3, k = rem - j * r3;
     // the 3 x 3 x 3 vertex neighbourhood once (clamped at the borders, where
@@ -289,7 +357,7 @@ __global__ void __launch_bounds__(256) k_eb3d_fix(const float* __restrict__ U, c
     if (gain && !(fb && fb[v]) && gain[v]) eb = fmin(max_pwr_eb, ldexp(eb, (int)gain[v]));
     code[sk.at(i, j, k)] = (uint8_t)eb_code_3d(eb, q3d, nq);
   }
-  if (bad) atomicOr(flags, 1);
+  if (bad) atomicOr(J.flags, 1);
 }
 
 // Self-check of the premises of the approximate bounds (cube_sign_bound_fast):
@@ -345,12 +413,13 @@ __global__ void __launch_bounds__(256) k_check_csb(uint32_t iters, uint32_t seed
 // value 8k+j at bit 7-j of byte k. Block y = component; each wave takes 16
 // consecutive groups, loading all of them before its ballots.
 constexpr int kSignGroups = 16;
-__global__ void __launch_bounds__(256) k_signmap(const float* __restrict__ U, const float* __restrict__ V,
-                                                 const float* __restrict__ W, size_t n, size_t nq,
-                                                 uint64_t* __restrict__ out) {
+__global__ void __launch_bounds__(256) k_signmap(const Eb3Job* __restrict__ jobs, int nj) {
+  const Eb3Job& J = eb3_job(jobs, nj, blockIdx.x, &Eb3Job::sg0);
+  const size_t n = J.n, nq = J.nq;
+  const auto out = glob(J.smap);
   const int p = blockIdx.y, lane = threadIdx.x & 63;
-  const float* X = p == 0 ? U : (p == 1 ? V : W);
-  const size_t q0 = ((size_t)blockIdx.x * 4 + (threadIdx.x >> 6)) * kSignGroups;
+  const auto X = glob(p == 0 ? J.U : (p == 1 ? J.V : J.W));
+  const size_t q0 = ((size_t)(blockIdx.x - J.sg0) * 4 + (threadIdx.x >> 6)) * kSignGroups;
   float v[kSignGroups];
 #pragma unroll
   for (int r = 0; r < kSignGroups; r++) {
@@ -365,19 +434,29 @@ __global__ void __launch_bounds__(256) k_signmap(const float* __restrict__ U, co
 }
 
 // log_transform (include/sz_cp_preserve_utils.hpp:205-221): log2f(|x|), -100
-// for 0, written in wave layout. Block x = one (i, j) row, y = k range.
-__global__ void k_log(const float* __restrict__ U, const float* __restrict__ V,
-                      const float* __restrict__ W, Skew3 s, LibmView lv, float* __restrict__ L) {
-  const uint32_t l = xcd_block(blockIdx.x + blockIdx.y * gridDim.x, gridDim.x * gridDim.y);
-  const uint32_t row = l % gridDim.x;
-  const int k = (int)(l / gridDim.x) * blockDim.x + threadIdx.x;
-  if (k >= s.r3) return;
+// for 0, written in wave layout. A block takes `rows` (i, j) rows of bx
+// threads (short rows share a block). A row lands as 16 bytes in each of many
+// KiB, which the rows beside it fill up: blocks in flight are on neighbouring
+// rows of an XCD's share, so that its L2 puts them together (four rows one
+// after the other per block: 0.67 against 0.50 ms at 256^3; turning the values
+// in LDS: 0.69, the logarithm's table look-ups overlapping less).
+__global__ void __launch_bounds__(256) k_log(const Eb3Job* __restrict__ jobs, int nj, LibmView lv) {
+  const uint32_t l = xcd_block(blockIdx.x, gridDim.x);
+  const Eb3Job& J = eb3_job(jobs, nj, l, &Eb3Job::lg0);
+  const Skew3 s = J.sk;
+  const auto U = glob(J.U), V = glob(J.V), W = glob(J.W);
+  const auto L = glob(J.L);
+  const uint32_t bx = (uint32_t)J.bx, tid = threadIdx.x;
+  const uint32_t sub = (tid >= bx) + (tid >= 2 * bx) + (tid >= 3 * bx), row = (l - J.lg0) * (uint32_t)J.rows + sub;
+  if (sub >= (uint32_t)J.rows || row >= (uint32_t)s.r1 * (uint32_t)s.r2) return;
   const int i = (int)(row / (uint32_t)s.r2), j = (int)(row - (uint32_t)i * s.r2);
-  const size_t v = (size_t)row * s.r3 + k, o = s.at(i, j, k);
-  const float x0 = U[v], x1 = V[v], x2 = W[v];
-  L[o] = x0 != 0 ? host_log2f(lv, fabsf(x0)) : -100.f;
-  L[s.per + o] = x1 != 0 ? host_log2f(lv, fabsf(x1)) : -100.f;
-  L[2 * s.per + o] = x2 != 0 ? host_log2f(lv, fabsf(x2)) : -100.f;
+  for (int k = (int)(tid - sub * bx); k < s.r3; k += (int)bx) {
+    const size_t v = (size_t)row * s.r3 + k, o = s.at(i, j, k);
+    const float x0 = U[v], x1 = V[v], x2 = W[v];
+    L[o] = x0 != 0 ? host_log2f(lv, fabsf(x0)) : -100.f;
+    L[s.per + o] = x1 != 0 ? host_log2f(lv, fabsf(x1)) : -100.f;
+    L[2 * s.per + o] = x2 != 0 ? host_log2f(lv, fabsf(x2)) : -100.f;
+  }
 }
 
 // ------------------------------------------------------------- wavefront --
@@ -421,10 +500,6 @@ __device__ __forceinline__ float comp4(const float4& v, int s) {
   return s == 0 ? v.x : (s == 1 ? v.y : (s == 2 ? v.z : v.w));
 }
 
-// global address space: pointers read from memory (the batch table) are
-// generic; accessed through these the loads and stores stay global (not flat)
-// accesses, which LDS waits do not wait for
-#define GLB __attribute__((address_space(1)))
 // constant address space: the batch table is not written while the kernel
 // runs, so uniform reads of it become scalar loads
 #define CST __attribute__((address_space(4)))
@@ -959,41 +1034,93 @@ void c3_bind(C3Work& w, uint8_t* p) {
   w.flags = carve<int>(p, 4);
 }
 
-void c3_eb(Ctx& ctx, C3Work& w, double max_pwr_eb, const EbOverride& ov) {
-  CPSZ_REQUIRE(w.dU && w.dV && w.dW, kErrArg, "compress_3d: bad arguments");
-  check_dims_3d(w.r1, w.r2, w.r3, "compress_3d");
-  hipStream_t st = ctx.stream();
-  const size_t r1 = w.r1, r2 = w.r2, r3 = w.r3, n = r1 * r2 * r3;
-  const Skew3 sk = make_skew(r1, r2, r3);
-  const Ctx::LibmDev& lm = ctx.libm_dev();
-  CPSZ_HIP(hipMemsetAsync(w.flags, 0, 16, st));
-  {
-    dim3 grid((unsigned)div_up(r3, kMK), (unsigned)div_up(r2, kMJ), (unsigned)div_up(r1, kMS));
-    if (ov.eb_out) {
-      k_eb3d<false><<<grid, 256, 0, st>>>(w.dU, w.dV, w.dW, (int)r1, (int)r2, (int)r3, max_pwr_eb, ctx.d_q3d(),
-                                          ctx.q3d_size(), sk, w.ebc, w.flags, ov.gain, ov.fallback, ov.eb_out,
-                                          nullptr, nullptr);
-    } else {
-      // the undecided-vertex list (at most n entries) lives in R, which the
-      // wavefront fills only later
-      uint32_t* fix = (uint32_t*)w.R;
-      uint32_t* nfix = (uint32_t*)(w.flags + 1);
-      k_eb3d<true><<<grid, 256, 0, st>>>(w.dU, w.dV, w.dW, (int)r1, (int)r2, (int)r3, max_pwr_eb, ctx.d_q3d(),
-                                         ctx.q3d_size(), sk, w.ebc, w.flags, ov.gain, ov.fallback, nullptr, fix,
-                                         nfix);
-      k_eb3d_fix<<<1024, 256, 0, st>>>(w.dU, w.dV, w.dW, (int)r1, (int)r2, (int)r3, max_pwr_eb, ctx.d_q3d(),
-                                       ctx.q3d_size(), sk, w.ebc, w.flags, ov.gain, ov.fallback, fix, nfix);
+namespace {
+// The job table of nf fields' passes, on the device; returns the grids.
+struct Eb3Grids {
+  uint32_t eb = 0, fx = 0, sg = 0, lg = 0;
+};
+Eb3Grids send_eb3_jobs(Ctx& ctx, Eb3Job* jobs, int nf, Eb3Job*& d_jobs) {
+  std::vector<std::pair<size_t, size_t>> tiles;
+  for (int k = 0; k < nf; k++)
+    tiles.push_back({div_up((size_t)jobs[k].r3, (size_t)kMK) * div_up((size_t)jobs[k].r2, (size_t)kMJ), (size_t)jobs[k].r1});
+  const int ms = eb3_strip(tiles);
+  Eb3Grids g;
+  for (int k = 0; k < nf; k++) {
+    Eb3Job& J = jobs[k];
+    J.sk = make_skew(J.r1, J.r2, J.r3);
+    J.n = (size_t)J.r1 * J.r2 * J.r3;
+    J.nq = div_up(J.n, 64);
+    J.ms = ms;
+    J.gx = (int)div_up(J.r3, kMK);
+    J.gy = (int)div_up(J.r2, kMJ);
+    J.bx = std::min(256, (int)div_up(J.r3, 64) * 64);
+    J.rows = 256 / J.bx;
+    J.fxn = (uint32_t)std::min<size_t>(div_up(J.n, 16384), 1024);
+    J.sgn = (uint32_t)div_up(J.nq, 4 * kSignGroups);
+    const size_t eb = tiles[k].first * div_up(J.r1, ms), lg = div_up((size_t)J.r1 * J.r2, (size_t)J.rows);
+    CPSZ_REQUIRE(g.eb + eb < (1ull << 31) && g.lg + lg < (1ull << 31) && (size_t)g.sg + J.sgn < (1ull << 31),
+                 kErrUnsupported, "compress_3d: batch too large for one launch");
+    J.eb0 = g.eb;
+    J.fx0 = g.fx;
+    J.sg0 = g.sg;
+    J.lg0 = g.lg;
+    g.eb += (uint32_t)eb;
+    g.fx += J.fxn;
+    g.sg += J.sgn;
+    g.lg += (uint32_t)lg;
+  }
+  const size_t bytes = nf * sizeof(Eb3Job);
+  d_jobs = (Eb3Job*)ctx.buf<uint8_t>("e3.jobs", bytes);
+  void* h = ctx.host_table("e3.jobs", bytes);
+  std::memcpy(h, jobs, bytes);
+  ctx.upload_table("e3.jobs", d_jobs, h, bytes);
+  k_eb3d_flags<<<1, 256, 0, ctx.stream()>>>(d_jobs, nf);
+  CPSZ_HIP(hipGetLastError());
+  return g;
+}
+}  // namespace
+
+void c3_eb(Ctx& ctx, C3Work* const* w, size_t nf, double max_pwr_eb, const EbOverride* ov) {
+  std::vector<Eb3Job> jobs(nf);
+  for (size_t k = 0; k < nf; k++) {
+    const C3Work& x = *w[k];
+    CPSZ_REQUIRE(x.dU && x.dV && x.dW, kErrArg, "compress_3d: bad arguments");
+    check_dims_3d(x.r1, x.r2, x.r3, "compress_3d");
+    Eb3Job& J = jobs[k];
+    J = Eb3Job{};
+    J.U = x.dU;
+    J.V = x.dV;
+    J.W = x.dW;
+    J.r1 = (int)x.r1;
+    J.r2 = (int)x.r2;
+    J.r3 = (int)x.r3;
+    J.code = x.ebc;
+    J.flags = x.flags;
+    J.smap = x.smap;
+    J.L = x.L;
+    // the undecided-vertex list (at most n entries) lives in R, which the
+    // wavefront fills only later
+    J.fix = (uint32_t*)x.R;
+    if (ov) {
+      J.gain = ov[k].gain;
+      J.fb = ov[k].fallback;
+      J.eb_out = ov[k].eb_out;
+      CPSZ_REQUIRE(!J.eb_out == !ov[0].eb_out, kErrInternal, "compress_3d: bounds of some fields of a batch");
     }
-    CPSZ_HIP(hipGetLastError());
   }
+  hipStream_t st = ctx.stream();
+  Eb3Job* d;
+  const Eb3Grids g = send_eb3_jobs(ctx, jobs.data(), (int)nf, d);
+  if (jobs[0].eb_out) {
+    k_eb3d<false><<<g.eb, 256, 0, st>>>(d, (int)nf, max_pwr_eb, ctx.d_q3d(), ctx.q3d_size());
+  } else {
+    k_eb3d<true><<<g.eb, 256, 0, st>>>(d, (int)nf, max_pwr_eb, ctx.d_q3d(), ctx.q3d_size());
+    k_eb3d_fix<<<g.fx, 256, 0, st>>>(d, (int)nf, max_pwr_eb, ctx.d_q3d(), ctx.q3d_size());
+  }
+  CPSZ_HIP(hipGetLastError());
   ctx.mark("eb");
-  const size_t nq = div_up(n, 64);
-  k_signmap<<<dim3((unsigned)div_up(nq, 4 * kSignGroups), 3), 256, 0, st>>>(w.dU, w.dV, w.dW, n, nq, w.smap);
-  {
-    const int bx = r3 >= 256 ? 256 : (int)div_up(r3, 64) * 64;
-    dim3 grid((unsigned)(r1 * r2), (unsigned)div_up(r3, bx));
-    k_log<<<grid, bx, 0, st>>>(w.dU, w.dV, w.dW, sk, lm.log2f, w.L);
-  }
+  k_signmap<<<dim3(g.sg, 3), 256, 0, st>>>(d, (int)nf);
+  k_log<<<g.lg, 256, 0, st>>>(d, (int)nf, ctx.libm_dev().log2f);
   CPSZ_HIP(hipGetLastError());
   ctx.mark("log");
 }
@@ -1168,8 +1295,8 @@ void compress_3d_device(Ctx& ctx, const float* dU, const float* dV, const float*
   w.r2 = r2;
   w.r3 = r3;
   c3_bind(w, ctx.buf<uint8_t>("c3.scratch", c3_scratch_bytes(r1, r2, r3)));
-  c3_eb(ctx, w, max_pwr_eb, ov);
   C3Work* wp = &w;
+  c3_eb(ctx, &wp, 1, max_pwr_eb, &ov);
   c3_check(ctx, &wp, 1);
   c3_wavefront(ctx, &wp, 1, 1024);
   ctx.mark("lorenzo");
@@ -1182,13 +1309,20 @@ void eb_3d_device(Ctx& ctx, const float* dU, const float* dV, const float* dW, s
   CPSZ_REQUIRE(dU && dV && dW && dE, kErrArg, "eb_3d: bad arguments");
   check_dims_3d(r1, r2, r3, "eb_3d");
   hipStream_t st = ctx.stream();
-  const Skew3 sk = make_skew(r1, r2, r3);
-  uint8_t* code = ctx.buf<uint8_t>("e3.code", sk.per);
   int* flags = ctx.buf<int>("e3.flags", 4);
-  CPSZ_HIP(hipMemsetAsync(flags, 0, 16, st));
-  dim3 grid((unsigned)div_up(r3, kMK), (unsigned)div_up(r2, kMJ), (unsigned)div_up(r1, kMS));
-  k_eb3d<false><<<grid, 256, 0, st>>>(dU, dV, dW, (int)r1, (int)r2, (int)r3, max_pwr_eb, ctx.d_q3d(),
-                                      ctx.q3d_size(), sk, code, flags, nullptr, nullptr, dE, nullptr, nullptr);
+  Eb3Job J{};
+  J.U = dU;
+  J.V = dV;
+  J.W = dW;
+  J.r1 = (int)r1;
+  J.r2 = (int)r2;
+  J.r3 = (int)r3;
+  J.code = ctx.buf<uint8_t>("e3.code", make_skew(r1, r2, r3).per);
+  J.flags = flags;
+  J.eb_out = dE;
+  Eb3Job* d;
+  const Eb3Grids g = send_eb3_jobs(ctx, &J, 1, d);
+  k_eb3d<false><<<g.eb, 256, 0, st>>>(d, 1, max_pwr_eb, ctx.d_q3d(), ctx.q3d_size());
   CPSZ_HIP(hipGetLastError());
   int* h = (int*)ctx.host_buf("e3.hflags", 16);
   CPSZ_HIP(hipMemcpyAsync(h, flags, 16, hipMemcpyDeviceToHost, st));

@@ -39,7 +39,8 @@ struct C3Work {
 };
 size_t c3_scratch_bytes(size_t r1, size_t r2, size_t r3);
 void c3_bind(C3Work& w, uint8_t* scratch);  // carves c3_scratch_bytes of device memory
-void c3_eb(Ctx& ctx, C3Work& w, double max_pwr_eb, const EbOverride& ov);
+// nf fields in one launch per pass (ov: null or one override per field)
+void c3_eb(Ctx& ctx, C3Work* const* w, size_t nf, double max_pwr_eb, const EbOverride* ov);
 void c3_check(Ctx& ctx, C3Work* const* w, size_t nf);  // synchronizes
 void c3_wavefront(Ctx& ctx, C3Work* const* w, size_t nf, int grid_cap);
 void c3_entropy(Ctx& ctx, const C3Work& w, DeviceStream& out);  // synchronizes
