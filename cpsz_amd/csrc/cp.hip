@@ -19,6 +19,7 @@
 // root plus a complex pair, Descartes' rule of signs for three real roots.
 #include <algorithm>
 #include <cmath>
+#include <cstring>
 #include <mutex>
 #include <numeric>
 #include <vector>
@@ -218,6 +219,118 @@ void critical_points_3d(Ctx& ctx, const float* dU, const float* dV, const float*
     CPSZ_HIP(hipGetLastError());
   }
   collect(ctx, o, dc, ids, types, cap, count);
+}
+
+// ---- many 2D fields, both tests, in one launch. Field by field and test by
+// test, each list cost two waits and fresh host arrays of 65536 entries: 5 of
+// the 13.7 ms of a learned compression of 12 fields.
+namespace {
+struct CpJob2d {
+  const float *U, *V;
+  int r1, r2;
+  uint32_t blk0;  // first block
+};
+
+// key: list (2 field + sos) << 44 | id << 4 | type
+__global__ void __launch_bounds__(256) k_cp2d_multi(const CpJob2d* __restrict__ jobs, int nj,
+                                                    unsigned long long* __restrict__ count,
+                                                    unsigned long long* __restrict__ keys, unsigned long long cap) {
+  int lo = 0, hi = nj - 1;
+  while (lo < hi) {
+    const int mid = (lo + hi + 1) >> 1;
+    if (jobs[mid].blk0 <= blockIdx.x) lo = mid;
+    else hi = mid - 1;
+  }
+  const CpJob2d& J = jobs[lo];
+  const float* const U = J.U;
+  const float* const V = J.V;
+  const int r1 = J.r1, r2 = J.r2;
+  const long long cell = (blockIdx.x - J.blk0) * (long long)blockDim.x + threadIdx.x;
+  const long long nci = r1 - 3, ncj = r2 - 3;  // i in [1, r1-3], j in [1, r2-3]
+  if (cell >= nci * ncj) return;
+  const int i = 1 + (int)(cell / ncj), j = 1 + (int)(cell % ncj);
+  const size_t v = (size_t)i * r2 + j;
+  const size_t idx[4] = {v, v + r2, v + 1, v + r2 + 1};
+  float x[4][2];
+  for (int p = 0; p < 4; p++) {
+    x[p][0] = U[idx[p]];
+    x[p][1] = V[idx[p]];
+  }
+  const unsigned long long sid = 2ull * ((unsigned long long)i * (r2 - 1) + j);
+  for (int t = 0; t < 2; t++) {
+    const int c[3] = {0, t == 0 ? 1 : 2, 3};
+    float f[3][2];
+    long long gi[3];
+    for (int p = 0; p < 3; p++) {
+      f[p][0] = x[c[p]][0];
+      f[p][1] = x[c[p]][1];
+      gi[p] = (long long)idx[c[p]];
+    }
+    const int type[2] = {tri_cp(f, t), tri_cp_sos(f, gi, t)};
+    for (int m = 0; m < 2; m++)
+      if (type[m] >= 0) {
+        const unsigned long long k = atomicAdd(count, 1ull);
+        if (k < cap) keys[k] = (unsigned long long)(2 * lo + m) << 44 | (sid + t) << 4 | (unsigned long long)type[m];
+      }
+  }
+}
+}  // namespace
+
+void critical_points_2d_batch(Ctx& ctx, const std::vector<CpField2d>& fields, std::vector<CpLists2d>& out) {
+  hipStream_t st = ctx.stream();
+  const size_t nf = fields.size();
+  out.assign(nf, CpLists2d());
+  std::vector<CpJob2d> jobs;
+  std::vector<size_t> of;  // job's field
+  uint64_t blocks = 0;
+  for (size_t k = 0; k < nf; k++) {
+    const CpField2d& F = fields[k];
+    CPSZ_REQUIRE(F.dU && F.dV && F.r1 * F.r2 < (1ull << 32), kErrArg, "critical_points_2d_batch: bad arguments");
+    if (F.r1 <= 3 || F.r2 <= 3) continue;
+    jobs.push_back(CpJob2d{F.dU, F.dV, (int)F.r1, (int)F.r2, (uint32_t)blocks});
+    of.push_back(k);
+    blocks += div_up((F.r1 - 3) * (F.r2 - 3), 256);
+    CPSZ_REQUIRE(blocks < (1ull << 31) && jobs.size() < (1u << 19), kErrUnsupported,
+                 "critical_points_2d_batch: batch too large");
+  }
+  if (jobs.empty()) return;
+  const size_t tb = jobs.size() * sizeof(CpJob2d);
+  CpJob2d* d = (CpJob2d*)ctx.buf<uint8_t>("cpb.jobs", tb);
+  void* h = ctx.host_table("cpb.jobs", tb);
+  std::memcpy(h, jobs.data(), tb);
+  ctx.upload_table("cpb.jobs", d, h, tb);
+  unsigned long long* dc = ctx.buf<unsigned long long>("cpb.count", 1);
+  unsigned long long* hc = (unsigned long long*)ctx.host_buf("cpb.count", 8);
+  unsigned long long* keys;
+  size_t n = 0;
+  for (size_t cap = 1u << 16;; cap = n) {  // a second launch only if there are more than that
+    keys = ctx.buf<unsigned long long>("cpb.keys", cap);
+    k_zero_count<<<1, 1, 0, st>>>(dc);
+    k_cp2d_multi<<<(unsigned)blocks, 256, 0, st>>>(d, (int)jobs.size(), dc, keys, cap);
+    CPSZ_HIP(hipGetLastError());
+    CPSZ_HIP(hipMemcpyAsync(hc, dc, 8, hipMemcpyDeviceToHost, st));
+    CPSZ_HIP(hipStreamSynchronize(st));
+    n = (size_t)*hc;
+    if (n <= cap) break;
+  }
+  if (!n) return;
+  uint64_t* hk = (uint64_t*)ctx.host_buf("cpb.keys", 8 * n);
+  CPSZ_HIP(hipMemcpyAsync(hk, keys, 8 * n, hipMemcpyDeviceToHost, st));
+  CPSZ_HIP(hipStreamSynchronize(st));
+  std::sort(hk, hk + n);
+  for (size_t a = 0, b; a < n; a = b) {
+    const uint64_t list = hk[a] >> 44;
+    b = std::lower_bound(hk + a, hk + n, (list + 1) << 44) - hk;
+    CpLists2d& L = out[of[list >> 1]];
+    std::vector<int64_t>& id = L.id[list & 1];
+    std::vector<int32_t>& ty = L.type[list & 1];
+    id.resize(b - a);
+    ty.resize(b - a);
+    for (size_t k = a; k < b; k++) {
+      id[k - a] = (int64_t)(hk[k] >> 4 & ((1ull << 40) - 1));
+      ty[k - a] = (int32_t)(hk[k] & 15);
+    }
+  }
 }
 
 }  // namespace cpsz

@@ -3,7 +3,9 @@
 // compressors (single 2D field; batches of 3D fields).
 #include <algorithm>
 #include <cmath>
+#include <cstdlib>
 #include <cstring>
+#include <memory>
 #include <string>
 #include <vector>
 
@@ -180,13 +182,18 @@ __global__ void __launch_bounds__(256) k_gemm_bf16(int M, int N, int K, const ui
 // ------------------------------------------------------ fused inference --
 // Feature build + both hidden layers + output in one kernel, for compression
 // (training keeps the GEMM path, whose activations the backward pass needs).
-// A wave takes 32 vertices at a time: its lanes write the BF16 features of the
-// 5x5 (2D) / 3x3x3 (3D) patch into the wave's LDS tile (lane t: vertex t%32,
-// features of half t/32), then layer 1 and layer 2 run on
+// A wave takes 32 vertices at a time: its lanes read the 5x5 (2D) / 3x3x3 (3D)
+// patch once into registers (lane t: vertex t%32, features 2k + t/32, whose
+// offsets are constants) and write the BF16 features into the wave's LDS tile, then layer 1 and layer 2 run on
 // v_mfma_f32_32x32x16_bf16 with the transposed BF16 weights resident in LDS,
 // bias + ReLU between them in FP32, and the output layer reduces the 32 lanes
 // that share a row. The hidden rows overwrite the feature tile in place (a
-// wave's LDS reads complete before its later writes). Operand layout: lane t
+// wave's LDS reads complete before its later writes). LDS rows are padded by 16
+// bytes: unpadded, their 128 or 256 bytes put a column's lanes on the same
+// banks. Bound by the feature build's loads and divisions, then by LDS: 12
+// fields of 10 million vertices in all took 4.95 ms with the patch read twice
+// at computed indexes, unpadded rows and 8 waves a CU, 1.31 ms as it stands
+// (the matrix products alone are 0.2 ms). Operand layout: lane t
 // supplies A(t%32, 8*(t/32)+q) and B(8*(t/32)+q, t%32), q = 0..7, and
 // receives D(8*(r/4) + 4*(t/32) + r%4, t%32) in accumulator r.
 typedef __bf16 bf16x8m __attribute__((ext_vector_type(8)));
@@ -195,7 +202,7 @@ template <int DIM>
 struct InferCfg;
 template <>
 struct InferCfg<2> {
-  static constexpr int F = kFeatDim, P = kFeatUsed - 1, WPB = 8;  // 50 patch values, then the bound
+  static constexpr int F = kFeatDim, P = kFeatUsed - 1, WPB = 12;  // 50 patch values, then the bound
 };
 template <>
 struct InferCfg<3> {
@@ -206,6 +213,21 @@ __device__ __forceinline__ bf16x8m lds_bf16x8(const uint16_t* p) {
   bf16x8m v;
   __builtin_memcpy(&v, p, 16);
   return v;
+}
+
+// Sum over the lane's half wave in the order of a butterfly (1, 2, 4, 8, 16):
+// once a group's lanes agree, a mirror reaches the other group as well as an
+// exclusive or does, and needs no LDS.
+template <int CTRL>
+__device__ __forceinline__ float dpp_of(float x) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), CTRL, 0xF, 0xF, true));
+}
+__device__ __forceinline__ float sum_of_32(float x) {
+  x += dpp_of<0xB1>(x);   // quad_perm 1,0,3,2
+  x += dpp_of<0x4E>(x);   // quad_perm 2,3,0,1
+  x += dpp_of<0x141>(x);  // row_half_mirror
+  x += dpp_of<0x140>(x);  // row_mirror
+  return x + __shfl_xor(x, 16);
 }
 
 // W1t[n][k] = bf16(W1[k][n]), W2t[n][k] = bf16(W2[k][n])
@@ -228,13 +250,17 @@ __global__ void __launch_bounds__(64 * InferCfg<DIM>::WPB) k_mlp_infer(
     const double* __restrict__ E, int r1, int r2, int r3, double max_pwr_eb, const uint16_t* __restrict__ W1t,
     const uint16_t* __restrict__ W2t, const float* __restrict__ P, NetLayout L, size_t v0, size_t m,
     uint8_t* __restrict__ gain) {
-  constexpr int F = InferCfg<DIM>::F, NP = InferCfg<DIM>::P, WPB = InferCfg<DIM>::WPB, HALF = F / 2;
-  __shared__ __align__(16) uint16_t sW1[kHidden * F];
-  __shared__ __align__(16) uint16_t sW2[kHidden * kHidden];
+  constexpr int F = InferCfg<DIM>::F, NP = InferCfg<DIM>::P, WPB = InferCfg<DIM>::WPB;
+  constexpr int FP = F + 8, HP = kHidden + 8;  // LDS row pitches
+  __shared__ __align__(16) uint16_t sW1[kHidden * FP];
+  __shared__ __align__(16) uint16_t sW2[kHidden * HP];
   __shared__ float sb1[kHidden], sb2[kHidden], sw3[kHidden];
-  __shared__ __align__(16) uint16_t sbuf[WPB][32 * kHidden];  // features, then the hidden rows
-  for (int i = threadIdx.x; i < kHidden * F; i += blockDim.x) sW1[i] = W1t[i];
-  for (int i = threadIdx.x; i < kHidden * kHidden; i += blockDim.x) sW2[i] = W2t[i];
+  __shared__ __align__(16) uint16_t sbuf[WPB][32 * HP];  // features, then the hidden rows
+  // eight weights at a time (rows of F and kHidden are multiples of eight)
+  for (int i = threadIdx.x * 8; i < kHidden * F; i += blockDim.x * 8)
+    __builtin_memcpy(&sW1[i / F * FP + i % F], __builtin_assume_aligned(W1t + i, 16), 16);
+  for (int i = threadIdx.x * 8; i < kHidden * kHidden; i += blockDim.x * 8)
+    __builtin_memcpy(&sW2[i / kHidden * HP + i % kHidden], __builtin_assume_aligned(W2t + i, 16), 16);
   for (int i = threadIdx.x; i < kHidden; i += blockDim.x) {
     sb1[i] = P[L.b1 + i];
     sb2[i] = P[L.b2 + i];
@@ -244,7 +270,6 @@ __global__ void __launch_bounds__(64 * InferCfg<DIM>::WPB) k_mlp_infer(
   const float b3 = P[L.b3];
   const int wave = threadIdx.x >> 6, t = threadIdx.x & 63, col = t & 31, hf = t >> 5;
   uint16_t* buf = sbuf[wave];
-  const float* src[3] = {U, V, W};
   for (size_t tile = (size_t)blockIdx.x * WPB + wave; tile * 32 < m; tile += (size_t)gridDim.x * WPB) {
     // ---- features (as k_feat2d / k_feat3d write them)
     const size_t q = tile * 32 + col;
@@ -261,38 +286,48 @@ __global__ void __launch_bounds__(64 * InferCfg<DIM>::WPB) k_mlp_infer(
       j = (int)(rem / (size_t)r3);
       k = (int)(rem - (size_t)j * r3);
     }
-    // patch value of feature f (0 outside the field); the largest magnitude
-    // first, then the values again (cached) for the normalized BF16 features
-    auto patch = [&](int f) -> float {
-      int c;
-      bool in;
-      size_t o;
-      if (DIM == 2) {
-        c = f / 25;
-        const int a = (f % 25) / 5, b = f % 5, ii = i + a - 2, jj = j + b - 2;
-        in = ii >= 0 && ii < r1 && jj >= 0 && jj < r2;
-        o = in ? (size_t)ii * r2 + jj : 0;
-      } else {
-        c = f / 27;
-        const int oo = f % 27, ii = i + oo / 9 - 1, jj = j + (oo / 3) % 3 - 1, kk = k + oo % 3 - 1;
-        in = ii >= 0 && ii < r1 && jj >= 0 && jj < r2 && kk >= 0 && kk < r3;
-        o = in ? ((size_t)ii * r2 + jj) * r3 + kk : 0;
+    // patch values (0 outside the field) of features 2 k + hf: both halves'
+    // offsets are constants, a lane takes one of the two
+    constexpr int NV = (NP + 1) / 2;
+    float x[NV];
+#pragma unroll
+    for (int kk = 0; kk < NV; kk++) {
+      bool in[2];
+      size_t o[2];
+      const float* from[2];
+#pragma unroll
+      for (int h = 0; h < 2; h++) {
+        const int f = 2 * kk + h < NP ? 2 * kk + h : 0;
+        if (DIM == 2) {
+          const int ii = i + (f % 25) / 5 - 2, jj = j + f % 5 - 2;
+          in[h] = ii >= 0 && ii < r1 && jj >= 0 && jj < r2;
+          o[h] = (size_t)ii * r2 + jj;
+          from[h] = f / 25 ? V : U;
+        } else {
+          const int oo = f % 27, ii = i + oo / 9 - 1, jj = j + (oo / 3) % 3 - 1, k3 = k + oo % 3 - 1;
+          in[h] = ii >= 0 && ii < r1 && jj >= 0 && jj < r2 && k3 >= 0 && k3 < r3;
+          o[h] = ((size_t)ii * r2 + jj) * r3 + k3;
+          from[h] = f / 27 == 0 ? U : f / 27 == 1 ? V : W;
+        }
+        in[h] = in[h] && 2 * kk + h < NP;
       }
-      return in ? src[c][o] : 0.f;
-    };
-    float smax = 0.f;
-    for (int ff = 0; ff < HALF; ff++) {
-      const int f = hf * HALF + ff;
-      if (f < NP) smax = fmaxf(smax, fabsf(patch(f)));
+      const bool ok = hf ? in[1] : in[0];
+      const float y = (hf ? from[1] : from[0])[ok ? (hf ? o[1] : o[0]) : 0];
+      x[kk] = ok ? y : 0.f;
     }
+    float smax = 0.f;
+#pragma unroll
+    for (int kk = 0; kk < NV; kk++) smax = fmaxf(smax, fabsf(x[kk]));
     smax = fmaxf(smax, __shfl_xor(smax, 32));
     if (!(smax > 0.f)) smax = 1.f;
     const double e = E[v];
     const float le = e > 0 ? fmaxf((float)log2(e / max_pwr_eb), -64.f) / 16.f : -4.f;
-    for (int ff = 0; ff < HALF; ff++) {
-      const int f = hf * HALF + ff;
-      const uint16_t h = f < NP ? f2bf(patch(f) / smax) : (f == NP ? f2bf(le) : (uint16_t)0);
-      buf[col * F + f] = valid ? h : (uint16_t)0;
+#pragma unroll
+    for (int kk = 0; kk < F / 2; kk++) {
+      uint16_t h = 0;
+      if (kk < NV) h = f2bf(x[kk] / smax);
+      if (2 * kk + 1 >= NP) h = 2 * kk + hf < NP ? h : 2 * kk + hf == NP ? f2bf(le) : (uint16_t)0;
+      buf[col * FP + 2 * kk + hf] = valid ? h : (uint16_t)0;
     }
     // ---- layer 1: Z1 = X W1 (K = F)
     floatx16 acc[4];
@@ -301,10 +336,10 @@ __global__ void __launch_bounds__(64 * InferCfg<DIM>::WPB) k_mlp_infer(
       for (int r = 0; r < 16; r++) acc[nt][r] = 0.f;
 #pragma unroll
     for (int ks = 0; ks < F / 16; ks++) {
-      const bf16x8m a = lds_bf16x8(buf + col * F + ks * 16 + hf * 8);
+      const bf16x8m a = lds_bf16x8(buf + col * FP + ks * 16 + hf * 8);
 #pragma unroll
       for (int nt = 0; nt < 4; nt++) {
-        const bf16x8m b = lds_bf16x8(sW1 + (nt * 32 + col) * F + ks * 16 + hf * 8);
+        const bf16x8m b = lds_bf16x8(sW1 + (nt * 32 + col) * FP + ks * 16 + hf * 8);
         acc[nt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, acc[nt], 0, 0, 0);
       }
     }
@@ -315,7 +350,7 @@ __global__ void __launch_bounds__(64 * InferCfg<DIM>::WPB) k_mlp_infer(
       for (int r = 0; r < 16; r++) {
         const int row = 8 * (r >> 2) + 4 * hf + (r & 3), c = nt * 32 + col;
         const float z = acc[nt][r] + sb1[c];
-        buf[row * kHidden + c] = f2bf(z > 0.f ? z : 0.f);
+        buf[row * HP + c] = f2bf(z > 0.f ? z : 0.f);
       }
     // ---- layer 2: Z2 = H1 W2 (K = 128)
 #pragma unroll
@@ -323,10 +358,10 @@ __global__ void __launch_bounds__(64 * InferCfg<DIM>::WPB) k_mlp_infer(
       for (int r = 0; r < 16; r++) acc[nt][r] = 0.f;
 #pragma unroll
     for (int ks = 0; ks < kHidden / 16; ks++) {
-      const bf16x8m a = lds_bf16x8(buf + col * kHidden + ks * 16 + hf * 8);
+      const bf16x8m a = lds_bf16x8(buf + col * HP + ks * 16 + hf * 8);
 #pragma unroll
       for (int nt = 0; nt < 4; nt++) {
-        const bf16x8m b = lds_bf16x8(sW2 + (nt * 32 + col) * kHidden + ks * 16 + hf * 8);
+        const bf16x8m b = lds_bf16x8(sW2 + (nt * 32 + col) * HP + ks * 16 + hf * 8);
         acc[nt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, acc[nt], 0, 0, 0);
       }
     }
@@ -342,7 +377,7 @@ __global__ void __launch_bounds__(64 * InferCfg<DIM>::WPB) k_mlp_infer(
         const float z = acc[nt][r] + sb2[c];
         sacc = fmaf(z > 0.f ? z : 0.f, sw3[c], sacc);
       }
-      for (int o = 1; o < 32; o <<= 1) sacc += __shfl_xor(sacc, o);
+      sacc = sum_of_32(sacc);
       const size_t row = tile * 32 + 8 * (r >> 2) + 4 * hf + (r & 3);
       if (col == r && row < m) {  // the proposal gain = clamp(floor(y), 0, kMaxGain), as k_gain
         const float f = floorf(sacc + b3);
@@ -583,13 +618,15 @@ void mlp_infer_gains(Ctx& ctx, int dim, const float* dU, const float* dV, const 
   uint16_t* W2t = ctx.buf<uint16_t>("inf.w2t", (size_t)kHidden * kHidden);
   const size_t nw = (size_t)kHidden * fdim + (size_t)kHidden * kHidden;
   k_weights_t<<<blocks_for(nw), 256, 0, st>>>(d_params, fdim, L.w1, L.w2, W1t, W2t);
+  // one block of waves fills a CU's LDS: as many blocks as CUs, each loads the
+  // weights once
   const size_t tiles = div_up(m, (size_t)32);
   if (dim == 2) {
-    const int grid = (int)std::min<size_t>(div_up(tiles, (size_t)InferCfg<2>::WPB), 2048);
+    const int grid = (int)std::min<size_t>(div_up(tiles, (size_t)InferCfg<2>::WPB), 256);
     k_mlp_infer<2><<<grid, 64 * InferCfg<2>::WPB, 0, st>>>(dU, dV, nullptr, dE, (int)r1, (int)r2, 1, max_pwr_eb,
                                                           W1t, W2t, d_params, L, v0, m, d_gain);
   } else {
-    const int grid = (int)std::min<size_t>(div_up(tiles, (size_t)InferCfg<3>::WPB), 2048);
+    const int grid = (int)std::min<size_t>(div_up(tiles, (size_t)InferCfg<3>::WPB), 256);
     k_mlp_infer<3><<<grid, 64 * InferCfg<3>::WPB, 0, st>>>(dU, dV, dW, dE, (int)r1, (int)r2, (int)r3, max_pwr_eb,
                                                           W1t, W2t, d_params, L, v0, m, d_gain);
   }
@@ -726,20 +763,6 @@ void train_2d(Ctx& ctx, const std::vector<TrainField>& fields, double max_pwr_eb
 }
 
 namespace {
-void cp_list(Ctx& ctx, const float* dU, const float* dV, size_t r1, size_t r2, std::vector<int64_t>& ids,
-             std::vector<int32_t>& types, bool sos = false) {
-  size_t cap = 1 << 16, count = 0;
-  for (;;) {
-    ids.resize(cap);
-    types.resize(cap);
-    critical_points_2d(ctx, dU, dV, r1, r2, ids.data(), types.data(), cap, &count, sos);
-    if (count <= cap) break;
-    cap = count;
-  }
-  ids.resize(count);
-  types.resize(count);
-}
-
 // simplices whose critical point appeared, vanished or changed type
 std::vector<int64_t> cp_changes(const std::vector<int64_t>& id0, const std::vector<int32_t>& ty0,
                                 const std::vector<int64_t>& id1, const std::vector<int32_t>& ty1) {
@@ -757,19 +780,111 @@ std::vector<int64_t> cp_changes(const std::vector<int64_t>& id0, const std::vect
   return bad;
 }
 
+struct Mark {
+  uint64_t at, value;
+};
+__global__ void k_set_marks(const Mark* __restrict__ m, size_t n, uint8_t* __restrict__ d) {
+  const size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x;
+  if (i < n) d[m[i].at] = (uint8_t)m[i].value;
+}
+
+// out[0] += gains above 0, out[1] += those whose vertex fell back
+__global__ void __launch_bounds__(256) k_count_gains(const uint8_t* __restrict__ gain, const uint8_t* __restrict__ fb,
+                                                     size_t n, unsigned long long* __restrict__ out) {
+  unsigned a = 0, b = 0;
+  for (size_t i = blockIdx.x * (size_t)256 + threadIdx.x; i < n; i += (size_t)gridDim.x * 256) {
+    const bool g = gain[i] != 0, f = fb[i] != 0;
+    a += g;
+    b += g && f;
+  }
+  for (int o = 32; o > 0; o >>= 1) {
+    a += __shfl_xor(a, o);
+    b += __shfl_xor(b, o);
+  }
+  if ((threadIdx.x & 63) == 0) {
+    if (a) atomicAdd(&out[0], (unsigned long long)a);
+    if (b) atomicAdd(&out[1], (unsigned long long)b);
+  }
+}
+
+// The fallback marks of n vertices, on the device and (zero pages until
+// written) on the host; a round sends the marks that it changed. (Whole arrays
+// of bytes sent each round, and the gains fetched to be counted on the host,
+// took 2.1 ms of 15.8 for 12 fields of 10 million vertices in all.)
+class FallbackMarks {
+ public:
+  FallbackMarks(Ctx& ctx, const char* tag, size_t n)
+      : ctx_(ctx), tag_(tag), n_(n), d_(ctx.buf<uint8_t>(tag, n)), h_((uint8_t*)std::calloc(n, 1), &std::free) {
+    CPSZ_REQUIRE(h_, kErrAlloc, "learned compression: out of host memory");
+    CPSZ_HIP(hipMemsetAsync(d_, 0, n, ctx.stream()));
+  }
+  const uint8_t* device() const { return d_; }
+  uint8_t get(size_t i) const { return h_[i]; }
+  void set(size_t i, uint8_t v) {
+    if (h_[i] == v) return;
+    h_[i] = v;
+    touched_.push_back(i);
+  }
+  // every vertex of [b, e) at least v
+  void raise(size_t b, size_t e, uint8_t v) {
+    for (size_t i = b; i < e; i++) h_[i] = std::max(h_[i], v);
+    ranges_.push_back({b, e});
+  }
+  void send() {
+    for (const auto& [b, e] : ranges_)
+      CPSZ_HIP(hipMemcpyAsync(d_ + b, h_.get() + b, e - b, hipMemcpyHostToDevice, ctx_.stream()));
+    ranges_.clear();
+    if (touched_.empty()) return;
+    const std::string t = tag_ + ".marks";
+    const size_t n = touched_.size(), bytes = n * sizeof(Mark);
+    Mark* h = (Mark*)ctx_.host_table(t.c_str(), bytes);
+    Mark* d = (Mark*)ctx_.buf<uint8_t>(t.c_str(), bytes);
+    for (size_t k = 0; k < n; k++) h[k] = Mark{touched_[k], h_[touched_[k]]};
+    touched_.clear();
+    ctx_.upload_table(t.c_str(), d, h, bytes);
+    k_set_marks<<<(unsigned)div_up(n, 256), 256, 0, ctx_.stream()>>>(d, n, d_);
+    CPSZ_HIP(hipGetLastError());
+  }
+  // boosted and fallen-back vertices (the marks are those last sent)
+  void count(const uint8_t* gain, LearnedStats& stats) {
+    hipStream_t st = ctx_.stream();
+    unsigned long long* c = ctx_.buf<unsigned long long>((tag_ + ".cnt").c_str(), 2);
+    unsigned long long* h = (unsigned long long*)ctx_.host_buf((tag_ + ".cnt").c_str(), 16);
+    CPSZ_HIP(hipMemsetAsync(c, 0, 16, st));
+    k_count_gains<<<(unsigned)std::min<size_t>(div_up(n_, 4096), 2048), 256, 0, st>>>(gain, d_, n_, c);
+    CPSZ_HIP(hipGetLastError());
+    CPSZ_HIP(hipMemcpyAsync(h, c, 16, hipMemcpyDeviceToHost, st));
+    CPSZ_HIP(hipStreamSynchronize(st));
+    stats.boosted_vertices = h[0];
+    stats.fallback_vertices = h[1];
+  }
+
+ private:
+  Ctx& ctx_;
+  const std::string tag_;
+  const size_t n_;
+  uint8_t* const d_;
+  std::unique_ptr<uint8_t[], void (*)(void*)> h_;
+  std::vector<size_t> touched_;
+  std::vector<std::pair<size_t, size_t>> ranges_;
+};
+
 // Per-vertex fallback of the learned bound: 0 learned, 1 the analytic bound
 // (which keeps every critical point of the reference's closed-simplex test),
 // 2 stored exactly (eb 0). A triangle the closed test sees change sends its
 // vertices to the analytic bound; one only the Simulation-of-Simplicity test
 // sees change (a degenerate zero the analytic bound need not keep) sends
 // them one step further.
-void mark_triangles(const std::vector<int64_t>& bad, size_t r2, uint8_t* hf, bool sos) {
+void mark_triangles(const std::vector<int64_t>& bad, size_t r2, FallbackMarks& fb, size_t v0, bool sos) {
   for (int64_t sid : bad) {
     const int64_t cell = sid / 2;
     const int t = (int)(sid % 2);
     const size_t ci = (size_t)(cell / (int64_t)(r2 - 1)), cj = (size_t)(cell % (int64_t)(r2 - 1));
     const size_t v[3] = {ci * r2 + cj, t == 0 ? (ci + 1) * r2 + cj : ci * r2 + cj + 1, (ci + 1) * r2 + cj + 1};
-    for (size_t x : v) hf[x] = sos ? (hf[x] ? 2 : 1) : (hf[x] ? hf[x] : 1);
+    for (size_t x : v) {
+      const uint8_t was = fb.get(v0 + x);
+      fb.set(v0 + x, sos ? (was ? 2 : 1) : (was ? was : 1));
+    }
   }
 }
 
@@ -779,23 +894,20 @@ void mark_triangles(const std::vector<int64_t>& bad, size_t r2, uint8_t* hf, boo
 constexpr int kLearnRounds = 16;
 constexpr int kLearnLast = kLearnRounds + 3;
 
-// Falls back as the round requires; returns false when the field is done.
-bool verify_round_2d(int it, const std::vector<int64_t>& id0, const std::vector<int32_t>& ty0,
-                     const std::vector<int64_t>& is0, const std::vector<int32_t>& ts0,
-                     const std::vector<int64_t>& id1, const std::vector<int32_t>& ty1,
-                     const std::vector<int64_t>& is1, const std::vector<int32_t>& ts1, size_t r2, uint8_t* hf,
+// Falls back as the round requires (v0: the field's first vertex among the
+// marks); returns false when the field is done.
+bool verify_round_2d(int it, const CpLists2d& was, const CpLists2d& now, size_t r2, FallbackMarks& fb, size_t v0,
                      size_t n) {
-  const std::vector<int64_t> bad = cp_changes(id0, ty0, id1, ty1);
-  const std::vector<int64_t> bad_s = cp_changes(is0, ts0, is1, ts1);
+  const std::vector<int64_t> bad = cp_changes(was.id[0], was.type[0], now.id[0], now.type[0]);
+  const std::vector<int64_t> bad_s = cp_changes(was.id[1], was.type[1], now.id[1], now.type[1]);
   if (bad.empty() && bad_s.empty()) return false;
   CPSZ_REQUIRE(bad.empty() || it < kLearnRounds, kErrInternal,
                "learned compression: the plain bound changed a critical point");
   CPSZ_REQUIRE(it < kLearnLast, kErrInternal, "learned compression did not converge");
-  mark_triangles(bad, r2, hf, false);
-  mark_triangles(bad_s, r2, hf, true);
-  if (it + 1 == kLearnRounds)
-    for (size_t v = 0; v < n; v++) hf[v] = hf[v] ? hf[v] : 1;
-  if (it + 1 == kLearnLast) std::fill(hf, hf + n, 2);
+  mark_triangles(bad, r2, fb, v0, false);
+  mark_triangles(bad_s, r2, fb, v0, true);
+  if (it + 1 == kLearnRounds) fb.raise(v0, v0 + n, 1);
+  if (it + 1 == kLearnLast) fb.raise(v0, v0 + n, 2);
   return true;
 }
 }  // namespace
@@ -812,29 +924,23 @@ void compress_2d_learned(Ctx& ctx, const float* dU, const float* dV, size_t r1, 
   CPSZ_HIP(hipMemcpyAsync(P, params, kNumParams * 4, hipMemcpyHostToDevice, st));
   uint8_t* gain = ctx.buf<uint8_t>("ln.gain", n);
   mlp_infer_gains(ctx, 2, dU, dV, nullptr, E, r1, r2, 1, max_pwr_eb, P, 0, n, gain);
-  std::vector<uint8_t> hg(n), hf(n, 0);
-  CPSZ_HIP(hipMemcpyAsync(hg.data(), gain, n, hipMemcpyDeviceToHost, st));
-  std::vector<int64_t> id0, id1, is0, is1;
-  std::vector<int32_t> ty0, ty1, ts0, ts1;
-  cp_list(ctx, dU, dV, r1, r2, id0, ty0);  // synchronizes
-  cp_list(ctx, dU, dV, r1, r2, is0, ts0, true);
-  for (size_t v = 0; v < n; v++) stats.boosted_vertices += hg[v] != 0;
-  uint8_t* fb = ctx.buf<uint8_t>("ln.fb", n);
+  std::vector<CpLists2d> cp0, cp1;
+  critical_points_2d_batch(ctx, {CpField2d{dU, dV, r1, r2}}, cp0);
+  FallbackMarks fb(ctx, "ln.fb", n);
   float* dU2 = ctx.buf<float>("ln.u2", n);
   float* dV2 = ctx.buf<float>("ln.v2", n);
   EbOverride ov;
   ov.gain = gain;
-  ov.fallback = fb;
+  ov.fallback = fb.device();
   for (int it = 0;; it++) {
-    CPSZ_HIP(hipMemcpyAsync(fb, hf.data(), n, hipMemcpyHostToDevice, st));
+    fb.send();
     compress_2d_device(ctx, dU, dV, r1, r2, max_pwr_eb, out, ov);
     decompress_2d_device(ctx, out.data, nullptr, out.size, r1, r2, dU2, dV2);
-    cp_list(ctx, dU2, dV2, r1, r2, id1, ty1);
-    cp_list(ctx, dU2, dV2, r1, r2, is1, ts1, true);
+    critical_points_2d_batch(ctx, {CpField2d{dU2, dV2, r1, r2}}, cp1);
     stats.iterations = it + 1;
-    if (!verify_round_2d(it, id0, ty0, is0, ts0, id1, ty1, is1, ts1, r2, hf.data(), n)) break;
+    if (!verify_round_2d(it, cp0[0], cp1[0], r2, fb, 0, n)) break;
   }
-  for (size_t v = 0; v < n; v++) stats.fallback_vertices += hf[v] && hg[v];
+  fb.count(gain, stats);
 }
 
 // =================================================================== 3D ====
@@ -1089,7 +1195,7 @@ void compress_3d_learned_batch(Ctx& ctx, const std::vector<TrainField3>& fields,
   float* P = ctx.buf<float>("l3.p", kNumParams3);
   CPSZ_HIP(hipMemcpyAsync(P, params, kNumParams3 * 4, hipMemcpyHostToDevice, st));
   uint8_t* gain = ctx.buf<uint8_t>("l3.gain", ntot);
-  uint8_t* fb = ctx.buf<uint8_t>("l3.fb", ntot);
+  FallbackMarks fb(ctx, "l3.fb", ntot);
   double* E = ctx.buf<double>("l3.e", maxn);
   for (size_t k = 0; k < nf; k++) {
     const TrainField3& F = fields[k];
@@ -1097,10 +1203,6 @@ void compress_3d_learned_batch(Ctx& ctx, const std::vector<TrainField3>& fields,
     analytic_eb_3d(ctx, F.dU, F.dV, F.dW, F.r1, F.r2, F.r3, max_pwr_eb, E);
     mlp_infer_gains(ctx, 3, F.dU, F.dV, F.dW, E, F.r1, F.r2, F.r3, max_pwr_eb, P, 0, n, gain + nofs[k]);
   }
-  std::vector<uint8_t> hg(ntot), hf(ntot, 0);
-  CPSZ_HIP(hipMemcpyAsync(hg.data(), gain, ntot, hipMemcpyDeviceToHost, st));
-  CPSZ_HIP(hipStreamSynchronize(st));
-  for (size_t v = 0; v < ntot; v++) stats.boosted_vertices += hg[v] != 0;
   // ---- critical points of the originals
   std::vector<std::vector<int64_t>> id0(nf);
   std::vector<std::vector<int32_t>> ty0(nf);
@@ -1123,7 +1225,7 @@ void compress_3d_learned_batch(Ctx& ctx, const std::vector<TrainField3>& fields,
   const int kMaxIter = 16;
   for (int it = 0; it <= kMaxIter && !pending.empty(); it++) {
     if (it == kMaxIter)  // the plain method for whatever is left
-      for (size_t k : pending) std::fill(hf.begin() + nofs[k], hf.begin() + nofs[k + 1], 1);
+      for (size_t k : pending) fb.raise(nofs[k], nofs[k + 1], 1);
     std::vector<Field3d> sub;
     std::vector<EbOverride> ov;
     for (size_t k : pending) {
@@ -1131,10 +1233,10 @@ void compress_3d_learned_batch(Ctx& ctx, const std::vector<TrainField3>& fields,
       sub.push_back(Field3d{F.dU, F.dV, F.dW, F.r1, F.r2, F.r3});
       EbOverride o;
       o.gain = gain + nofs[k];
-      o.fallback = fb + nofs[k];
+      o.fallback = fb.device() + nofs[k];
       ov.push_back(o);
-      CPSZ_HIP(hipMemcpyAsync(fb + nofs[k], hf.data() + nofs[k], nofs[k + 1] - nofs[k], hipMemcpyHostToDevice, st));
     }
+    fb.send();
     BatchOut bo;
     compress_3d_batch(ctx, sub, max_pwr_eb, cfg, bo, &ov);
     std::vector<const uint8_t*> ins;
@@ -1173,7 +1275,7 @@ void compress_3d_learned_batch(Ctx& ctx, const std::vector<TrainField3>& fields,
         int t = 0;
         while (judge_tet_sid(t) != which) t++;
         const int cs[4] = {0, judge_tet_a(t), judge_tet_b(t), 7};
-        for (int c : cs) hf[nofs[k] + org + (size_t)(c >> 2) * d0 + (size_t)((c >> 1) & 1) * d1 + (c & 1)] = 1;
+        for (int c : cs) fb.set(nofs[k] + org + (size_t)(c >> 2) * d0 + (size_t)((c >> 1) & 1) * d1 + (c & 1), 1);
       }
       still.push_back(k);
     }
@@ -1182,7 +1284,7 @@ void compress_3d_learned_batch(Ctx& ctx, const std::vector<TrainField3>& fields,
     pending.swap(still);
   }
   CPSZ_REQUIRE(pending.empty(), kErrInternal, "learned compression did not converge");
-  for (size_t v = 0; v < ntot; v++) stats.fallback_vertices += hf[v] && hg[v];
+  fb.count(gain, stats);
   base = out;
 }
 
@@ -1213,7 +1315,7 @@ void compress_2d_learned_batch(Ctx& ctx, const std::vector<TrainField>& fields, 
   float* P = ctx.buf<float>("l2b.p", kNumParams);
   CPSZ_HIP(hipMemcpyAsync(P, params, kNumParams * 4, hipMemcpyHostToDevice, st));
   uint8_t* gain = ctx.buf<uint8_t>("l2b.gain", ntot);
-  uint8_t* fb = ctx.buf<uint8_t>("l2b.fb", ntot);
+  FallbackMarks fb(ctx, "l2b.fb", ntot);
   double* E = ctx.buf<double>("l2b.e", maxn);
   for (size_t k = 0; k < nf; k++) {
     const TrainField& F = fields[k];
@@ -1221,17 +1323,11 @@ void compress_2d_learned_batch(Ctx& ctx, const std::vector<TrainField>& fields, 
     analytic_eb_2d(ctx, F.dU, F.dV, F.r1, F.r2, max_pwr_eb, E);
     mlp_infer_gains(ctx, 2, F.dU, F.dV, nullptr, E, F.r1, F.r2, 1, max_pwr_eb, P, 0, n, gain + nofs[k]);
   }
-  std::vector<uint8_t> hg(ntot), hf(ntot, 0);
-  CPSZ_HIP(hipMemcpyAsync(hg.data(), gain, ntot, hipMemcpyDeviceToHost, st));
-  CPSZ_HIP(hipStreamSynchronize(st));
-  for (size_t v = 0; v < ntot; v++) stats.boosted_vertices += hg[v] != 0;
   // ---- critical points of the originals (closed-simplex and SoS tests)
-  std::vector<std::vector<int64_t>> id0(nf), is0(nf);
-  std::vector<std::vector<int32_t>> ty0(nf), ts0(nf);
-  for (size_t k = 0; k < nf; k++) {
-    cp_list(ctx, fields[k].dU, fields[k].dV, fields[k].r1, fields[k].r2, id0[k], ty0[k]);
-    cp_list(ctx, fields[k].dU, fields[k].dV, fields[k].r1, fields[k].r2, is0[k], ts0[k], true);
-  }
+  std::vector<CpField2d> judged;
+  for (const TrainField& F : fields) judged.push_back(CpField2d{F.dU, F.dV, F.r1, F.r2});
+  std::vector<CpLists2d> cp0, cp1;
+  critical_points_2d_batch(ctx, judged, cp0);
   // ---- verify and fall back until every field keeps its critical points
   float* dec = ctx.buf<float>("l2b.dec", 2 * ntot);
   std::vector<size_t> soff(nf + 1, 0);
@@ -1252,10 +1348,10 @@ void compress_2d_learned_batch(Ctx& ctx, const std::vector<TrainField>& fields, 
       sub.push_back(Field2d{F.dU, F.dV, F.r1, F.r2});
       EbOverride o;
       o.gain = gain + nofs[k];
-      o.fallback = fb + nofs[k];
+      o.fallback = fb.device() + nofs[k];
       ov.push_back(o);
-      CPSZ_HIP(hipMemcpyAsync(fb + nofs[k], hf.data() + nofs[k], nofs[k + 1] - nofs[k], hipMemcpyHostToDevice, st));
     }
+    fb.send();
     BatchOut bo;
     compress_2d_batch(ctx, sub, max_pwr_eb, cfg, bo, &ov);
     std::vector<const uint8_t*> ins;
@@ -1270,16 +1366,15 @@ void compress_2d_learned_batch(Ctx& ctx, const std::vector<TrainField>& fields, 
       outs.push_back(Field2dOut{d, d + (nofs[k + 1] - nofs[k]), F.r1, F.r2});
     }
     decompress_2d_batch(ctx, ins, insz, outs, cfg);
+    judged.clear();
+    for (const Field2dOut& o : outs) judged.push_back(CpField2d{o.dU, o.dV, o.r1, o.r2});
+    critical_points_2d_batch(ctx, judged, cp1);
     stats.iterations = it + 1;
     std::vector<size_t> still;
     for (size_t q = 0; q < pending.size(); q++) {
       const size_t k = pending[q];
       const TrainField& F = fields[k];
-      std::vector<int64_t> id1, is1;
-      std::vector<int32_t> ty1, ts1;
-      cp_list(ctx, outs[q].dU, outs[q].dV, F.r1, F.r2, id1, ty1);
-      cp_list(ctx, outs[q].dU, outs[q].dV, F.r1, F.r2, is1, ts1, true);
-      if (!verify_round_2d(it, id0[k], ty0[k], is0[k], ts0[k], id1, ty1, is1, ts1, F.r2, hf.data() + nofs[k],
+      if (!verify_round_2d(it, cp0[k], cp1[q], F.r2, fb, nofs[k],
                            nofs[k + 1] - nofs[k])) {
         CPSZ_REQUIRE(bo.size[q] <= soff[k + 1] - soff[k], kErrInternal, "learned stream bound exceeded");
         CPSZ_HIP(hipMemcpyAsync(out + soff[k], bo.base + bo.off[q], bo.size[q], hipMemcpyDeviceToDevice, st));
@@ -1293,7 +1388,7 @@ void compress_2d_learned_batch(Ctx& ctx, const std::vector<TrainField>& fields, 
     pending.swap(still);
   }
   CPSZ_REQUIRE(pending.empty(), kErrInternal, "learned compression did not converge");
-  for (size_t v = 0; v < ntot; v++) stats.fallback_vertices += hf[v] && hg[v];
+  fb.count(gain, stats);
   base = out;
 }
 
