@@ -114,3 +114,27 @@ def test_slow_resynchronization(shape, sec, kind, depth):
     for got in [cz.sz_decompress_cp_preserve_2d_offline(t, r1, r2)] + batch:
         for g, e in zip(got, want):
             assert np.array_equal(g.view(np.uint32), e.view(np.uint32))
+
+
+def test_batch_unpredictable_values():
+    """Blocks with no, few and only unpredictable codes (land is stored as it is) in one batch, against the
+    single-field decoder."""
+    shapes = [(70, 300), (25, 13), (200, 97), (1, 40), (37, 1), (12, 12)]
+    dev, streams, want = [], [], []
+    for k, (r1, r2) in enumerate(shapes):
+        print(f"[unpredictable] {r1}x{r2}", flush=True)
+        U, V = _field(r1, r2)
+        rng = np.random.default_rng(k)
+        for F in (U, V):
+            F[rng.random(F.shape) < 0.03] = 0
+            F[r1 // 2:, : (2 * r2) // 3] = 0
+        s = cz.sz_compress_cp_preserve_2d_offline(U, V, 0.05)
+        want.append(cz.sz_decompress_cp_preserve_2d_offline(s, r1, r2))
+        streams.append(torch.from_numpy(np.array(s)).cuda())
+    outs = [(torch.empty(*s, device="cuda"), torch.empty(*s, device="cuda")) for s in shapes]
+    torch.cuda.synchronize()
+    cz.decompress_2d_batch_dev([(x.data_ptr(), x.numel()) for x in streams], shapes,
+                               [(u.data_ptr(), v.data_ptr()) for u, v in outs])
+    for o, w in zip(outs, want):
+        for g, e in zip(o, w):
+            assert np.array_equal(g.cpu().numpy().view(np.uint32), np.asarray(e).reshape(g.shape).view(np.uint32))
