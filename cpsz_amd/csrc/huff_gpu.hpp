@@ -686,16 +686,18 @@ __global__ void k_dec_chain(MDecTable jobs, uint64_t* totals);
 // block's 256 consecutive segments are contiguous in the output: they are
 // gathered in LDS and written out by consecutive threads (coalesced), instead
 // of each thread storing its own run one symbol at a time (64 scattered
-// 2-byte stores per instruction, which reach HBM as ~15x the bytes). A block
-// whose run exceeds the staging buffer writes directly. Sink::kBytes (1 or 2)
+// 2-byte stores per instruction, which reach HBM as ~15x the bytes), a
+// stage's worth after the other. Sink::kBytes (1 or 2)
 // is the width of a staged symbol. Bound by the decode's LDS latency, then by
-// the sinks' index arithmetic: 96 fields' ids 1.85 -> 1.56 ms and codes
+// the sinks' index arithmetic. 96 fields' ids 1.85 -> 1.56 ms and codes
 // 2.97 -> 2.38 ms with several codes from one fetched window in place of a bit
-// buffer refilled under a branch.
+// buffer refilled under a branch; 1.25 and 2.22 ms with stages small enough for
+// three blocks a CU, taken in turn (ids at 1.5 bits a code make 44000 symbols a
+// block, which a stage of 32768 left to scattered stores).
 template <int kBytes>
 struct DecStage {
   using T = typename std::conditional<kBytes == 1, uint8_t, uint16_t>::type;
-  static constexpr uint32_t kCap = kBytes == 1 ? 32768 : 12288;  // symbols per block
+  static constexpr uint32_t kCap = kBytes == 1 ? 24576 : 12288;  // symbols at a time: three blocks a CU
 };
 
 // Exclusive scan of the block's 256 values (x of thread 255 is the last);
@@ -746,56 +748,58 @@ __device__ __forceinline__ void dec_write_block(const MDecJob& J, const Sink& si
     __syncthreads();
   }
   const uint32_t limit = (uint32_t)min((uint64_t)tot, n - first);
-  if (limit > Stage::kCap) {  // uniform across the block
-    while (p < end && o < limit) out.put(first + o++, dec_one(t, slut, bits, p));
-    return;
-  }
   using S = typename Stage::T;
-  if (Sink::kBytes == 1) {
-    // up to 6 codes per fetch while they all start before `end` and fit
-    while (p < end && o < limit) {
-      uint32_t win = bits.window(p);
-      bool none = true;
+  // (o0 and o1 are uniform; a lane's run may span two stages)
+  for (uint32_t o0 = 0; o0 < limit; o0 += Stage::kCap) {
+    const uint32_t o1 = min(limit, o0 + Stage::kCap);
+    S* const at = stage - o0;
+    if (Sink::kBytes == 1) {
+      // up to 6 codes per fetch while they all start before `end` and fit
+      while (p < end && o < o1) {
+        uint32_t win = bits.window(p);
+        bool none = true;
 #pragma unroll
-      for (int r = 0; r < 2; r++) {
-        const uint32_t m = md[win & kLutMask];
-        const uint32_t len = m & 0xF, k = (m >> 4) & 3;
-        if (!k || p + len > end || o + k > limit) break;
-        S* d = stage + o;
-        d[0] = (S)(m >> 8);
-        if (k > 1) d[1] = (S)(m >> 16);
-        if (k > 2) d[2] = (S)(m >> 24);
-        o += k;
-        p += len;
-        win >>= len;
-        none = false;
+        for (int r = 0; r < 2; r++) {
+          const uint32_t m = md[win & kLutMask];
+          const uint32_t len = m & 0xF, k = (m >> 4) & 3;
+          if (!k || p + len > end || o + k > o1) break;
+          S* d = at + o;
+          d[0] = (S)(m >> 8);
+          if (k > 1) d[1] = (S)(m >> 16);
+          if (k > 2) d[2] = (S)(m >> 24);
+          o += k;
+          p += len;
+          win >>= len;
+          none = false;
+        }
+        if (none) at[o++] = (S)dec_one(t, slut, bits, p);
       }
-      if (none) stage[o++] = (S)dec_one(t, slut, bits, p);
-    }
-  } else {
-    // up to 3 codes per fetch
-    while (p < end && o < limit) {
-      const uint32_t win = bits.window(p);
-      uint32_t e = slut[win & kLutMask];
-      if (!short_code(e)) {
-        stage[o++] = (S)long_code(t, bits, e, p);
-        continue;
-      }
-      uint32_t used = e & 0xFF;
-      stage[o++] = (S)(e >> 8);
-      p += used;
+    } else {
+      // up to 3 codes per fetch
+      while (p < end && o < o1) {
+        const uint32_t win = bits.window(p);
+        uint32_t e = slut[win & kLutMask];
+        if (!short_code(e)) {
+          at[o++] = (S)long_code(t, bits, e, p);
+          continue;
+        }
+        uint32_t used = e & 0xFF;
+        at[o++] = (S)(e >> 8);
+        p += used;
 #pragma unroll
-      for (int r = 0; r < 2; r++) {
-        e = slut[(win >> used) & kLutMask];
-        if (p >= end || o >= limit || !short_code(e) || used > 32 - kLutBits) break;
-        stage[o++] = (S)(e >> 8);
-        used += e & 0xFF;
-        p += e & 0xFF;
+        for (int r = 0; r < 2; r++) {
+          e = slut[(win >> used) & kLutMask];
+          if (p >= end || o >= o1 || !short_code(e) || used > 32 - kLutBits) break;
+          at[o++] = (S)(e >> 8);
+          used += e & 0xFF;
+          p += e & 0xFF;
+        }
       }
     }
+    __syncthreads();
+    for (uint32_t x = o0 + threadIdx.x; x < o1; x += blockDim.x) out.put(first + x, at[x]);
+    __syncthreads();
   }
-  __syncthreads();
-  for (uint32_t x = threadIdx.x; x < limit; x += blockDim.x) out.put(first + x, stage[x]);
 }
 
 template <class Sink>
