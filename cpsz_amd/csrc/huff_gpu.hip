@@ -193,43 +193,68 @@ __global__ void __launch_bounds__(256) k_dec_follow(MDecTable jobs) {
   }
 }
 
-// The true chain over a stream's blocks, 64 at a time: the maps of 64 blocks
-// (one per lane, the next 64 in flight) are followed with lane reads, then the
-// lanes fetch the chosen totals and sum them.
-__global__ void __launch_bounds__(64) k_dec_chain(MDecTable jobs, uint64_t* __restrict__ totals) {
+// The true chain over a stream's blocks, 64 to a wave and 1024 at a time. Each
+// wave first composes its blocks' maps (lane e follows entry e, the maps come
+// by lane reads), the waves' maps then give every wave its entry, and it
+// follows its blocks once more from there; the lanes fetch the chosen totals
+// and sum them. One wave alone, 64 blocks after the other, took 0.19 ms for the
+// codes of a 256^3 field.
+__global__ void __launch_bounds__(1024) k_dec_chain(MDecTable jobs, uint64_t* __restrict__ totals) {
+  __shared__ uint32_t leads[16][16];  // [wave][entry]
+  __shared__ uint64_t sum[16];
   const MDecJob& J = jobs[blockIdx.x];
-  const uint32_t lane = threadIdx.x, nblk = J.nblk;
+  const uint32_t lane = threadIdx.x & 63, w = threadIdx.x >> 6, nblk = J.nblk;
   uint32_t cur = 0;
   uint64_t pos = 0;
-  // lanes past the last block lead nowhere and hold nothing
-  uint32_t one = lane < nblk ? J.bsel[lane] : 1u << 31;
-  uint64_t map = lane < nblk ? J.bmap[lane] : 0;
-  for (uint32_t b0 = 0; b0 < nblk; b0 += 64) {
-    const uint32_t b = b0 + lane, bn = b + 64;
-    const uint32_t one0 = one, lo = (uint32_t)map, hi = (uint32_t)(map >> 32);
-    one = bn < nblk ? J.bsel[bn] : 1u << 31;
-    map = bn < nblk ? J.bmap[bn] : 0;
-    uint32_t mine = 0;
-    if (__all(one0 >> 31)) {
-      cur = __builtin_amdgcn_readlane(lo, 63) & 15u;
+  for (uint32_t b0 = 0; b0 < nblk; b0 += 1024) {
+    const uint32_t b = b0 + threadIdx.x;
+    // lanes past the last block lead nowhere and hold nothing
+    const uint32_t one = b < nblk ? J.bsel[b] : 1u << 31;
+    const uint64_t map = b < nblk ? J.bmap[b] : 0;
+    const uint32_t lo = (uint32_t)map, hi = (uint32_t)(map >> 32);
+    const bool all_one = __all(one >> 31);
+    auto map_of = [&](uint32_t k) {
+      return (uint64_t)(uint32_t)__builtin_amdgcn_readlane(hi, k) << 32 | (uint32_t)__builtin_amdgcn_readlane(lo, k);
+    };
+    uint32_t c = lane & 15;
+    if (all_one) {
+      c = __builtin_amdgcn_readlane(lo, 63) & 15u;
     } else {
 #pragma unroll
+      for (uint32_t k = 0; k < 64; k++) c = (uint32_t)(map_of(k) >> (4 * c)) & 15u;
+    }
+    if (lane < 16) leads[w][lane] = c;
+    __syncthreads();
+    uint32_t entry = 0;
+    for (uint32_t q = 0; q < 16; q++) {
+      entry = q == w ? cur : entry;
+      cur = leads[q][cur];
+    }
+    uint32_t mine = 0;
+    if (!all_one) {
+      uint32_t e = __builtin_amdgcn_readfirstlane(entry);
+#pragma unroll
       for (uint32_t k = 0; k < 64; k++) {
-        mine = lane == k ? cur : mine;
-        const uint64_t m = (uint64_t)(uint32_t)__builtin_amdgcn_readlane(hi, k) << 32 |
-                           (uint32_t)__builtin_amdgcn_readlane(lo, k);
-        cur = (uint32_t)(m >> (4 * cur)) & 15u;
+        mine = lane == k ? e : mine;
+        e = (uint32_t)(map_of(k) >> (4 * e)) & 15u;
       }
     }
     const uint32_t tot = b < nblk ? J.btot[(size_t)b * kCand + mine] : 0u;
-    uint32_t incl = wave_incl_scan(tot);
-    if (b < nblk) {
-      J.bsel[b] = one0 | mine;
-      J.boff[b] = pos + incl - tot;
+    const uint32_t incl = wave_incl_scan(tot);
+    if (lane == 63) sum[w] = incl;
+    __syncthreads();
+    uint64_t before = 0, all = 0;
+    for (uint32_t q = 0; q < 16; q++) {
+      before += q < w ? sum[q] : 0;
+      all += sum[q];
     }
-    pos += __builtin_amdgcn_readlane(incl, 63);
+    if (b < nblk) {
+      J.bsel[b] = one | mine;
+      J.boff[b] = pos + before + incl - tot;
+    }
+    pos += all;
   }
-  if (lane == 0) totals[blockIdx.x] = pos;
+  if (threadIdx.x == 0) totals[blockIdx.x] = pos;
 }
 
 // Level-2 entry for the K bits u below `node`: sym << 8 | length of the leaf

@@ -985,7 +985,7 @@ DecodeResult decode_streams(Ctx& ctx, const DecJob<Sink>* jobs, int nj, const ch
   k_dec_serial<<<na, 64, 0, st>>>(tab, err, over);
   ctx.mark((t + ".cand").c_str());
   k_dec_follow<<<nblocks, 256, 0, st>>>(tab);
-  k_dec_chain<<<na, 64, 0, st>>>(tab, totals);
+  k_dec_chain<<<na, 1024, 0, st>>>(tab, totals);
   ctx.mark((t + ".chain").c_str());
   k_dec_write<Sink><<<nblocks, 256, 0, st>>>(tab);
   CPSZ_HIP(hipGetLastError());
