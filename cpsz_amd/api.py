@@ -101,6 +101,7 @@ _SIGS = {
     "cpsz_set_exact_2d_bounds": [C.c_int],
     "cpsz_tri_bound_2d_fast_host": [_P, _SZ, C.c_int, _P],
     "cpsz_ratio_ge1_host": [_P, _P, _SZ, _P],
+    "cpsz_wave2d_span": [_SZ, _SZ, C.c_int, C.POINTER(C.c_int), C.POINTER(C.c_uint64)],
 }
 
 
@@ -641,6 +642,14 @@ def set_exact_2d_bounds(on: bool) -> None:
     (default) = FP32 approximations of the last FP64 steps with exact fix-ups,
     True = every step in FP64. Both give identical streams."""
     _check(lib().cpsz_set_exact_2d_bounds(int(bool(on))))
+
+
+def wave2d_span(r1: int, r2: int, value_bytes: int):
+    """How the 2D wavefront addresses a field (for testing): whether by 64-bit offsets within a strip of rows, and
+    the bytes that a strip spans."""
+    far, span = C.c_int(), C.c_uint64()
+    _check(lib().cpsz_wave2d_span(r1, r2, value_bytes, C.byref(far), C.byref(span)))
+    return bool(far.value), span.value
 
 
 def tri_bound_2d_fast_host(uv6, ulps: int = 0):

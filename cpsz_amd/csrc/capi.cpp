@@ -786,6 +786,19 @@ int cpsz_lorenzo2d_emulate(const float* x, const uint16_t* c, size_t r1, size_t 
   });
 }
 
+int cpsz_wave2d_span(size_t r1, size_t r2, int value_bytes, int* far, uint64_t* span) {
+  return guarded([&] {
+    CPSZ_REQUIRE(r1 && r2 && far && span && (value_bytes == 4 || value_bytes == 8), kErrArg, "bad arguments");
+    const Tile2d t(r1, r2);
+    const size_t cols = t.row_len, rows = std::min<size_t>(t.column ? 1 : r1, 64);
+    // row l's columns are at steps l to l + cols - 1
+    const int last = (int)rows - 1;
+    const size_t tile = t.column ? t.at((int)cols - 1, 0) : t.at(last, (int)cols - 1);
+    *far = far_strip(cols, value_bytes);
+    *span = (std::max(rows * cols - 1, tile) + 1) * value_bytes;
+  });
+}
+
 int cpsz_set_timing(int device, int on) {
   return guarded([&] { ctx_of(device).timing = on != 0; });
 }

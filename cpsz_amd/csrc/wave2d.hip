@@ -129,7 +129,7 @@ __device__ __forceinline__ double restore(float pred, const Elem<double>& e) {
 // nothing. Buffer accesses do that in the address unit (offsets past the
 // resource's range), so every load and store is issued without a branch, and
 // the compiler can count the loads in flight. FAR: strips that span 4 GiB and
-// more take 64-bit addresses and masks.
+// more (far_strip) take 64-bit addresses and masks.
 template <typename V, bool FAR>
 struct Part;
 
@@ -552,13 +552,6 @@ __global__ void __launch_bounds__(256) k_wave2d_clear(StripBatch<T> b) {
   if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) *b.ticket = 0;
 }
 
-// A strip's rows, in bytes, no longer fit 32 bits: the kernel's 64-bit
-// addressing.
-template <typename T>
-bool far_rows(const Strip2dT<T>& f) {
-  return (uint64_t)f.r2 * 64 * sizeof(T) >= (1ull << 32);
-}
-
 // A field of one column is the same chain as a field of one row (each value's
 // prediction is its one neighbour), and its tiles are laid out as one.
 template <typename T>
@@ -581,7 +574,7 @@ void launch_one(Ctx& ctx, Strip2dT<T> f, int grid_cap) {
   const size_t words = published_words(f);
   k_wave2d_clear<T><<<(unsigned)std::min<size_t>(div_up(words, 256) + 1, 1024), 256, 0, st>>>(b);
   const int grid = std::min(b.items, grid_cap);
-  if (far_rows(f)) k_wave2d<T, S, COMPRESS, true><<<grid, 256 * S, 0, st>>>(b);
+  if (far_strip(f.r2, sizeof(T))) k_wave2d<T, S, COMPRESS, true><<<grid, 256 * S, 0, st>>>(b);
   else k_wave2d<T, S, COMPRESS, false><<<grid, 256 * S, 0, st>>>(b);
   CPSZ_HIP(hipGetLastError());
 }
@@ -622,8 +615,10 @@ void launch_many(Ctx& ctx, std::vector<Strip2d>& f, int grid_cap) {
   b.ticket = (int*)(d + ((tbytes + sbytes + 15) & ~(size_t)15));
   k_wave2d_clear<float><<<dim3((unsigned)std::min<size_t>(div_up(max_words, 256 * 8) + 1, 64), (unsigned)nf), 256, 0, st>>>(b);
   const int grid = std::min(b.items, grid_cap);
-  if (std::any_of(g.begin(), g.end(), far_rows<float>)) k_wave2d<float, kStrips, COMPRESS, true><<<grid, 256 * kStrips, 0, st>>>(b);
-  else k_wave2d<float, kStrips, COMPRESS, false><<<grid, 256 * kStrips, 0, st>>>(b);
+  if (std::any_of(g.begin(), g.end(), [](const Strip2d& x) { return far_strip(x.r2, sizeof(float)); }))
+    k_wave2d<float, kStrips, COMPRESS, true><<<grid, 256 * kStrips, 0, st>>>(b);
+  else
+    k_wave2d<float, kStrips, COMPRESS, false><<<grid, 256 * kStrips, 0, st>>>(b);
   CPSZ_HIP(hipGetLastError());
 }
 

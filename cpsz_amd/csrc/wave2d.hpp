@@ -95,6 +95,12 @@ template <typename T>
 inline int strip_groups(size_t r1) {
   return (int)div_up(r1, (size_t)64 * (sizeof(T) == 8 ? kStrips64 : kStrips));
 }
+// The wavefront addresses a strip's elements by 32-bit byte offsets from its
+// first one, unless the strip spans 4 GiB: row-major it takes 64 rows of r2
+// values, in tiles up to 78 steps a row more.
+inline bool far_strip(size_t r2, size_t value_bytes) {
+  return div_up(r2 + 63, (size_t)kTileSteps) * (64 * kTileSteps) * value_bytes >= (1ull << 32);
+}
 // 64-bit words of a field's boundary rows (enough for either type)
 inline size_t bnd_words(size_t r1, size_t r2) { return 2 * div_up(r1, (size_t)64 * kStrips64) * r2; }
 

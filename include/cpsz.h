@@ -242,6 +242,12 @@ int cpsz_eval_exp2f(const float* y, size_t n, float* out);
 int cpsz_lorenzo2d_emulate(const float* x, const uint16_t* c, size_t r1, size_t r2, int wide,
                            uint16_t* q, float* recon);
 
+/* How the 2D wavefront addresses a field of r1 x r2 values of value_bytes each
+ * (for testing): *far is 1 if it takes 64-bit offsets within a strip of rows,
+ * *span the bytes from a strip's first value to its last one's end, in the
+ * row-major arrays or in the codec's own, whichever is more. */
+int cpsz_wave2d_span(size_t r1, size_t r2, int value_bytes, int* far, uint64_t* span);
+
 /* Host emulations of the device 3D arithmetic: per-vertex bounds (the min
  * over incident tetrahedra of the reference's per-tet bound), and the Lorenzo
  * pass from log values L[3][n] and eb codes (255 = non-positive bound, else

@@ -71,3 +71,24 @@ def test_strip_of_four_gib(orc):
     assert np.array_equal(mask_2d_padding(s, r1, r2), mask_2d_padding(ref, r1, r2))
     got, want = cz.sz_decompress_cp_preserve_2d_offline(ref, r1, r2), orc.decompress_2d(ref, r1, r2)
     assert _same(got[0], want[0]) and _same(got[1], want[1])
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+def test_tiles_of_four_gib(orc, dtype):
+    """Rows a little under 4 GiB a strip, whose tiles are a little over: the last value of the third row lies past 4 GiB.
+    Zeros in every other column have it stored as it is."""
+    r1, r2 = 3, (1 << 32) // 64 // np.dtype(dtype).itemsize - 1
+    print(f"[wave2d] {np.dtype(dtype).name} {r1}x{r2}", flush=True)
+    rng = np.random.default_rng(1)
+    x = np.arange(r2, dtype=np.float32)
+    fields = []
+    for a, b in ((531, 713), (917, 389)):
+        f = np.stack([np.sin(x / a), np.cos(x / b), np.sin(x / b)]).astype(dtype) + dtype(1.5)
+        f[:, -60:] = rng.standard_normal((r1, 60))
+        f[:, -60::2] = 0
+        fields.append(f)
+    s = cz.sz_compress_cp_preserve_2d_offline(*fields, 0.1)
+    want = orc.decompress_2d(s, r1, r2, dtype)
+    assert all(w[2, -1] == f[2, -1] and w[2, -1] != 0 for w, f in zip(want, fields))
+    got = cz.sz_decompress_cp_preserve_2d_offline(s, r1, r2, dtype)
+    assert _same(got[0], want[0]) and _same(got[1], want[1])
