@@ -101,6 +101,7 @@ _SIGS = {
     "cpsz_set_exact_2d_bounds": [C.c_int],
     "cpsz_tri_bound_2d_fast_host": [_P, _SZ, C.c_int, _P],
     "cpsz_ratio_ge1_host": [_P, _P, _SZ, _P],
+    "cpsz_wave2d_boundary": [_P, _SZ, C.c_int, _P, _P, _P],
     "cpsz_wave2d_span": [_SZ, _SZ, C.c_int, C.POINTER(C.c_int), C.POINTER(C.c_uint64)],
 }
 
@@ -650,6 +651,15 @@ def wave2d_span(r1: int, r2: int, value_bytes: int):
     far, span = C.c_int(), C.c_uint64()
     _check(lib().cpsz_wave2d_span(r1, r2, value_bytes, C.byref(far), C.byref(span)))
     return bool(far.value), span.value
+
+
+def wave2d_boundary(x):
+    """The words by which strips of the 2D wavefront hand the values x to each other (for testing): (words, whether
+    each is taken as published, the values then read)."""
+    x = np.ascontiguousarray(x)
+    words, ready, read = np.zeros(x.size, np.uint64), np.zeros(x.size, np.uint8), np.empty_like(x)
+    _check(lib().cpsz_wave2d_boundary(_ptr(x), x.size, x.dtype.itemsize, _ptr(words), _ptr(ready), _ptr(read)))
+    return words, ready.astype(bool), read
 
 
 def tri_bound_2d_fast_host(uv6, ulps: int = 0):

@@ -799,6 +799,25 @@ int cpsz_wave2d_span(size_t r1, size_t r2, int value_bytes, int* far, uint64_t* 
   });
 }
 
+int cpsz_wave2d_boundary(const void* x, size_t n, int value_bytes, uint64_t* words, uint8_t* ready, void* read) {
+  return guarded([&] {
+    CPSZ_REQUIRE(x && words && ready && read && (value_bytes == 4 || value_bytes == 8), kErrArg, "bad arguments");
+    for (size_t k = 0; k < n; k++) {
+      if (value_bytes == 4) {
+        words[k] = bnd_word(((const float*)x)[k]);
+        ready[k] = bnd_ready(words[k], 0.f);
+        const float y = bnd_value(words[k], 0.f);
+        std::memcpy((float*)read + k, &y, 4);
+      } else {
+        words[k] = bnd_word(((const double*)x)[k]);
+        ready[k] = bnd_ready(words[k], 0.0);
+        const double y = bnd_value(words[k], 0.0);
+        std::memcpy((double*)read + k, &y, 8);
+      }
+    }
+  });
+}
+
 int cpsz_set_timing(int device, int on) {
   return guarded([&] { ctx_of(device).timing = on != 0; });
 }

@@ -37,8 +37,7 @@
 // issue slots of 16 waves bind.
 //
 // The row below a group travels through global memory value by value: each
-// 64-bit word carries a float with a tag (kBndTag), or a double replacing a
-// NaN pattern (kBndEmpty) that no reconstruction takes, so that the reader
+// 64-bit word is a published value or empty (bnd_word), so that the reader
 // needs no counter and the writer no wait for its stores. Groups are taken
 // from a ticket counter in dependency order: every wait targets an earlier
 // ticket, whose workgroup is resident or done.
@@ -58,8 +57,6 @@ constexpr int kPitch = 68;   // staged elements per step
 constexpr int kLag = 5;      // chunks between two strips: 63 steps + 1, rounded up, + 1 for the barrier
 constexpr int kAhead = 4;    // chunks between an input wave's loads and their use
 constexpr int kRing = 128;   // ring of a strip's last-row values (> kLag * kC + kC)
-constexpr uint64_t kBndTag = 1ull << 32;
-constexpr uint64_t kBndEmpty = 0x7FF4DEADBEEF0000ull;
 
 // Global address space: the pointers of a batch's table are generic, and flat
 // accesses would count with the LDS accesses that the barrier waits for.
@@ -72,12 +69,6 @@ __device__ __forceinline__ uint64_t ld_coh64(const GLB uint64_t* p) {
 __device__ __forceinline__ void st_coh64(GLB uint64_t* p, uint64_t v) {
   __hip_atomic_store((uint64_t*)p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
-__device__ __forceinline__ bool bnd_ready(uint64_t v, float) { return (v >> 32) != 0; }
-__device__ __forceinline__ bool bnd_ready(uint64_t v, double) { return v != kBndEmpty; }
-__device__ __forceinline__ uint64_t bnd_word(float x) { return kBndTag | l2d_bits(x); }
-__device__ __forceinline__ uint64_t bnd_word(double x) { return l2d_bits(x); }
-__device__ __forceinline__ float bnd_value(uint64_t v, float) { return l2d_float((uint32_t)v); }
-__device__ __forceinline__ double bnd_value(uint64_t v, double) { return l2d_double(v); }
 
 // lane l takes lane l - 1's src, lane 0 keeps lane0
 __device__ __forceinline__ float shr1(float src, float lane0) {

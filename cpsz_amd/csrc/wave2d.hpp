@@ -5,6 +5,7 @@
 
 #include "common.hpp"
 #include "ctx.hpp"
+#include "lorenzo2d_step.hpp"
 
 namespace cpsz {
 
@@ -101,6 +102,23 @@ inline int strip_groups(size_t r1) {
 inline bool far_strip(size_t r2, size_t value_bytes) {
   return div_up(r2 + 63, (size_t)kTileSteps) * (64 * kTileSteps) * value_bytes >= (1ull << 32);
 }
+// A word of a field's boundary rows: a float with a tag, or a double in place of
+// a NaN pattern (kBndEmpty). A corrupt stream's unpredictable values can hold
+// any pattern: that one is published as the NaN next to it, or the reader would
+// wait for it without end (the output keeps its own; what is predicted from
+// either is a NaN).
+constexpr uint64_t kBndTag = 1ull << 32;
+constexpr uint64_t kBndEmpty = 0x7FF4DEADBEEF0000ull;
+__host__ __device__ inline bool bnd_ready(uint64_t v, float) { return (v >> 32) != 0; }
+__host__ __device__ inline bool bnd_ready(uint64_t v, double) { return v != kBndEmpty; }
+__host__ __device__ inline uint64_t bnd_word(float x) { return kBndTag | l2d_bits(x); }
+__host__ __device__ inline uint64_t bnd_word(double x) {
+  const uint64_t b = l2d_bits(x);
+  return b == kBndEmpty ? b + 1 : b;
+}
+__host__ __device__ inline float bnd_value(uint64_t v, float) { return l2d_float((uint32_t)v); }
+__host__ __device__ inline double bnd_value(uint64_t v, double) { return l2d_double(v); }
+
 // 64-bit words of a field's boundary rows (enough for either type)
 inline size_t bnd_words(size_t r1, size_t r2) { return 2 * div_up(r1, (size_t)64 * kStrips64) * r2; }
 

@@ -248,6 +248,11 @@ int cpsz_lorenzo2d_emulate(const float* x, const uint16_t* c, size_t r1, size_t 
  * row-major arrays or in the codec's own, whichever is more. */
 int cpsz_wave2d_span(size_t r1, size_t r2, int value_bytes, int* far, uint64_t* span);
 
+/* The words by which strips of the 2D wavefront hand n values (of value_bytes
+ * each) to each other, whether the reader takes each as published, and what it
+ * then reads (for testing). */
+int cpsz_wave2d_boundary(const void* x, size_t n, int value_bytes, uint64_t* words, uint8_t* ready, void* read);
+
 /* Host emulations of the device 3D arithmetic: per-vertex bounds (the min
  * over incident tetrahedra of the reference's per-tet bound), and the Lorenzo
  * pass from log values L[3][n] and eb codes (255 = non-positive bound, else

@@ -1,4 +1,5 @@
-"""Host checks (no GPU) of the 2D wavefront's addressing."""
+"""Host checks (no GPU) of the 2D wavefront's addressing and of the words that its strips hand to each other."""
+import numpy as np
 import pytest
 
 import cpsz_amd as cz
@@ -22,3 +23,20 @@ def test_offsets_of_a_column(value_bytes):
     for r1 in [1, 1000, edge // 2, edge - 63, edge - 1, edge]:
         far, span = cz.wave2d_span(r1, 1, value_bytes)
         assert far or span <= (1 << 32) - 16
+
+
+@pytest.mark.parametrize("bits,value", [(np.uint32, np.float32), (np.uint64, np.float64)])
+def test_every_value_can_be_published(bits, value):
+    """Any pattern, as a corrupt stream can hold it, reads as published: numbers as they are, a NaN as a NaN."""
+    n = np.dtype(bits).itemsize * 8
+    rng = np.random.default_rng(3)
+    b = np.concatenate([rng.integers(0, (1 << n) - 1, 100000, dtype=bits, endpoint=True),
+                        np.array([0, 1 << (n - 1), (1 << n) - 1], bits)])
+    if n == 64:  # the NaNs around the pattern that stands for an empty word
+        empty = 0x7FF4DEADBEEF0000
+        b = np.concatenate([b, np.arange(empty - 3, empty + 4, dtype=np.uint64)])
+    x = b.view(value)
+    words, ready, read = cz.wave2d_boundary(x)
+    assert ready.all(), [hex(int(w)) for w in words[~ready]]
+    nan = np.isnan(x)
+    assert np.array_equal(read[~nan].view(bits), b[~nan]) and np.isnan(read[nan]).all()
