@@ -752,7 +752,6 @@ __device__ __forceinline__ void dec_write_block(const MDecJob& J, const Sink& si
   // (o0 and o1 are uniform; a lane's run may span two stages)
   for (uint32_t o0 = 0; o0 < limit; o0 += Stage::kCap) {
     const uint32_t o1 = min(limit, o0 + Stage::kCap);
-    S* const at = stage - o0;
     if (Sink::kBytes == 1) {
       // up to 6 codes per fetch while they all start before `end` and fit
       while (p < end && o < o1) {
@@ -763,7 +762,7 @@ __device__ __forceinline__ void dec_write_block(const MDecJob& J, const Sink& si
           const uint32_t m = md[win & kLutMask];
           const uint32_t len = m & 0xF, k = (m >> 4) & 3;
           if (!k || p + len > end || o + k > o1) break;
-          S* d = at + o;
+          S* d = stage + (o - o0);
           d[0] = (S)(m >> 8);
           if (k > 1) d[1] = (S)(m >> 16);
           if (k > 2) d[2] = (S)(m >> 24);
@@ -772,7 +771,7 @@ __device__ __forceinline__ void dec_write_block(const MDecJob& J, const Sink& si
           win >>= len;
           none = false;
         }
-        if (none) at[o++] = (S)dec_one(t, slut, bits, p);
+        if (none) stage[o++ - o0] = (S)dec_one(t, slut, bits, p);
       }
     } else {
       // up to 3 codes per fetch
@@ -780,24 +779,24 @@ __device__ __forceinline__ void dec_write_block(const MDecJob& J, const Sink& si
         const uint32_t win = bits.window(p);
         uint32_t e = slut[win & kLutMask];
         if (!short_code(e)) {
-          at[o++] = (S)long_code(t, bits, e, p);
+          stage[o++ - o0] = (S)long_code(t, bits, e, p);
           continue;
         }
         uint32_t used = e & 0xFF;
-        at[o++] = (S)(e >> 8);
+        stage[o++ - o0] = (S)(e >> 8);
         p += used;
 #pragma unroll
         for (int r = 0; r < 2; r++) {
           e = slut[(win >> used) & kLutMask];
           if (p >= end || o >= o1 || !short_code(e) || used > 32 - kLutBits) break;
-          at[o++] = (S)(e >> 8);
+          stage[o++ - o0] = (S)(e >> 8);
           used += e & 0xFF;
           p += e & 0xFF;
         }
       }
     }
     __syncthreads();
-    for (uint32_t x = o0 + threadIdx.x; x < o1; x += blockDim.x) out.put(first + x, at[x]);
+    for (uint32_t x = o0 + threadIdx.x; x < o1; x += blockDim.x) out.put(first + x, stage[x - o0]);
     __syncthreads();
   }
 }
