@@ -1055,7 +1055,11 @@ Eb3Grids send_eb3_jobs(Ctx& ctx, Eb3Job* jobs, int nf, Eb3Job*& d_jobs) {
     J.gy = (int)div_up(J.r2, kMJ);
     J.bx = std::min(256, (int)div_up(J.r3, 64) * 64);
     J.rows = 256 / J.bx;
-    J.fxn = (uint32_t)std::min<size_t>(div_up(J.n, 16384), 1024);
+    // a thread per vertex up to 1024 blocks: on noise most vertices are undecided,
+    // and each costs 24 exact tetrahedra (a block per 16384 vertices: 24^3 of noise
+    // compressed in 3.94 ms, 64^3 in 5.3, 128^3 in 6.7; here 0.60, 1.12 and 3.6;
+    // 256^3 and batches of smooth fields the same)
+    J.fxn = (uint32_t)std::min<size_t>(div_up(J.n, 256), 1024);
     J.sgn = (uint32_t)div_up(J.nq, 4 * kSignGroups);
     const size_t eb = tiles[k].first * div_up(J.r1, ms), lg = div_up((size_t)J.r1 * J.r2, (size_t)J.rows);
     CPSZ_REQUIRE(g.eb + eb < (1ull << 31) && g.lg + lg < (1ull << 31) && (size_t)g.sg + J.sgn < (1ull << 31),
