@@ -799,6 +799,14 @@ int cpsz_wave2d_span(size_t r1, size_t r2, int value_bytes, int* far, uint64_t* 
   });
 }
 
+int cpsz_scratch_bytes_2d(size_t r1, size_t r2, int value_bytes, uint64_t* compress, uint64_t* decompress) {
+  return guarded([&] {
+    CPSZ_REQUIRE(r1 && r2 && compress && decompress && (value_bytes == 4 || value_bytes == 8), kErrArg, "bad arguments");
+    *decompress = d2_scratch_bytes(r1, r2, value_bytes == 8);
+    *compress = c2_scratch_bytes(r1, r2);
+  });
+}
+
 int cpsz_wave2d_boundary(const void* x, size_t n, int value_bytes, uint64_t* words, uint8_t* ready, void* read) {
   return guarded([&] {
     CPSZ_REQUIRE(x && words && ready && read && (value_bytes == 4 || value_bytes == 8), kErrArg, "bad arguments");

@@ -2208,6 +2208,9 @@ void d2_unpred(Ctx& ctx, const uint8_t* d_in, const D2Plan& p, D2Work& w) {
 }  // namespace
 
 size_t d2_scratch_bytes(size_t r1, size_t r2, bool f64) {
+  // (the kernels' rows, columns and steps are ints)
+  CPSZ_REQUIRE(r1 < kMaxSide2d && r2 < kMaxSide2d && r1 * r2 < (1ull << 40), kErrUnsupported,
+               "decompress_2d: field too large");
   const size_t te = Tile2d(r1, r2).elems(r1);
   return 4 * al256(2 * te) + al256((f64 ? 16 : 8) * te) + al256(8 * bnd_words(r1, r2)) + al256(4) + al256(16);
 }

@@ -104,7 +104,8 @@ struct D2Work {
   bool f64 = false;
   double *dU64 = nullptr, *dV64 = nullptr;
 };
-size_t d2_scratch_bytes(size_t r1, size_t r2, bool f64 = false);
+constexpr size_t kMaxSide2d = (1ull << 31) - 1024;
+size_t d2_scratch_bytes(size_t r1, size_t r2, bool f64 = false);  // refuses fields beyond the kernels' range
 void d2_bind(D2Work& w, uint8_t* scratch);  // carves d2_scratch_bytes(r1, r2, w.f64)
 void d2_entropy(Ctx& ctx, const uint8_t* d_in, const uint8_t* h_in, size_t in_size, D2Work& w);
 // The entropy stage of many fields at once (headers and trees on `workers`

@@ -248,6 +248,9 @@ int cpsz_lorenzo2d_emulate(const float* x, const uint16_t* c, size_t r1, size_t 
  * row-major arrays or in the codec's own, whichever is more. */
 int cpsz_wave2d_span(size_t r1, size_t r2, int value_bytes, int* far, uint64_t* span);
 
+/* Device scratch of one 2D field's compression and decompression (for testing). */
+int cpsz_scratch_bytes_2d(size_t r1, size_t r2, int value_bytes, uint64_t* compress, uint64_t* decompress);
+
 /* The words by which strips of the 2D wavefront hand n values (of value_bytes
  * each) to each other, whether the reader takes each as published, and what it
  * then reads (for testing). */

@@ -40,3 +40,11 @@ def test_every_value_can_be_published(bits, value):
     assert ready.all(), [hex(int(w)) for w in words[~ready]]
     nan = np.isnan(x)
     assert np.array_equal(read[~nan].view(bits), b[~nan]) and np.isnan(read[nan]).all()
+
+
+@pytest.mark.parametrize("shape", [(1, 1 << 32), ((1 << 32) + 7, 1), (3, 1 << 31), (1 << 21, 1 << 21), ((1 << 31) - 1, 2)])
+def test_decompression_refuses_sides_beyond_its_range(shape):
+    """(Scratch sized from a side cut to 32 bits would be written past its end.)"""
+    for value_bytes in (4, 8):
+        with pytest.raises(cz.CpszError):
+            cz.scratch_bytes_2d(*shape, value_bytes)
