@@ -101,6 +101,7 @@ _SIGS = {
     "cpsz_set_exact_2d_bounds": [C.c_int],
     "cpsz_tri_bound_2d_fast_host": [_P, _SZ, C.c_int, _P],
     "cpsz_ratio_ge1_host": [_P, _P, _SZ, _P],
+    "cpsz_tile_index_2d": [_SZ, _SZ, _P, C.POINTER(C.c_uint64)],
     "cpsz_scratch_bytes_2d": [_SZ, _SZ, C.c_int, C.POINTER(C.c_uint64), C.POINTER(C.c_uint64)],
     "cpsz_wave2d_boundary": [_P, _SZ, C.c_int, _P, _P, _P],
     "cpsz_wave2d_span": [_SZ, _SZ, C.c_int, C.POINTER(C.c_int), C.POINTER(C.c_uint64)],
@@ -652,6 +653,13 @@ def wave2d_span(r1: int, r2: int, value_bytes: int):
     far, span = C.c_int(), C.c_uint64()
     _check(lib().cpsz_wave2d_span(r1, r2, value_bytes, C.byref(far), C.byref(span)))
     return bool(far.value), span.value
+
+
+def tile_index_2d(r1: int, r2: int):
+    """Where the 2D codec's own arrays keep each element of a field (r1 x r2 indexes), and such an array's elements."""
+    at, n = np.zeros((r1, r2), np.uint64), C.c_uint64()
+    _check(lib().cpsz_tile_index_2d(r1, r2, _ptr(at), C.byref(n)))
+    return at, n.value
 
 
 def scratch_bytes_2d(r1: int, r2: int, value_bytes: int = 4):

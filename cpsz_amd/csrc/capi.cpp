@@ -790,12 +790,23 @@ int cpsz_wave2d_span(size_t r1, size_t r2, int value_bytes, int* far, uint64_t* 
   return guarded([&] {
     CPSZ_REQUIRE(r1 && r2 && far && span && (value_bytes == 4 || value_bytes == 8), kErrArg, "bad arguments");
     const Tile2d t(r1, r2);
-    const size_t cols = t.row_len, rows = std::min<size_t>(t.column ? 1 : r1, 64);
-    // row l's columns are at steps l to l + cols - 1
-    const int last = (int)rows - 1;
-    const size_t tile = t.column ? t.at((int)cols - 1, 0) : t.at(last, (int)cols - 1);
+    const size_t cols = t.flip ? r1 : r2, rows = std::min<size_t>(t.flip ? r2 : r1, 64);
+    const size_t tile = t.flip ? t.at((int)cols - 1, (int)rows - 1) : t.at((int)rows - 1, (int)cols - 1);
     *far = far_strip(cols, value_bytes);
     *span = (std::max(rows * cols - 1, tile) + 1) * value_bytes;
+  });
+}
+
+int cpsz_tile_index_2d(size_t r1, size_t r2, uint64_t* at, uint64_t* elems) {
+  return guarded([&] {
+    CPSZ_REQUIRE(r1 && r2 && at && elems && r1 < kMaxSide2d && r2 < kMaxSide2d, kErrArg, "bad arguments");
+    const Tile2d t(r1, r2);
+    for (size_t i = 0; i < r1; i++)
+      for (size_t j = 0; j < r2; j++) {
+        at[i * r2 + j] = t.at((int)i, (int)j);
+        CPSZ_REQUIRE(at[i * r2 + j] == t.at_linear(i * r2 + j), kErrInternal, "tile index by element number");
+      }
+    *elems = t.elems();
   });
 }
 

@@ -537,6 +537,8 @@ struct SrcIds2d {
 // loads (3 a lane) and reads 18 codes a lane from there, in the blocks' order.
 // Row ii of the chunk lands one code later than row ii - 1 (the tiles are
 // skewed by a step a row), so row ii, column j is at first + ii (kPitch + 1) + j.
+// A flipped field's columns lie in the tiles as runs: a chunk, the whole of a block
+// row, takes the 24 codes from a multiple of 8 on that hold 12 rows of each.
 template <typename T>
 struct SrcCodes2dT {
   const uint16_t* q;  // tiles
@@ -549,13 +551,18 @@ struct SrcCodes2dT {
   const uint64_t* uoff = nullptr;
   T* unp = nullptr;
   static constexpr bool kUnpred = true;
+  bool flip;
   static constexpr int kBlocks = 8, kRun = 18, kPitch = 128, kSegs = 15, kLds = kBlock2d * kPitch;
+  static constexpr int kFlipPitch = 24, kFlipSegs = 3;
   static_assert(kBlocks * kBlock2d * kBlock2d == 64 * kRun && kSegs * 8 >= 7 + kBlock2d - 1 + kBlocks * kBlock2d);
+  static_assert(kFlipPitch >= 7 + kBlock2d && 64 * kFlipPitch <= kLds && 63 * kFlipSegs <= 3 * 64 && kBlocks * kBlock2d >= 63);
   // a one-column field is laid out, and has its codes in the order of, a one-row field
   SrcCodes2dT(const uint16_t* q_, const Tile2d& t_, size_t r1_, size_t r2_, const T* x_ = nullptr)
-      : q(q_), t(t_), r1((int)(t_.column ? 1 : r1_)), r2((int)(t_.column ? r1_ : r2_)),
-        nby((int)div_up((size_t)r2, (size_t)kBlock2d)), per((int)div_up((size_t)nby, (size_t)kBlocks)), x(x_) {}
+      : q(q_), t(t_), r1((int)(r2_ == 1 ? 1 : r1_)), r2((int)(r2_ == 1 ? r1_ : r2_)),
+        nby((int)div_up((size_t)r2, (size_t)kBlock2d)), per((int)div_up((size_t)nby, (size_t)kBlocks)), x(x_),
+        flip(t_.flip && r2_ > 1) {}
   size_t chunks() const { return div_up((size_t)r1, (size_t)kBlock2d) * per; }
+  __device__ bool flipped() const { return __builtin_amdgcn_readfirstlane((int)flip) != 0; }  // (a scalar branch)
   // first block of chunk c
   __device__ void first(size_t c, int& bi, int& bj) const {
     if (c < (1ull << 32)) {
@@ -570,19 +577,33 @@ struct SrcCodes2dT {
     int bi, bj;
     first(c, bi, bj);
     const uint32_t i0 = (uint32_t)bi * kBlock2d, sx = (uint32_t)min(kBlock2d, r1 - (int)i0);
-    const uint32_t t0 = ((uint32_t)bj * kBlock2d + (i0 & 63)) & ~7u;
     u32x4 v[3];
+    if (flipped()) {
+#pragma unroll
+      for (int k = 0; k < 3; k++) {
+        const uint32_t s = (threadIdx.x & 63) + 64 * k, col = s / kFlipSegs, seg = s % kFlipSegs;
+        const uint32_t step = ((i0 + col) & ~7u) + 8 * seg;
+        // (8 steps that hold none of the rows are not read)
+        const bool in = col < (uint32_t)r2 && step < i0 + sx + col;
+        v[k] = *glob(reinterpret_cast<const u32x4*>(q + t.at_step(0, in ? col : 0u, in ? step : 0u)));
+      }
+#pragma unroll
+      for (int k = 0; k < 3; k++) {
+        const uint32_t s = (threadIdx.x & 63) + 64 * k;
+        *reinterpret_cast<u32x4*>(lds + s / kFlipSegs * kFlipPitch + 8 * (s % kFlipSegs)) = v[k];
+      }
+      return;
+    }
+    const uint32_t t0 = ((uint32_t)bj * kBlock2d + (i0 & 63)) & ~7u;
 #pragma unroll
     for (int k = 0; k < 3; k++) {
       const uint32_t s = (threadIdx.x & 63) + 64 * k, row = s / kSegs, seg = s % kSegs;
       const uint32_t i = i0 + row, l = i & 63;
       // the step within the row's own strip (the next one's steps start over)
       const int step = (int)(t0 + 8 * seg) - (l < (i0 & 63) ? 64 : 0);
-      const bool in = row < sx && step >= 0 && step < (int)(t.nch * kTileSteps);
-      const uint32_t u = in ? (uint32_t)step : 0u;
-      const size_t at = ((size_t)(in ? i >> 6 : 0u) * t.nch + u / kTileSteps) * (64 * kTileSteps) +
-                        (in ? l : 0u) * kTileSteps + u % kTileSteps;
-      v[k] = *glob(reinterpret_cast<const u32x4*>(q + at));
+      // (8 steps that hold none of the row's columns are not read)
+      const bool in = row < sx && step >= 0 && step < r2 + (int)l;
+      v[k] = *glob(reinterpret_cast<const u32x4*>(q + t.at_step(in ? i >> 6 : 0u, in ? l : 0u, in ? (uint32_t)step : 0u)));
     }
 #pragma unroll
     for (int k = 0; k < 3; k++) {
@@ -610,7 +631,7 @@ struct SrcCodes2dT {
     int bi, bj, sx, b, ii, jj, w, last_w;
     first(c, bi, bj);
     const uint32_t rem = ((uint32_t)bj * kBlock2d + ((uint32_t)(bi * kBlock2d) & 63)) & 7u;
-    if (bi * kBlock2d + kBlock2d <= r1 && (bj + kBlocks) * kBlock2d <= r2) {
+    if (!flipped() && bi * kBlock2d + kBlock2d <= r1 && (bj + kBlocks) * kBlock2d <= r2) {
       // whole blocks: three half rows a lane, eight lanes a block
       const uint32_t lane = threadIdx.x & 63, s = lane & 7, odd = s & 1;
       const uint16_t* p = lds + rem + ((3 * s) >> 1) * (kPitch + 1) + (lane >> 3) * kBlock2d + 6 * odd;
@@ -624,19 +645,23 @@ struct SrcCodes2dT {
       return kRun;
     }
     const int left = place(c, bi, bj, sx, b, ii, jj, w, last_w);
+    auto walk = [&](auto at) {
 #pragma unroll
-    for (int k = 0; k < kRun; k++) {
-      const bool in = k < left;
-      sym[k] = lds[in ? (int)rem + ii * (kPitch + 1) + b * kBlock2d + jj : (int)rem];
-      if (++jj == w) {
-        jj = 0;
-        if (++ii == sx) {
-          ii = 0;
-          b++;
-          w = bj + b == nby - 1 ? last_w : kBlock2d;
+      for (int k = 0; k < kRun; k++) {
+        const bool in = k < left;
+        sym[k] = lds[in ? at(ii, b * kBlock2d + jj) : (int)rem];
+        if (++jj == w) {
+          jj = 0;
+          if (++ii == sx) {
+            ii = 0;
+            b++;
+            w = bj + b == nby - 1 ? last_w : kBlock2d;
+          }
         }
       }
-    }
+    };
+    if (flipped()) walk([&](int i, int col) { return col * kFlipPitch + ((bi * kBlock2d + col) & 7) + i; });
+    else walk([&](int i, int col) { return (int)rem + i * (kPitch + 1) + col; });
     return max(0, min(kRun, left));
   }
   __device__ size_t elem(size_t c, int k) const {
@@ -703,7 +728,7 @@ struct SinkCodes2d {
       // division is some 30 instructions, of 32 bits): p / (12 r2) is
       // (p / 12) / r2
       const uint32_t p32 = (uint32_t)p, rb = (uint32_t)rowblk;
-      const uint32_t b = t.column ? p32 / kBlock2d : t.rows_in(p32 / kBlock2d), rem = p32 - b * rb;
+      const uint32_t b = t.rows_in(p32 / kBlock2d), rem = p32 - b * rb;
       bi = (int)b;
       const uint32_t sx = (uint32_t)min(kBlock2d, r1 - bi * kBlock2d);
       bj = min((int)(sx == kBlock2d ? rem / (kBlock2d * kBlock2d) : rem / (sx * kBlock2d)), nby - 1);
@@ -852,7 +877,7 @@ __global__ void __launch_bounds__(256) k_finish2d(float* __restrict__ U, float* 
 // count of code 0 leaves the pads out.
 struct U16Hist {
   const uint16_t* p;  // 8-byte aligned (the code arrays are 256-byte aligned)
-  size_t n;           // a multiple of 1024
+  size_t n;
   uint32_t pads;
   static constexpr int kChunk = 1024;
   // four codes per item, one 8-byte load
@@ -866,6 +891,7 @@ struct U16Hist {
     return 4;
   }
   static constexpr bool kPads = true;  // code-0 pads, counted out of bin 0
+  __device__ uint32_t at(size_t i) const { return p[i]; }
 };
 
 // ---- batched entropy stage: many fields' streams per launch -----------------
@@ -1332,13 +1358,13 @@ size_t al256(size_t x) { return (x + 255) & ~(size_t)255; }
 
 // ------------------------------------------------------------- staged form --
 size_t c2_scratch_bytes(size_t r1, size_t r2) {
-  const size_t n = r1 * r2, te = Tile2d(r1, r2).elems(r1);
+  const size_t n = r1 * r2, te = Tile2d(r1, r2).elems();
   return 2 * al256(2 * n) + 4 * al256(2 * te) + al256((kMaxEbCode + 2 * 65536) * 4) + al256(16) + al256(8 * bnd_words(r1, r2)) + al256(4);
 }
 
 void c2_bind(C2Work& w, uint8_t* p) {
   w.t = Tile2d(w.r1, w.r2);
-  const size_t n = w.r1 * w.r2, te = w.t.elems(w.r1);
+  const size_t n = w.r1 * w.r2, te = w.t.elems();
   auto take = [&](size_t bytes) {
     uint8_t* q = p;
     p += al256(bytes);
@@ -1497,6 +1523,7 @@ void c2_wavefront(Ctx& ctx, C2Work* const* w, size_t nf, int grid_cap) {
     sa.r1 = (int)w[0]->r1;
     sa.r2 = (int)w[0]->r2;
     sa.ngroups = strip_groups<double>(w[0]->r1);
+    sa.t = w[0]->t;
     sa.shift = 2;
     wavefront2d_compress64(ctx, sa, grid_cap);
     return;
@@ -1520,6 +1547,7 @@ void c2_wavefront(Ctx& ctx, C2Work* const* w, size_t nf, int grid_cap) {
     sa.ticket = w[k]->ticket;
     sa.r1 = (int)w[k]->r1;
     sa.r2 = (int)w[k]->r2;
+    sa.t = w[k]->t;
     sa.wide = w[k]->wide;
     sa.flags = w[k]->flags_on_device ? w[k]->flags : nullptr;
     CPSZ_REQUIRE(!(lg && (sa.wide || sa.flags)), kErrInternal, "compress_2d_log: eb id beyond the base-2 range");
@@ -1539,10 +1567,10 @@ void c2_entropy_of(Ctx& ctx, const C2Work& w, DeviceStream& out) {
   // ---- histograms of the quant codes
   {
     const uint32_t win_lo = 32768 - 8192, win_n = 16384;
-    const size_t te = w.t.elems(r1);
+    const size_t te = w.t.elems();
     U16Hist hu{qu, te, (uint32_t)(te - n)}, hv{qv, te, (uint32_t)(te - n)};
     const size_t nch = te / U16Hist::kChunk;
-    const int grid = (int)std::min<size_t>(encode_blocks(nch), 512);
+    const int grid = (int)std::min<size_t>(std::max<size_t>(encode_blocks(nch), 1), 512);
     k_hist<<<grid, 256, win_n * 4, st>>>(hu, nch, hist + kMaxEbCode, win_lo, win_n);
     k_hist<<<grid, 256, win_n * 4, st>>>(hv, nch, hist + kMaxEbCode + 65536, win_lo, win_n);
     CPSZ_HIP(hipGetLastError());
@@ -1796,14 +1824,14 @@ void c2_entropy_batch(Ctx& ctx, C2Work* const* w, size_t nf, uint8_t* dout, cons
   for (size_t k = 0; k < nf; k++) {
     const C2Work& W = *w[k];
     const G& x = g[k];
-    const size_t te = W.t.elems(W.r1), nch = te / U16Hist::kChunk;
+    const size_t te = W.t.elems(), nch = te / U16Hist::kChunk;
     for (int c = 0; c < 2; c++) {
       HistJob<U16Hist>& h = hj[2 * k + c];
       h.src = U16Hist{c ? W.qv : W.qu, te, (uint32_t)(te - x.n)};
       h.nchunks = nch;
       h.hist = W.hist + kMaxEbCode + c * 65536;
       // 128 chunks per block: a block clears and flushes its 16384-bin window once per 131072 codes
-      h.nblk = (uint32_t)std::min<size_t>(div_up(nch, 128), 512);
+      h.nblk = (uint32_t)std::min<size_t>(std::max<size_t>(div_up(nch, 128), 1), 512);
       h.blk0 = hblk;
       hblk += h.nblk;
     }
@@ -2196,11 +2224,11 @@ void d2_unpred(Ctx& ctx, const uint8_t* d_in, const D2Plan& p, D2Work& w) {
     if (w.f64)
       k_scatter_unpred<double><<<unp_grid(nb), 256, 0, st>>>(qs[c], w.t, (const double*)vals, (int)r1, (int)r2, p.nby,
                                                              nb, zoff + c * (nb + 1), p.comp[c].unp_count,
-                                                             (double*)w.raw + c * w.t.elems(r1), w.err);
+                                                             (double*)w.raw + c * w.t.elems(), w.err);
     else
       k_scatter_unpred<float><<<unp_grid(nb), 256, 0, st>>>(qs[c], w.t, (const float*)vals, (int)r1, (int)r2, p.nby, nb,
                                                             zoff + c * (nb + 1), p.comp[c].unp_count,
-                                                            w.raw + c * w.t.elems(r1), w.err);
+                                                            w.raw + c * w.t.elems(), w.err);
     CPSZ_HIP(hipGetLastError());
   }
 }
@@ -2211,13 +2239,13 @@ size_t d2_scratch_bytes(size_t r1, size_t r2, bool f64) {
   // (the kernels' rows, columns and steps are ints)
   CPSZ_REQUIRE(r1 < kMaxSide2d && r2 < kMaxSide2d && r1 * r2 < (1ull << 40), kErrUnsupported,
                "decompress_2d: field too large");
-  const size_t te = Tile2d(r1, r2).elems(r1);
+  const size_t te = Tile2d(r1, r2).elems();
   return 4 * al256(2 * te) + al256((f64 ? 16 : 8) * te) + al256(8 * bnd_words(r1, r2)) + al256(4) + al256(16);
 }
 
 void d2_bind(D2Work& w, uint8_t* p) {
   w.t = Tile2d(w.r1, w.r2);
-  const size_t te = w.t.elems(w.r1);
+  const size_t te = w.t.elems();
   auto take = [&](size_t bytes) {
     uint8_t* q = p;
     p += al256(bytes);
@@ -2345,7 +2373,7 @@ void d2_unpred_batch(Ctx& ctx, const std::vector<const uint8_t*>& d_in, const st
       u.nby = p.nby;
       u.nb = p.nb;
       u.off = zoff + zb[k] + c * p.nb;
-      u.out = W.raw + c * W.t.elems(W.r1);
+      u.out = W.raw + c * W.t.elems();
       u.count = p.comp[c].unp_count;
       u.err = W.err;
       u.blk0 = blk;
@@ -2546,7 +2574,7 @@ void d2_entropy_batch(Ctx& ctx, const std::vector<const uint8_t*>& d_in, const s
 
 void d2_wavefront(Ctx& ctx, D2Work* const* w, size_t nf, int grid_cap) {
   if (nf == 1 && w[0]->f64) {
-    const size_t n = w[0]->t.elems(w[0]->r1);
+    const size_t n = w[0]->t.elems();
     Strip2d64 sa{};
     sa.c[0] = w[0]->sid_u;
     sa.c[1] = w[0]->sid_v;
@@ -2561,6 +2589,7 @@ void d2_wavefront(Ctx& ctx, D2Work* const* w, size_t nf, int grid_cap) {
     sa.r1 = (int)w[0]->r1;
     sa.r2 = (int)w[0]->r2;
     sa.ngroups = strip_groups<double>(w[0]->r1);
+    sa.t = w[0]->t;
     sa.shift = 2;
     wavefront2d_decompress64(ctx, sa, grid_cap);
     return;
@@ -2571,7 +2600,7 @@ void d2_wavefront(Ctx& ctx, D2Work* const* w, size_t nf, int grid_cap) {
   for (size_t k = 0; k < nf; k++) {
     Strip2d& sa = f[k];
     sa = Strip2d{};
-    const size_t n = w[k]->t.elems(w[k]->r1);
+    const size_t n = w[k]->t.elems();
     sa.c[0] = w[k]->sid_u;
     sa.c[1] = w[k]->log ? w[k]->sid_u : w[k]->sid_v;
     sa.shift = w[k]->log ? 1 : 2;
@@ -2586,6 +2615,7 @@ void d2_wavefront(Ctx& ctx, D2Work* const* w, size_t nf, int grid_cap) {
     sa.ticket = w[k]->ticket;
     sa.r1 = (int)w[k]->r1;
     sa.r2 = (int)w[k]->r2;
+    sa.t = w[k]->t;
     sa.wide = w[k]->wide;
     CPSZ_REQUIRE(!(w[k]->log && sa.wide), kErrStream, "decompress_2d_log: eb id beyond the base-2 range");
   }

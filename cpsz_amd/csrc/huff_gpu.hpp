@@ -136,8 +136,9 @@ struct EncJob {
   uint32_t* zc;          // optional: per-chunk symbol-0 counts (with the bits), for the offsets of gathered values
 };
 
-// A source whose symbols include `pads` extra symbols 0 (kPads), which the
-// histogram does not count.
+// A source whose n symbols include `pads` extra symbols 0 (kPads), which the
+// histogram does not count. (Those past the last whole chunk, fewer than one, are
+// counted one by one.)
 template <class S, class = void>
 struct HasPads : std::false_type {};
 template <class S>
@@ -178,7 +179,10 @@ __device__ __forceinline__ void hist_block(const Src& src, size_t nchunks, uint3
   for (int o = 32; o > 0; o >>= 1) zeros += __shfl_xor(zeros, o);
   if (lane == 0 && zeros) atomicAdd(&hist[0], zeros);
   if constexpr (HasPads<Src>::value) {
-    if (blk == 0 && threadIdx.x == 0) atomicSub(&hist[0], src.pads);
+    if (blk == 0) {
+      if (threadIdx.x == 0) atomicSub(&hist[0], src.pads);
+      for (size_t i = nchunks * Src::kChunk + threadIdx.x; i < src.n; i += blockDim.x) atomicAdd(&hist[src.at(i)], 1u);
+    }
   }
   __syncthreads();
   // blocks start their flush at different bins so that their global atomics

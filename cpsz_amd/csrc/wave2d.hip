@@ -13,8 +13,8 @@
 // between them through LDS. Its waves are specialised:
 //   S recurrence waves   one per strip: the prediction and what depends on it,
 //                        nothing else. Each step reads one staged element from
-//                        LDS and writes one result (compress ~20, decompress
-//                        ~8 instructions a step).
+//                        LDS and writes one result (compress 17 vector
+//                        instructions a step and 22 in all, decompress 6 and 9).
 //   2S input waves       two per strip: load a chunk's tile of codes and its
 //                        values (16 columns of 4 rows per instruction), prepare
 //                        what depends on the element alone, and stage it in
@@ -31,10 +31,11 @@
 // 21 bytes. Measured on 96 uneven fields (220M vertices) with one wave per
 // strip doing everything / specialised waves / and tiles: compress 3.96 / 2.72
 // / 1.47 ms, decompress 5.55 / 2.90 / 2.18 ms; one 2400x3600 field 1.57 / 0.94
-// / 0.62 and 2.39 / 0.83 / 0.64 ms. One strip alone takes 0.6 us a chunk
-// (decompress, its recurrence 1220 cycles of 1440) to 0.9 us (compress, 2100 of
-// 2270); four on one CU 1.4 us, where the values' row-major accesses and the
-// issue slots of 16 waves bind.
+// / 0.62 and 2.39 / 0.83 / 0.64 ms. (Compress is at 1.35 and 0.55 since no copy
+// of the field's descriptor is in scratch memory, see group_item.) One strip alone
+// takes 0.56 us a chunk (decompress) to 0.86 us (compress), where the recurrence
+// binds; four on one CU 1.4 us, where the values' row-major accesses and the issue
+// slots of 16 waves bind.
 //
 // The row below a group travels through global memory value by value: each
 // 64-bit word is a published value or empty (bnd_word), so that the reader
@@ -164,15 +165,19 @@ struct Part<V, true> {
 
 // One item: S consecutive strips of one component (group g). `wave` is
 // uniform: 0..S-1 recurrence, S..3S-1 input, 3S..4S-1 output. FAR: a strip
-// spans 4 GiB or more (64-bit offsets within it).
-template <typename T, int S, bool COMPRESS, bool FAR>
-__device__ __forceinline__ void group_item(const Strip2dT<T>& a, bool wide, int comp, int g, int wave, int lane,
+// spans 4 GiB or more (64-bit offsets within it). FLIP: the field may be flipped
+// (in decompression, masking the rows that such a field lacks costs a single
+// strip 10%: 0.54 against 0.60 ms for 64 rows of 15627). The field's descriptor is read
+// by scalar loads where a role needs it: members held since the kernel's beginning
+// would spill, and a copy to choose the component from would be in scratch memory.
+template <typename T, int S, bool COMPRESS, bool FAR, bool FLIP>
+__device__ __forceinline__ void group_item(const CST Strip2dT<T>& a, bool wide, int comp, int g, int wave, int lane,
                                            WaveLds<T, S, COMPRESS>& sh) {
   constexpr bool kMayWide = sizeof(T) == 4;  // double fields have one step for all ids
   const int r1 = a.r1, r2 = a.r2;
   const int nstrips = (r1 + 63) >> 6;
   const int ns = min(S, nstrips - g * S);        // strips of this group
-  const int nch = (r2 + 63 + kC - 1) / kC;       // chunks of a strip
+  const int nch = a.t.nch;                       // chunks of a strip
   // strip w computes chunk e - 1 in iteration it = e + kLag w: its input waves
   // stage chunk e, its output wave stores chunk e - 2 (iterations rounded up
   // to the input waves' rotation of kAhead sets)
@@ -275,21 +280,24 @@ __device__ __forceinline__ void group_item(const Strip2dT<T>& a, bool wide, int 
     using Off = typename std::conditional<FAR, size_t, uint32_t>::type;
     // The code arrays are tiles: chunk c of the strip is one contiguous piece,
     // and a lane takes 8 consecutive steps (from k8) of row lt of it.
+    const int rows_log = a.t.rows_log, tile_log = rows_log + 4;
+    const size_t strip_at = (size_t)(g * S + w) * nch << tile_log;
+    // The row-major arrays: row l, column t - l is at l * ls + t * cs
+    const int cs = FLIP ? a.cs : 1, ls = cs == 1 ? r2 - 1 : 1 - cs;
     const int lt = 32 * half + (lane >> 1), k8 = 8 * (lane & 1);
-    const size_t strip_at = (size_t)(g * S + w) * nch * (64 * kC);
-    const uint32_t lane_at = (uint32_t)(lt * kC + k8);
-    const GLB uint16_t* C = (const GLB uint16_t*)(comp ? a.c[1] : a.c[0]) + strip_at;
-    const GLB uint16_t* Q = (const GLB uint16_t*)(comp ? a.q[1] : a.q[0]) + strip_at;
+    const uint32_t lane_at = (uint32_t)(min(lt, (1 << rows_log) - 1) * kC + k8);  // (rows past a short tile's last: any)
+    const GLB uint16_t* C = (const GLB uint16_t*)a.c[comp] + strip_at;
+    const GLB uint16_t* Q = (const GLB uint16_t*)a.q[comp] + strip_at;
     // The values of a compression are row-major: 16 columns of 4 rows per
     // instruction; chunk c, group i: row lx + 4 i, column c kC + kx - row.
     // (one element per lane: a load of two floats costs three times a load of
     // one here, and at 2-byte alignment a load of two codes four times)
     const int kx = lane & 15, lx = 32 * half + (lane >> 4);
     const size_t first = (size_t)row0 * r2;
-    const Part<T, FAR> X((COMPRESS ? (comp ? a.x[1] : a.x[0]) + first : (comp ? a.raw[1] : a.raw[0]) + strip_at),
-                         COMPRESS ? (size_t)r1 * r2 - first : (size_t)nch * (64 * kC));
-    Off lane0 = (Off)lx * (Off)(r2 - 1) + kx;
-    const Off istep = 4 * (Off)(r2 - 1);
+    const Part<T, FAR> X(COMPRESS ? a.x[comp] + first : a.raw[comp] + strip_at,
+                         COMPRESS ? (size_t)r1 * r2 - first : (size_t)nch << tile_log);
+    Off lane0 = (Off)lx * (Off)ls + (Off)kx * (Off)cs;
+    const Off istep = 4 * (Off)ls, cstep = kC * (Off)cs;
     int lane_col = kx - lx;
     // What a wave holds of a chunk on its way from memory to LDS: eb codes
     // and values, or stream ids, quantization codes and unpredictable values.
@@ -315,7 +323,7 @@ __device__ __forceinline__ void group_item(const Strip2dT<T>& a, bool wide, int 
     const bool row_in = row0 + lt < r1;
     auto inside = [&](int c, int m) { return row_in && (uint32_t)(c * kC + k8 + m - lt) < (uint32_t)r2; };
     auto load = [&](int c, Values& x, Codes& s) {
-      const size_t at = (size_t)min(max(c, 0), nch - 1) * (64 * kC);
+      const size_t at = (size_t)min(max(c, 0), nch - 1) << tile_log;
       ld16(C + at + lane_at, s.c);
       if constexpr (!COMPRESS) {
         ld16(Q + at + lane_at, s.q);
@@ -324,13 +332,13 @@ __device__ __forceinline__ void group_item(const Strip2dT<T>& a, bool wide, int 
         // before the first and after the last one are outside the row)
 #pragma unroll
         for (int i = 0; i < 8; i++)
-          x.v[i] = X.load(lane0 + ((Off)c * kC + i * istep), (uint32_t)(lane_col + (c * kC - 4 * i)) < (uint32_t)r2);
+          x.v[i] = X.load(lane0 + ((Off)c * cstep + i * istep), (uint32_t)(lane_col + (c * kC - 4 * i)) < (uint32_t)r2);
       }
     };
     // decompress: the unpredictable values, where the code is 0
     auto load_raw = [&](int c, Values& x, const Codes& s) {
       if constexpr (!COMPRESS) {
-        const Off at = (Off)min(max(c, 0), nch - 1) * (64 * kC) + lane_at;
+        const Off at = ((Off)min(max(c, 0), nch - 1) << tile_log) + lane_at;
 #pragma unroll
         for (int m = 0; m < 8; m++) x.v[m] = X.load(at + m, nth(s.q, m) == 0);
       }
@@ -414,15 +422,19 @@ __device__ __forceinline__ void group_item(const Strip2dT<T>& a, bool wide, int 
   } else {
     const bool publish = w == S - 1 && g + 1 < a.ngroups;
     GLB uint64_t* bout = (GLB uint64_t*)a.bnd + ((size_t)comp * a.ngroups + g) * r2;
-    // compress: the chunk's codes are one tile, 8 steps of a row per lane;
+    // compress: the chunk's codes are one tile, 8 steps of a row per lane and half;
     // decompress: values, 16 columns of 4 rows per instruction
     const int lt = lane >> 1, k8 = 8 * (lane & 1);
-    GLB uint16_t* Q = (GLB uint16_t*)(comp ? a.q[1] : a.q[0]) + (size_t)(g * S + w) * nch * (64 * kC);
+    const int tile_log = a.t.rows_log + 4, tile_rows = 1 << a.t.rows_log;
+    GLB uint16_t* Q = (GLB uint16_t*)a.q[comp] + ((size_t)(g * S + w) * nch << tile_log);
     const int k = lane & 15, rs = lane >> 4;
     using Off = typename std::conditional<FAR, size_t, uint32_t>::type;
     const size_t first = (size_t)row0 * r2;
-    const Part<T, FAR> O((comp ? a.out[1] : a.out[0]) + first, (size_t)r1 * r2 - first);
-    const Off lane0 = (Off)rs * (Off)(r2 - 1) + k, istep = 4 * (Off)(r2 - 1);
+    const Part<T, FAR> O(a.out[comp] + first, (size_t)r1 * r2 - first);
+    const int cs = FLIP ? a.cs : 1, ls = cs == 1 ? r2 - 1 : 1 - cs;
+    const Off lane0 = (Off)rs * (Off)ls + (Off)k * (Off)cs, istep = 4 * (Off)ls, cstep = kC * (Off)cs;
+    // (row-major, a row past the field's last lies past the array's end)
+    const int rows = cs == 1 ? 64 : r1;
     for (int it = -kAhead; it < it_end; it++) {
       const int c = it + e0 - 2;
       if (c >= 0 && c < nch) {
@@ -443,14 +455,16 @@ __device__ __forceinline__ void group_item(const Strip2dT<T>& a, bool wide, int 
 #pragma unroll
             for (int m = 0; m < 4; m++)
               p[m] = l2d_code(v[8 * h + 2 * m]) | (uint32_t)l2d_code(v[8 * h + 2 * m + 1]) << 16;
-            *(GLB u32x4*)(Q + ((size_t)c * (64 * kC) + (lt + 32 * h) * kC + k8)) = p;
+            const int l = lt + 32 * h;
+            if (l < tile_rows) *(GLB u32x4*)(Q + (((size_t)c << tile_log) + l * kC + k8)) = p;
           }
         } else {
 #pragma unroll
           for (int i = 0; i < 16; i++) v[i] = out[k][4 * i + rs];
 #pragma unroll
           for (int i = 0; i < 16; i++)
-            O.store(lane0 + ((Off)c * kC + i * istep), (uint32_t)(c * kC + k - rs - 4 * i) < (uint32_t)r2, v[i]);
+            O.store(lane0 + ((Off)c * cstep + i * istep),
+                    (!FLIP || rs + 4 * i < rows) && (uint32_t)(c * kC + k - rs - 4 * i) < (uint32_t)r2, v[i]);
         }
       }
       lds_barrier();
@@ -464,14 +478,14 @@ __device__ __forceinline__ void group_item(const Strip2dT<T>& a, bool wide, int 
 // field and taken from one ticket counter.
 template <typename T>
 struct StripBatch {
-  Strip2dT<T> one;
+  Strip2dT<T> one;  // (first: the kernel finds it at the beginning of its arguments)
   const Strip2dT<T>* f;  // null: the single field `one`
   const int* start;
   int nf, items;
   int* ticket;
 };
 
-template <typename T, int S, bool COMPRESS, bool FAR>
+template <typename T, int S, bool COMPRESS, bool FAR, bool FLIP>
 __global__ void __launch_bounds__(256 * S) k_wave2d(StripBatch<T> b) {
   __shared__ WaveLds<T, S, COMPRESS> sh;
   __shared__ int s_item;
@@ -494,38 +508,21 @@ __global__ void __launch_bounds__(256 * S) k_wave2d(StripBatch<T> b) {
       }
       at = item - ((const CST int*)b.start)[lo];
     }
-    Strip2dT<T> a = b.one;
-    if (b.f) {
-      // the table is not written while the kernel runs: scalar loads
-      const CST Strip2dT<T>* f = (const CST Strip2dT<T>*)b.f + lo;
-#pragma unroll
-      for (int k = 0; k < 2; k++) {
-        a.x[k] = f->x[k];
-        a.c[k] = f->c[k];
-        a.q[k] = f->q[k];
-        a.raw[k] = f->raw[k];
-        a.out[k] = f->out[k];
-      }
-      a.bnd = f->bnd;
-      a.r1 = f->r1;
-      a.r2 = f->r2;
-      a.ngroups = f->ngroups;
-      a.wide = f->wide;
-      a.shift = f->shift;
-      a.flags = f->flags;
+    // (constant address space: neither is written while the kernel runs)
+    const CST Strip2dT<T>* const f = b.f ? (const CST Strip2dT<T>*)b.f + lo
+                                         : (const CST Strip2dT<T>*)__builtin_amdgcn_kernarg_segment_ptr();  // b.one
+    bool skip = false, wide = f->wide;
+    if (f->flags) {
+      skip = __builtin_amdgcn_readfirstlane(f->flags[0]) != 0;  // every item of the field skips: no group waits on another
+      wide = __builtin_amdgcn_readfirstlane(f->flags[1]) != 0;
     }
-    bool skip = false, wide = a.wide;
-    if (a.flags) {
-      skip = __builtin_amdgcn_readfirstlane(a.flags[0]) != 0;  // every item of the field skips: no group waits on another
-      wide = __builtin_amdgcn_readfirstlane(a.flags[1]) != 0;
-    }
-    if (!skip) group_item<T, S, COMPRESS, FAR>(a, wide, at & 1, at >> 1, wave, lane, sh);
+    if (!skip) group_item<T, S, COMPRESS, FAR, FLIP>(*f, wide, at & 1, at >> 1, wave, lane, sh);
     __syncthreads();
   }
 }
 
 // 64-bit words of a field's published rows: none when one group carries all
-// its rows (which is so for a field of one column, whatever room it has).
+// its rows (which is so for every flipped field).
 template <typename T>
 __host__ __device__ size_t published_words(const Strip2dT<T>& f) {
   return f.ngroups > 1 ? (size_t)2 * f.ngroups * f.r2 : 0;
@@ -543,20 +540,31 @@ __global__ void __launch_bounds__(256) k_wave2d_clear(StripBatch<T> b) {
   if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) *b.ticket = 0;
 }
 
-// A field of one column is the same chain as a field of one row (each value's
-// prediction is its one neighbour), and its tiles are laid out as one.
+// The kernel's rows and columns: a flipped field's are exchanged, one strip.
 template <typename T>
-void as_row(Strip2dT<T>& f) {
-  if (f.r2 != 1) return;
-  f.r2 = f.r1;
-  f.r1 = 1;
+void orient(Strip2dT<T>& f) {
+  f.cs = 1;
+  if (!f.t.flip) return;
+  f.cs = f.r2;
+  std::swap(f.r1, f.r2);
   f.ngroups = 1;
+}
+
+// The kernel for the fields of one launch: the plainest that takes them all
+// (compression and 64-bit offsets always take flipped fields).
+template <typename T, int S, bool COMPRESS>
+void launch_wave(Ctx& ctx, const StripBatch<T>& b, int grid_cap, bool far, bool flip) {
+  const int grid = std::min(b.items, grid_cap);
+  if (far) k_wave2d<T, S, COMPRESS, true, true><<<grid, 256 * S, 0, ctx.stream()>>>(b);
+  else if (COMPRESS || flip) k_wave2d<T, S, COMPRESS, false, true><<<grid, 256 * S, 0, ctx.stream()>>>(b);
+  else k_wave2d<T, S, COMPRESS, false, COMPRESS><<<grid, 256 * S, 0, ctx.stream()>>>(b);
+  CPSZ_HIP(hipGetLastError());
 }
 
 template <typename T, int S, bool COMPRESS>
 void launch_one(Ctx& ctx, Strip2dT<T> f, int grid_cap) {
   hipStream_t st = ctx.stream();
-  as_row(f);
+  orient(f);
   StripBatch<T> b{};
   b.one = f;
   b.nf = 1;
@@ -564,10 +572,7 @@ void launch_one(Ctx& ctx, Strip2dT<T> f, int grid_cap) {
   b.ticket = f.ticket;
   const size_t words = published_words(f);
   k_wave2d_clear<T><<<(unsigned)std::min<size_t>(div_up(words, 256) + 1, 1024), 256, 0, st>>>(b);
-  const int grid = std::min(b.items, grid_cap);
-  if (far_strip(f.r2, sizeof(T))) k_wave2d<T, S, COMPRESS, true><<<grid, 256 * S, 0, st>>>(b);
-  else k_wave2d<T, S, COMPRESS, false><<<grid, 256 * S, 0, st>>>(b);
-  CPSZ_HIP(hipGetLastError());
+  launch_wave<T, S, COMPRESS>(ctx, b, grid_cap, far_strip(f.r2, sizeof(T)), f.t.flip);
 }
 
 template <bool COMPRESS>
@@ -583,7 +588,7 @@ void launch_many(Ctx& ctx, std::vector<Strip2d>& f, int grid_cap) {
   const size_t nf = f.size();
   CPSZ_REQUIRE(nf <= 65535, kErrUnsupported, "2D batch: at most 65535 fields per call");
   std::vector<Strip2d> g(f);
-  for (Strip2d& x : g) as_row(x);
+  for (Strip2d& x : g) orient(x);
   auto steps = [](const Strip2d& a) { return (int64_t)div_up((size_t)a.r1, (size_t)64) * kLag * kC + a.r2; };
   std::stable_sort(g.begin(), g.end(), [&](const Strip2d& a, const Strip2d& b) { return steps(a) > steps(b); });
   std::vector<int> start(nf + 1, 0);
@@ -605,12 +610,9 @@ void launch_many(Ctx& ctx, std::vector<Strip2d>& f, int grid_cap) {
   b.items = start[nf];
   b.ticket = (int*)(d + ((tbytes + sbytes + 15) & ~(size_t)15));
   k_wave2d_clear<float><<<dim3((unsigned)std::min<size_t>(div_up(max_words, 256 * 8) + 1, 64), (unsigned)nf), 256, 0, st>>>(b);
-  const int grid = std::min(b.items, grid_cap);
-  if (std::any_of(g.begin(), g.end(), [](const Strip2d& x) { return far_strip(x.r2, sizeof(float)); }))
-    k_wave2d<float, kStrips, COMPRESS, true><<<grid, 256 * kStrips, 0, st>>>(b);
-  else
-    k_wave2d<float, kStrips, COMPRESS, false><<<grid, 256 * kStrips, 0, st>>>(b);
-  CPSZ_HIP(hipGetLastError());
+  launch_wave<float, kStrips, COMPRESS>(
+      ctx, b, grid_cap, std::any_of(g.begin(), g.end(), [](const Strip2d& x) { return far_strip(x.r2, sizeof(float)); }),
+      std::any_of(g.begin(), g.end(), [](const Strip2d& x) { return x.t.flip; }));
 }
 
 }  // namespace

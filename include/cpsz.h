@@ -248,6 +248,9 @@ int cpsz_lorenzo2d_emulate(const float* x, const uint16_t* c, size_t r1, size_t 
  * row-major arrays or in the codec's own, whichever is more. */
 int cpsz_wave2d_span(size_t r1, size_t r2, int value_bytes, int* far, uint64_t* span);
 
+/* Where the 2D codec's own arrays keep the r1 * r2 elements of a field, row by
+ * row, and the elements of such an array (for testing). */
+int cpsz_tile_index_2d(size_t r1, size_t r2, uint64_t* at, uint64_t* elems);
 /* Device scratch of one 2D field's compression and decompression (for testing). */
 int cpsz_scratch_bytes_2d(size_t r1, size_t r2, int value_bytes, uint64_t* compress, uint64_t* decompress);
 

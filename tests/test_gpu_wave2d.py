@@ -35,6 +35,8 @@ def _same(a, b):
 
 SHAPES = [(1, 1), (1, 2), (2, 1), (1, 17), (300, 1), (3, 15), (63, 16), (64, 17), (65, 2), (127, 64), (128, 65), (129, 33),
           (255, 79), (256, 80), (257, 81), (513, 31), (320, 200)]
+# fewer columns than 64 and than rows: taken with rows and columns exchanged
+SHAPES += [(2, 2), (3, 2), (40, 25), (64, 63), (130, 63), (200, 12), (97, 13), (1000, 3), (301, 48), (75, 24)]
 
 
 @pytest.mark.parametrize("shape", SHAPES, ids=lambda s: f"{s[0]}x{s[1]}")

@@ -18,11 +18,12 @@ def test_offsets_within_a_strip_fit(rows, value_bytes):
 
 
 @pytest.mark.parametrize("value_bytes", [4, 8])
-def test_offsets_of_a_column(value_bytes):
+@pytest.mark.parametrize("cols", [1, 2, 33, 63])
+def test_offsets_of_a_few_columns(cols, value_bytes):
     edge = (1 << 32) // (64 * value_bytes)
-    for r1 in [1, 1000, edge // 2, edge - 63, edge - 1, edge]:
-        far, span = cz.wave2d_span(r1, 1, value_bytes)
-        assert far or span <= (1 << 32) - 16
+    for r1 in [64, 1000, edge // 2] + list(range(edge - 100, edge + 3)):
+        far, span = cz.wave2d_span(r1, cols, value_bytes)
+        assert far or span <= (1 << 32) - 16, (r1, cols, span)
 
 
 @pytest.mark.parametrize("bits,value", [(np.uint32, np.float32), (np.uint64, np.float64)])
@@ -48,3 +49,26 @@ def test_decompression_refuses_sides_beyond_its_range(shape):
     for value_bytes in (4, 8):
         with pytest.raises(cz.CpszError):
             cz.scratch_bytes_2d(*shape, value_bytes)
+
+
+@pytest.mark.parametrize("r1", [1, 2, 5, 16, 33, 63, 64, 65, 128, 130, 300])
+def test_every_element_has_a_place_of_its_own(r1):
+    for r2 in [1, 2, 3, 7, 8, 9, 15, 16, 17, 31, 40, 55, 56, 57, 63, 64, 65, 100, 128, 301]:
+        at, n = cz.tile_index_2d(r1, r2)
+        assert np.unique(at).size == r1 * r2 and at.max() < n, r2
+
+
+# (r1, r2, slots per value): a compression keeps two components' eb codes by value and, by slot, these and the
+# quantization codes again, a decompression ids, codes and unpredictable values by slot; either has the groups'
+# boundary rows, at most 0.25 bytes a value
+THIN = [(1, 1 << 20, 1), (1 << 20, 1, 1), (3, 1 << 20, 4 / 3), (33, 1 << 16, 64 / 33), (65, 1 << 16, 128 / 65), (1 << 18, 2, 1),
+        (1 << 18, 3, 4 / 3), (1 << 18, 16, 1), (1 << 18, 17, 32 / 17), (1 << 18, 63, 64 / 63), (1 << 16, 64, 2),
+        (1 << 16, 256, 1.25), (4096, 4096, 1.02)]
+
+
+@pytest.mark.parametrize("r1,r2,slots", THIN)
+def test_scratch_of_thin_fields(r1, r2, slots):
+    comp, dec = (x / (r1 * r2) for x in cz.scratch_bytes_2d(r1, r2))
+    assert comp <= (4 + 8 * slots + 0.25) * 1.01 + 1.2 and dec <= (16 * slots + 0.25) * 1.01
+    # a row of 2^28 values is decompressed in a few gigabytes
+    assert cz.scratch_bytes_2d(1, 1 << 28)[1] < 5 << 30
