@@ -1,11 +1,11 @@
 // Batched compression / decompression of many 3D fields (timesteps of a
 // simulation, ensemble members), possibly of different sizes.
 //
-// Compress: the eb, sign and log kernels take all fields in a launch each, then ONE persistent wavefront launch covers every field's (plane
-// group, row block) items (a 192^3 field alone offers 144 workgroups of work
-// to 256 CUs), then the entropy stages (histograms, host Huffman trees,
-// encode, stream assembly) of different fields run concurrently on the worker
-// pool. Decompress: parsing, Huffman decoding and scatter per field on the
+// Compress: the eb, sign and log kernels take all fields in a launch each, then
+// ONE persistent wavefront launch covers every field's (plane group, row block)
+// items (a 192^3 field alone offers 144 workgroups of work to 256 CUs), then the
+// entropy stages (histograms, host Huffman trees, encode, stream assembly) of
+// different fields run concurrently on the worker pool. Decompress: parsing, Huffman decoding and scatter per field on the
 // workers, one persistent wavefront launch, then the exp2 finish per field.
 // Every field's stream is byte-identical to the single-field codec's.
 #include <algorithm>

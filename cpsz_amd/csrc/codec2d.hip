@@ -2,12 +2,14 @@
 // sz_compress_cp_preserve_2d_offline / sz_decompress_cp_preserve_2d_offline).
 //
 // Device pipeline (compress), all inputs resident in HBM:
-//   k_eb2d        per-cell triangle bounds in LDS (8x64 vertex tiles + 1-cell
+//   k_eb2d*       per-cell triangle bounds in LDS (16x32 vertex tiles + 1-cell
 //                 halo), ordered per-vertex min, |U|,|V| scaling and the base-4
-//                 eb id -> eb code per vertex and component, id histogram
+//                 eb id -> eb code per vertex and component (row-major for the id
+//                 encoder, in tiles for the wavefront), id histogram
 //   k_wave2d      strip-pipelined wavefront Lorenzo + linear quantization (wave2d.hip)
-//   Huffman       histogram -> host tree (reference tie-break) -> encode
-//   unpredictable values compacted in 12x12 block-major order
+//   Huffman       histogram -> tree on the host or, in batches, the device
+//                 (reference tie-break) -> encode, with the unpredictable
+//                 values compacted in 12x12 block-major order
 // Decompress mirrors it: parallel Huffman decode of ids and codes, block-major
 // unpredictable scatter, wavefront reconstruction.
 //
@@ -786,10 +788,6 @@ struct BlockView {
     sy = min(kBlock2d, r2 - j0);
     m = sx * sy;
   }
-  __device__ size_t elem(int k, int r2) const {
-    const int ii = k / sy, jj = k - ii * sy;
-    return (size_t)(i0 + ii) * r2 + j0 + jj;
-  }
   __device__ size_t tile_elem(int k, const Tile2d& t) const {
     const int ii = k / sy, jj = k - ii * sy;
     return t.at(i0 + ii, j0 + jj);
@@ -1398,7 +1396,7 @@ void launch_eb_fast(Ctx& ctx, const Eb2dJob* dj, int nj, uint32_t blk, double ma
   k_fill_u32<<<1, 64, 0, st>>>(fx, 1, 0);
   k_eb2d_multi<true><<<blk, 256, 0, st>>>(dj, nj, max_pwr_eb, ctx.d_q2d(), ctx.q2d_size(), fx + 1, fx);
   // a listed tile costs a few dependent global loads per marked vertex: enough
-  // blocks to keep every CU's slots filled (70 VGPRs: 7 blocks per CU)
+  // blocks to keep every CU's slots filled (72 VGPRs: 7 blocks per CU)
   k_eb2d_fix<<<std::min<uint32_t>(blk, 2048), 256, 0, st>>>(dj, nj, fx + 1, fx, max_pwr_eb, ctx.d_q2d(),
                                                             ctx.q2d_size());
 }

@@ -98,7 +98,10 @@ __global__ void __launch_bounds__(256) k_dec_cand(MDecTable jobs, int* __restric
 }
 
 // One wave per stream; leaves at once unless the stream needs it. Lane 0 walks
-// the whole stream, so each of its segments has its one true start.
+// the whole stream, so each of its segments has its one true start, at 1.7 us a
+// code (1744 ms for 10^6 codes of 17 bits; of 16 bits, without it, 1.2). It takes
+// runs of codes above 16 bits and of one length: streams made for it, as uniform
+// noise (2400 x 3600, at bounds from 0.1 down to 1e-5) does not come to it.
 __global__ void __launch_bounds__(64) k_dec_serial(MDecTable jobs, int* __restrict__ err, const int* __restrict__ over) {
   __shared__ uint32_t slut[1 << kLutBits];
   __shared__ uint32_t sw[kStageWords];

@@ -193,7 +193,7 @@ __global__ void __launch_bounds__(256) k_gemm_bf16(int M, int N, int K, const ui
 // banks. Bound by the feature build's loads and divisions, then by LDS: 12
 // fields of 10 million vertices in all took 4.95 ms with the patch read twice
 // at computed indexes, unpadded rows and 8 waves a CU, 1.31 ms as it stands
-// (the matrix products alone are 0.2 ms). Operand layout: lane t
+// (the matrix products alone are 0.2 ms); one 97 x 130 x 111 field 1.04 and 0.31 ms. Operand layout: lane t
 // supplies A(t%32, 8*(t/32)+q) and B(8*(t/32)+q, t%32), q = 0..7, and
 // receives D(8*(r/4) + 4*(t/32) + r%4, t%32) in accumulator r.
 typedef __bf16 bf16x8m __attribute__((ext_vector_type(8)));
