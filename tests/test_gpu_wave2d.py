@@ -75,6 +75,20 @@ def test_strip_of_four_gib(orc):
     assert _same(got[0], want[0]) and _same(got[1], want[1])
 
 
+def test_flipped_strip_of_four_gib(orc):
+    """Two columns, taken as two rows of 2^24."""
+    r1, r2 = 1 << 24, 2
+    print(f"[wave2d] {r1}x{r2}", flush=True)
+    x = np.arange(r1, dtype=np.float32)
+    U = np.stack([np.sin(x / 531), np.cos(x / 917)], axis=1).astype(np.float32) + np.float32(1e-3)
+    V = np.stack([np.cos(x / 713), np.sin(x / 389)], axis=1).astype(np.float32)
+    U[::97] = 0
+    s, ref = cz.sz_compress_cp_preserve_2d_offline(U, V, 0.1), orc.compress_2d(U, V, 0.1)
+    assert np.array_equal(mask_2d_padding(s, r1, r2), mask_2d_padding(ref, r1, r2))
+    got, want = cz.sz_decompress_cp_preserve_2d_offline(ref, r1, r2), orc.decompress_2d(ref, r1, r2)
+    assert _same(got[0], want[0]) and _same(got[1], want[1])
+
+
 @pytest.mark.parametrize("dtype", [np.float32, np.float64])
 def test_tiles_of_four_gib(orc, dtype):
     """Rows a little under 4 GiB a strip, whose tiles are a little over: the last value of the third row lies past 4 GiB.
